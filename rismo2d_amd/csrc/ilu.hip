@@ -36,6 +36,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 #include "rmx_internal.h"
 
@@ -1132,173 +1133,204 @@ __global__ void __launch_bounds__(512) k_sweep_stage(const int* __restrict__ ble
 // ---------------------------------------------------------------------------------------
 // block sweeps: one wave per block, both triangles in one launch
 
-constexpr int BS_ROWS = 2047;      // rows per block (11-bit positions)
-constexpr int BS_LROWS = 32;       // rows per level (5-bit row numbers)
-constexpr int BS_LPAIRS = 64;      // entry pairs per level (one per lane)
-constexpr int BS_PAD = 256;        // padding after every entry stream (clamped loads)
-constexpr unsigned BS_EM = (1u << 21) - 1;
-constexpr int BS_DEPTH = 4;        // levels whose loads are in flight ahead of the level
+constexpr int BS_ROWS = 2047;      // rows per block
+constexpr int BS_GROUP_ROWS = 4093; // rows per wave (12-bit positions)
+constexpr int BS_WAVES = 1024;     // waves that fill the chip (one per SIMD)
+constexpr int BS_SLOTS = 16;       // slots per pass (4 lanes each)
+constexpr int BS_MAXW = 128;       // columns per node (8 slots of 16)
+constexpr int BS_PAD = 64;         // padding after every stream (loads past the last node)
 constexpr int BS_GATHER = 8;       // rows per lane whose loads are issued together
+constexpr int BS_DEPTH = 4;        // passes whose loads are in flight ahead
 
-template <class VT> struct VPair;
-template <> struct VPair<float> { using T = float2; using Q = float4; };
-template <> struct VPair<double> { using T = double2; using Q = double4; };
+// Slot descriptor: x = first row group of the slot's values (18 bits) | position of the
+// node's first row << 18 (12 bits) | column groups in the slot - 1 << 30; y = first column
+// group (16 bits) | node << 16 (12 bits) | rows << 28 (0: empty slot) | log2(slots of the
+// node) << 30.  A node's slots are aligned to their number.  Descriptor 0 of a triangle is
+// empty.
+constexpr unsigned BS_VM = (1u << 18) - 1, BS_CM = (1u << 16) - 1, BS_PM = (1u << 12) - 1;
 
-// One step of an inclusive scan over lanes segmented by key (equal keys are contiguous,
-// keys >= 1): every lane adds the value DPP control C brings from another lane when that
-// lane has the same key and the step applies to the lane's row (ok).  A lane the control
-// leaves without a source reads zeros (key 0: no match).
+template <class T> struct Triple { T x, y, z; };   // loaded without the padding's register
+template <class VT> struct VQuad;
+template <> struct VQuad<float> { using T = float4; };
+template <> struct VQuad<double> { using T = double4; };
+
 template <int C>
-__device__ __forceinline__ void seg_step(double& v, int key, bool ok)
+__device__ __forceinline__ double dpp_get(double v)
 {
-  const int ks = __builtin_amdgcn_mov_dpp(key, C, 0xF, 0xF, true);
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), C, 0xF, 0xF, true);
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), C, 0xF, 0xF, true);
-  const double vs = __hiloint2double(hi, lo);
-  v = (ks == key && ok) ? v + vs : v;
+  return __hiloint2double(hi, lo);
 }
-
-// Sum of v over each run of equal keys, complete at the run's last lane: shifts by 1, 2, 4
-// and 8 inside each row of 16 lanes, then lane 15 of rows 0 and 2 into rows 1 and 3, then
-// lane 31 into rows 2 and 3 (each row already holds its own part when it is passed on).
-__device__ __forceinline__ double seg_sum(double v, int key, bool rows13, bool rows23)
+template <class T>
+__device__ __forceinline__ T ld_off(const void* base, unsigned off)
 {
-  seg_step<0x111>(v, key, true);     // row_shr:1
-  seg_step<0x112>(v, key, true);     // row_shr:2
-  seg_step<0x114>(v, key, true);     // row_shr:4
-  seg_step<0x118>(v, key, true);     // row_shr:8
-  seg_step<0x142>(v, key, rows13);   // row_bcast:15
-  seg_step<0x143>(v, key, rows23);   // row_bcast:31
-  return v;
+  return *reinterpret_cast<const T*>(static_cast<const char*>(base) + off);
 }
+// doubles at a byte offset of the dynamic LDS (kernels without static LDS: it starts at 0, so
+// the offset is the address)
+typedef __attribute__((address_space(3))) double lds_double;
+__device__ __forceinline__ double ld_lds(unsigned off) { return *(const lds_double*)off; }
+__device__ __forceinline__ void st_lds(unsigned off, double v) { *(lds_double*)off = v; }
 
-// The levels of one triangle of one block.  A level lists nodes (units of 1-3 rows); its
-// entries are the couplings of those rows to rows outside their node, a row's entries
-// padded to an even count (at least one pair), lane L taking pair L.  Loaded BS_DEPTH
-// levels ahead into a register ring: the value pair, the packed pair of column | row-in-
-// level words, the level's table entries (kept uniform) and, for lane j, node j's record
-// and couplings.  A level: every lane multiplies its pair by the solved values of the
-// columns, a segmented scan sums each row at its last lane, which leaves the sum in LDS;
-// then lane j solves node j's rows in order with the couplings inside the node: the lower
-// sweep x_r += sum_r + sum of l_rs x_s (factors stored negated), the upper sweep (rows in
-// reverse) x_r = (x_r - sum_r - sum of u_rs x_s) / u_rr.  One wave works the block, so a
-// level ends without a workgroup barrier.
-template <class VT, bool LOWER>
-__device__ __forceinline__ void block_levels(int nlev, const unsigned* tab,
+// The passes of one triangle of one block.  A pass holds up to 16 slots of 4 lanes; a slot
+// holds up to 16 columns of one node, a node takes 1, 2, 4 or 8 neighbouring slots, and the
+// nodes of a pass do not depend on each other.  Lane q of a slot multiplies column group q
+// into the node's (at most 3) row sums; two DPP exchanges add them over the quad (nodes of
+// more slots: row mirrors and a shuffle; M: none in the block, at most 2 slots, any), so every
+// lane of the node has them and solves the node's rows in registers: the lower sweep x_r +=
+// sum_r + sum of l_rs x_s (factors stored negated), the upper sweep (rows in reverse) x_r =
+// (x_r - sum_r - sum of u_rs x_s) / u_rr; lane r of the node's first slot writes row r.
+// Column groups that a slot does not have read the block's zero group and the zero slot
+// before x; rows that a node does not have read what follows and are not used.
+// The chain from one pass to the next is one LDS read, four products, two exchanges, the
+// node's solve and one LDS write, and a wave working alone is bound by its instructions
+// (about 105 a pass, 4 cycles each; a branch costs about 70): nothing waits for memory, since
+// values, columns, couplings and reciprocal diagonals are loaded D passes ahead into a
+// register ring, the descriptors that name them 2 D, and the pass table's entries 3 D ahead.
+// One wave works the block, so a pass ends without a workgroup barrier.
+template <class VT, bool LOWER, int M, int D>
+__device__ __forceinline__ void block_passes(int np, const unsigned* __restrict__ tab,
+                                             const uint2* __restrict__ desc,
                                              const VT* __restrict__ vals,
-                                             const unsigned short* __restrict__ meta,
-                                             const unsigned* __restrict__ unit,
+                                             const uint2* __restrict__ cols,
                                              const VT* __restrict__ uval,
-                                             const double4* __restrict__ rdg, double* x,
-                                             double* acc, double* sink, int lane, int m)
+                                             const double4* __restrict__ rdg, int lane)
 {
-  using V2 = typename VPair<VT>::T;
-  using V4 = typename VPair<VT>::Q;
-  constexpr int D = BS_DEPTH;
-  const V2* vp = reinterpret_cast<const V2*>(vals);           // entry bases are even
-  const unsigned* mp = reinterpret_cast<const unsigned*>(meta);
-  const V4* up4 = reinterpret_cast<const V4*>(uval);          // 4 couplings per node
-  V2 vv[D];
-  V4 ua[D];
-  double4 ub[D];
-  unsigned cm[D], ui[D], ta[D], tb[D];
-  const bool rows13 = (lane >> 4) & 1, rows23 = lane >= 32;
-#pragma unroll
-  for (int k = 0; k < D; k++) {                            // the first D levels are empty
-    ta[k] = 0; tb[k] = 0; cm[k] = 0; ui[k] = 1u << 11;
-    vv[k].x = (VT)0; vv[k].y = (VT)0;
-  }
-  // stages run for levels 0, 1, 2, ...; past the last level the doubled sentinel makes an
-  // empty level with the same loads.  The table entry after the stage's level is read one
-  // stage ahead, so no stage waits for it.
-  unsigned t_lo = __builtin_amdgcn_readfirstlane(tab[0]);
-  unsigned t_hi_v = tab[min(1, nlev + 1)];
-  int ls = 0;
-  auto stage = [&](int k) {
-    const unsigned t0 = t_lo, t1 = __builtin_amdgcn_readfirstlane(t_hi_v);
-    t_hi_v = tab[min(ls + 2, nlev + 1)];
-    t_lo = t1;
-    ls++;
-    ta[k] = t0; tb[k] = t1;
-    const int e0 = (int)(t0 & BS_EM), np = ((int)(t1 & BS_EM) - e0) >> 1;
-    const int q = (e0 >> 1) + min(lane, max(np - 1, 0));
-    vv[k] = vp[q];
-    cm[k] = mp[q];
-    const int U0 = (int)(t0 >> 21), nu = (int)(t1 >> 21) - U0;
-    const int u = U0 + min(lane, max(nu - 1, 0));
-    ui[k] = unit[u];
-    ua[k] = up4[u];
-    if (!LOWER) ub[k] = rdg[u];
-  };
-  auto level = [&](int k) {
-    const unsigned t0 = ta[k], t1 = tb[k];
-    const int np = ((int)(t1 & BS_EM) - (int)(t0 & BS_EM)) >> 1;
-    const int nu = (int)(t1 >> 21) - (int)(t0 >> 21);
-    const unsigned ca = cm[k] & 0xffffu, cb = cm[k] >> 16;   // one row: the same row bits
-    double v = (double)vv[k].x * x[ca & 2047u] + (double)vv[k].y * x[cb & 2047u];
-    const bool on = lane < np;
-    const int key = on ? 1 + (int)(ca >> 11) : 64;
-    v = on ? v : 0.0;
-    v = seg_sum(v, key, rows13, rows23);
-    const int kn = __builtin_amdgcn_mov_dpp(key, 0x130, 0xF, 0xF, true);   // wave_shl:1
-    if (on && kn != key) acc[key - 1] = v;
-    wave_sync();
-    if (lane < nu) {
-      // branch-free: rows past the node's last read valid slots, take neutral operands and
-      // store to the sink
-      const unsigned inf = ui[k];
-      const int p = (int)(inf & 2047u), nr = (int)((inf >> 11) & 3u), s0 = (int)(inf >> 13);
-      const bool h1 = nr > 1, h2 = nr > 2;
-      const int r1 = h1 ? 1 : 0, r2 = h2 ? 2 : r1;
-      const double a0 = acc[s0], a1 = acc[s0 + r1], a2 = acc[s0 + r2];
-      const double x0 = x[p], x1 = x[p + r1], x2 = x[p + r2];
-      double y0, y1, y2;
-      if (LOWER) {
-        // couplings l10, l20, l21 (zero where absent)
-        y0 = x0 + a0;
-        y1 = x1 + a1 + (double)ua[k].x * y0;
-        y2 = x2 + a2 + (double)ua[k].y * y0 + (double)ua[k].z * y1;
-      } else {
-        // couplings u01, u02, u12 (zero where absent), reciprocal diagonals (1 where
-        // absent); last row first
-        y2 = (h2 ? x2 - a2 : 0.0) * ub[k].z;
-        y1 = (h1 ? x1 - a1 - (double)ua[k].z * y2 : 0.0) * ub[k].y;
-        y0 = (x0 - a0 - (double)ua[k].x * y1 - (double)ua[k].y * y2) * ub[k].x;
-      }
-      x[p] = y0;
-      *(h1 ? x + p + 1 : sink) = y1;
-      *(h2 ? x + p + 2 : sink) = y2;
-    }
-    wave_sync();
-  };
-  // no branch around a stage, so that every level issues the same loads and the wait
-  // before a level's first use of its registers leaves the later levels' loads in flight;
-  // the first D (empty) levels issue the loads of levels 0 .. D - 1, so that every load
-  // of the ring is issued inside the loop, into the same registers
-  for (int l0 = -D; l0 < nlev; l0 += D) {
+  using V4 = typename VQuad<VT>::T;
+  constexpr unsigned VB = sizeof(V4);
+  const unsigned slot = lane >> 2, q = lane & 3;
+  V4 va[D], vb[D], vc[D];
+  Triple<VT> wu[D];
+  Triple<double> rd[D];
+  uint2 ca[D], dr[D];
+  unsigned xo[D], wo[D], fl[D];            // byte offsets: first row, result (0: none); rows
+                                           // and log2 of the slots << 2
+  // descriptors of D passes from the table's entries (one per lane)
+  auto fetch = [&](unsigned t, uint2* d) {
 #pragma unroll
     for (int k = 0; k < D; k++) {
-      level(k);
+      const unsigned s0 = __builtin_amdgcn_readlane(t, k), s1 = __builtin_amdgcn_readlane(t, k + 1);
+      d[k] = desc[slot < s1 - s0 ? s0 + slot : 0u];
+    }
+  };
+  const unsigned tl = min(lane, D);
+  fetch(tab[tl], dr);
+  tab += D;
+  unsigned tv = tab[tl];
+#pragma unroll
+  for (int k = 0; k < D; k++) {             // the first D passes are empty
+    ca[k] = make_uint2(0u, 0u);
+    va[k] = vb[k] = vc[k] = V4{};
+    wu[k] = Triple<VT>{};
+    rd[k] = Triple<double>{};
+    xo[k] = wo[k] = fl[k] = 0u;
+    // waited for here: pending at the loop's entry, they would be waited for in every round,
+    // with the loads in flight behind them
+    asm volatile("" : "+v"(dr[k].x), "+v"(dr[k].y));
+  }
+  asm volatile("" : "+v"(tv));
+  auto stage = [&](int k) {
+    const uint2 d = dr[k];
+    const unsigned R = d.y >> 28 & 3u, lg = d.y >> 30;
+    const bool has = q <= d.x >> 30;
+    ca[k] = ld_off<uint2>(cols, has ? ((d.y & BS_CM) + q) * 8u : 0u);
+    const unsigned ov = has ? ((d.x & BS_VM) + q * R) * VB : 0u;
+    va[k] = ld_off<V4>(vals, ov);
+    vb[k] = ld_off<V4>(vals, ov + VB);
+    vc[k] = ld_off<V4>(vals, ov + 2u * VB);
+    const unsigned u = d.y >> 16 & BS_PM;
+    wu[k] = ld_off<Triple<VT>>(uval, u * VB);
+    if (!LOWER) rd[k] = ld_off<Triple<double>>(rdg, u * 32u);
+    xo[k] = ((d.x >> 18 & BS_PM) + 1u) * 8u;
+    wo[k] = q < R && (M == 0 || (slot & ((1u << lg) - 1u)) == 0u) ? xo[k] + 8u * q : 0u;
+    fl[k] = d.y >> 28;
+  };
+  double h0 = 0.0, h1 = 0.0, h2 = 0.0;      // right-hand sides of the next pass's nodes
+  auto pass = [&](int k) {
+    const double xa = ld_lds(ca[k].x & 0xffffu), xc = ld_lds(ca[k].x >> 16);
+    const double xd = ld_lds(ca[k].y & 0xffffu), xe = ld_lds(ca[k].y >> 16);
+    // read a pass ahead (no other pass writes them), behind the reads that this pass waits for
+    const double x0 = h0, x1 = h1, x2 = h2;
+    const int kn = (k + 1) % D;
+    h0 = ld_lds(xo[kn]); h1 = ld_lds(xo[kn] + 8u); h2 = ld_lds(xo[kn] + 16u);
+    __builtin_amdgcn_sched_barrier(0);
+    double s0 = (double)va[k].x * xa, s1 = (double)vb[k].x * xa, s2 = (double)vc[k].x * xa;
+    s0 += (double)va[k].y * xc; s1 += (double)vb[k].y * xc; s2 += (double)vc[k].y * xc;
+    s0 += (double)va[k].z * xd; s1 += (double)vb[k].z * xd; s2 += (double)vc[k].z * xd;
+    s0 += (double)va[k].w * xe; s1 += (double)vb[k].w * xe; s2 += (double)vc[k].w * xe;
+    s0 += dpp_get<0xB1>(s0); s1 += dpp_get<0xB1>(s1); s2 += dpp_get<0xB1>(s2);   // lane ^ 1
+    s0 += dpp_get<0x4E>(s0); s1 += dpp_get<0x4E>(s1); s2 += dpp_get<0x4E>(s2);   // lane ^ 2
+    if (M > 0) {                                            // nodes of 2 or more slots
+      const unsigned lg = fl[k] >> 2;
+      double e0 = dpp_get<0x141>(s0), e1 = dpp_get<0x141>(s1), e2 = dpp_get<0x141>(s2);
+      s0 += lg >= 1u ? e0 : 0.0; s1 += lg >= 1u ? e1 : 0.0; s2 += lg >= 1u ? e2 : 0.0;
+      if (M > 1) {
+        if (__any(lg > 1u)) {
+          e0 = dpp_get<0x140>(s0); e1 = dpp_get<0x140>(s1); e2 = dpp_get<0x140>(s2);
+          s0 += lg >= 2u ? e0 : 0.0; s1 += lg >= 2u ? e1 : 0.0; s2 += lg >= 2u ? e2 : 0.0;
+          e0 = __shfl_xor(s0, 16, 64); e1 = __shfl_xor(s1, 16, 64); e2 = __shfl_xor(s2, 16, 64);
+          s0 += lg >= 3u ? e0 : 0.0; s1 += lg >= 3u ? e1 : 0.0; s2 += lg >= 3u ? e2 : 0.0;
+        }
+      }
+    }
+    double y0, y1, y2;
+    if (LOWER) {
+      // couplings l10, l20, l21 (zero where absent)
+      y0 = x0 + s0;
+      y1 = x1 + s1 + (double)wu[k].x * y0;
+      y2 = x2 + s2 + (double)wu[k].y * y0 + (double)wu[k].z * y1;
+    } else {
+      // couplings u01, u02, u12 (zero where absent), reciprocal diagonals; last row first,
+      // rows past the node's zero
+      const unsigned R = fl[k] & 3u;
+      y2 = (R > 2u ? x2 - s2 : 0.0) * rd[k].z;
+      y1 = (R > 1u ? x1 - s1 - (double)wu[k].z * y2 : 0.0) * rd[k].y;
+      y0 = (x0 - s0 - (double)wu[k].x * y1 - (double)wu[k].y * y2) * rd[k].x;
+    }
+    asm volatile("" : "+v"(y0), "+v"(y1), "+v"(y2));        // selected, not branched around
+    const double y = q == 0u ? y0 : (q == 1u ? y1 : y2);
+    // a wave's LDS operations complete in order: the compiler must keep the order, no wait
+    asm volatile("" ::: "memory");
+    if (wo[k]) st_lds(wo[k], y);
+    asm volatile("" ::: "memory");
+  };
+  // no branch around a stage, so that every pass issues the same loads and the wait before
+  // a pass's first use of its registers leaves the later passes' loads in flight; the first
+  // D (empty) passes issue the loads of passes 0 .. D - 1, and the table's last entry is
+  // repeated past the last pass (empty passes)
+  for (int l0 = -D; l0 < np; l0 += D) {
+    // the descriptors that the next D stages decode: asked for before anything else, so that
+    // taking them over at the end leaves this round's loads in flight
+    uint2 dn[D];
+    fetch(tv, dn);
+    tab += D;
+    const unsigned tn = tab[tl];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+      pass(k);
       stage(k);
     }
+#pragma unroll
+    for (int k = 0; k < D; k++) dr[k] = dn[k];
+    tv = tn;
   }
 }
 
-// One block per one-wave workgroup: the block's right-hand side is gathered into LDS (in
-// local positions), swept down and up in place, and written back in equation order (with
+// One block (or a group of independent blocks) per one-wave workgroup: its right-hand side is
+// gathered into LDS (in local positions), swept down and up in place, and written back in equation order (with
 // aidx, plus aval[aidx[e]]: the coarse prolongation folded into the write).  Blocks hold
 // disjoint rows, so b and x may be the same vector.
 template <class VT>
 __global__ void __launch_bounds__(64) k_block_sweep(const int4* __restrict__ info,
                                                     const int* __restrict__ gidx,
-                                                    const unsigned* __restrict__ levt,
+                                                    const unsigned* __restrict__ tab,
+                                                    const uint2* __restrict__ desc,
                                                     const VT* __restrict__ vlo,
-                                                    const unsigned short* __restrict__ mlo,
-                                                    const unsigned* __restrict__ ulo,
+                                                    const uint2* __restrict__ clo,
                                                     const VT* __restrict__ wlo,
                                                     const VT* __restrict__ vup,
-                                                    const unsigned short* __restrict__ mup,
-                                                    const unsigned* __restrict__ uup,
+                                                    const uint2* __restrict__ cup,
                                                     const VT* __restrict__ wup,
                                                     const double4* __restrict__ rdg,
                                                     const double* rhs, double* out,
@@ -1307,14 +1339,11 @@ __global__ void __launch_bounds__(64) k_block_sweep(const int4* __restrict__ inf
 {
   constexpr int G = BS_GATHER;
   extern __shared__ double smem[];
-  const int4 i0 = info[2 * blockIdx.x], i1 = info[2 * blockIdx.x + 1];
-  const int rb = i0.x, m = i0.y, lb = i0.z, nl = i0.w, nu = i1.x, ub = i1.y;
+  const int4 i0 = info[4 * blockIdx.x], i1 = info[4 * blockIdx.x + 1];
+  const int4 i2 = info[4 * blockIdx.x + 2], i3 = info[4 * blockIdx.x + 3];
+  const int rb = i0.x, m = i0.y, ub = i0.z, tb = i0.w;
   const int lane = threadIdx.x;
-  double* x = smem;                                           // [m] local positions
-  double* acc = smem + m;                                     // [BS_LROWS] row sums
-  double* sink = acc + BS_LROWS;                              // [2] stores of absent rows
-  unsigned* tl = reinterpret_cast<unsigned*>(sink + 2);       // [nl + 2]
-  unsigned* tu = tl + nl + 2;                                 // [nu + 2]
+  double* x = smem + 1;                                       // [m] local positions; [-1]: zero
   // gathers: every load of a chunk issued before any is waited for
   for (int k0 = 0; k0 < m; k0 += 64 * G) {
     int g[G];
@@ -1327,20 +1356,24 @@ __global__ void __launch_bounds__(64) k_block_sweep(const int4* __restrict__ inf
     for (int j = 0; j < G; j++)
       if (k0 + lane + 64 * j < m) x[k0 + lane + 64 * j] = v[j];
   }
-  const int nt = nl + nu + 4;                                 // both tables, contiguous
-  for (int k0 = 0; k0 < nt; k0 += 64 * G) {
-    unsigned t[G];
-#pragma unroll
-    for (int j = 0; j < G; j++) t[j] = levt[lb + min(k0 + lane + 64 * j, nt - 1)];
-#pragma unroll
-    for (int j = 0; j < G; j++)
-      if (k0 + lane + 64 * j < nt) tl[k0 + lane + 64 * j] = t[j];
-  }
+  if (lane < 3) smem[lane ? m + lane : 0] = 0.0;       // the zero slot, rows past the last
   wave_sync();
-  block_levels<VT, true>(nl, tl, vlo + i1.z, mlo + i1.z, ulo + ub, wlo + 4 * (long long)ub,
-                         nullptr, x, acc, sink, lane, m);
-  block_levels<VT, false>(nu, tu, vup + i1.w, mup + i1.w, uup + ub, wup + 4 * (long long)ub,
-                          rdg + ub, x, acc, sink, lane, m);
+  auto lower = [&](auto mode) {
+    block_passes<VT, true, decltype(mode)::value, BS_DEPTH>(
+        i1.x, tab + tb, desc + i1.y, vlo + 4 * (long long)i2.x, clo + i2.y,
+        wlo + 4 * (long long)ub, nullptr, lane);
+  };
+  auto upper = [&](auto mode) {
+    block_passes<VT, false, decltype(mode)::value, BS_DEPTH>(
+        i1.z, tab + tb + i1.x + 4 * BS_DEPTH, desc + i1.w, vup + 4 * (long long)i2.z, cup + i2.w,
+        wup + 4 * (long long)ub, rdg + ub, lane);
+  };
+  if (i3.x == 0) lower(std::integral_constant<int, 0>());
+  else if (i3.x == 1) lower(std::integral_constant<int, 1>());
+  else lower(std::integral_constant<int, 2>());
+  if (i3.y == 0) upper(std::integral_constant<int, 0>());
+  else if (i3.y == 1) upper(std::integral_constant<int, 1>());
+  else upper(std::integral_constant<int, 2>());
   wave_sync();
   for (int k0 = 0; k0 < m; k0 += 64 * G) {
     int e[G];
@@ -1475,49 +1508,70 @@ static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>&
   order = prow;
 }
 
-// Block sweep layout.  A block is the rows of one strip in one segment; a unit is a run of
+// Block sweep layout.  A block is the rows of one strip in one segment, and a wave works a
+// group of blocks of one strip (below, the layout of a group); a unit is a run of
 // rows of one node (group), at most 3 (every row its own unit without `group`).  Unit
 // levels: a unit's lower level is one more than the highest of the units its rows couple to
-// below them in the block (upper: above); units of a level are independent.  Local
-// positions list the units in lower level order, a unit's rows together.  Levels are split
-// into parts of at most BS_LROWS rows and BS_LPAIRS entry pairs.  Entries keep the strip
-// sweeps' rule (the strict triangle inside the row's block), minus the couplings inside a
-// unit, which go to the unit's record.  Off (the strip sweeps run) when a block has more than
-// BS_ROWS rows or its entries do not fit 21 bits.
-static void build_blocks(Ilu& I, const std::vector<int>* group, hipStream_t s)
+// below them in the block (upper: above); units of a level are independent.  A unit's
+// columns are the union of its rows' columns outside the unit (the rows of a node have the
+// same ones), in groups of 4 (zero-padded), a slot for every 4 groups, the slots rounded up
+// to a power of two (the added ones hold no columns).  Units of a level are listed by
+// falling slot count, so that a unit's slots are aligned to their number, and cut into
+// passes of at most 16 slots.  Local positions list the units in lower order, a unit's rows
+// together.  The first column group and the first 3 row groups of a block's streams are zero.
+// Entries keep the strip sweeps' rule (the strict triangle inside the row's
+// block), minus the couplings inside a unit, which go to the unit's record.  Off (the strip
+// sweeps run) when a block has more than BS_ROWS rows or a group does not fit the
+// descriptors.
+// scol, spos: every row's columns ascending and their places in the row.
+static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vector<int>& scol,
+                         const std::vector<unsigned char>& spos, hipStream_t s)
 {
   BlockSweep& B = I.bs;
   B.on = false;
   const int n = I.n, nstrip = I.nblk, nseg = std::max(1, I.nseg);
   const std::vector<int>& rp = I.h_rp;
-  const std::vector<int>& cl = I.h_cols;
   const bool sg = !I.seg.empty();
   auto segof = [&](int i) { return sg ? I.seg[i] : 0; };
   if (nseg == 1)
     for (int b = 0; b < nstrip; b++)
       if (I.bstart[b + 1] - I.bstart[b] > BS_ROWS) return;
-  // tighter level caps (tests of the level split): RMX_BLOCK_LEVEL_ROWS, RMX_BLOCK_LEVEL_PAIRS
-  int cap_rows = BS_LROWS, cap_pairs = BS_LPAIRS;
-  if (const char* e = getenv("RMX_BLOCK_LEVEL_ROWS")) cap_rows = std::max(3, std::min(BS_LROWS, atoi(e)));
-  if (const char* e = getenv("RMX_BLOCK_LEVEL_PAIRS")) cap_pairs = std::max(1, std::min(BS_LPAIRS, atoi(e)));
+  // tighter pass caps (tests of the level split): rows and entry pairs (each row's entries in
+  // pairs, at least one) of a pass; a node needing more sits alone
+  int cap_rows = 3 * BS_SLOTS, cap_pairs = INT_MAX;
+  if (const char* e = getenv("RMX_BLOCK_LEVEL_ROWS")) cap_rows = std::max(3, std::min(cap_rows, atoi(e)));
+  if (const char* e = getenv("RMX_BLOCK_LEVEL_PAIRS")) cap_pairs = std::max(1, atoi(e));
   // CSR position of entry (r, c), -1 if the pattern has none
   auto find = [&](int r, int c) {
-    for (int q = rp[r]; q < rp[r + 1]; q++)
-      if (cl[q] == c) return q;
-    return -1;
+    const auto b = scol.begin() + rp[r], e = scol.begin() + rp[r + 1];
+    const auto it = std::lower_bound(b, e, c);
+    return it != e && *it == c ? rp[r] + (int)spos[it - scol.begin()] : -1;
   };
   struct Part {
     std::vector<int> rows;               // equation at every local position
-    std::vector<unsigned> tab[2];        // level tables (lower, upper)
-    std::vector<unsigned short> meta[2];
-    std::vector<int> src[2];
-    std::vector<unsigned> unit[2];       // unit records
+    std::vector<unsigned> tab[2];        // pass tables: first slot of every pass (lower, upper)
+    std::vector<uint2> desc[2];          // slot descriptors
+    int npass[2] = {0, 0}, lgmax[2] = {0, 0};   // lgmax: log2 of the most slots of a node
+    std::vector<unsigned short> col[2];  // columns, LDS byte offsets, 4 per group
+    std::vector<int> src[2];             // CSR position of every value (4 per row group)
     std::vector<int> usrc[2];            // unit coupling sources (4 per unit)
     std::vector<int> dsrc;               // unit diagonal sources (4 per unit)
     bool fits = true;
   };
+  // Blocks per wave: neighbouring segments of a strip share a wave, level by level, where a
+  // wave per block would leave each SIMD more than one (their levels hold a few nodes each,
+  // so a wave alone uses a few of its 16 slots and the chip issues mostly empty lanes): about
+  // BS_WAVES groups in all, of at most BS_GROUP_ROWS rows.
+  std::vector<int> gps(nstrip, nseg);          // groups of every strip
+  for (int b = 0; b < nstrip; b++) {
+    const int rows = I.bstart[b + 1] - I.bstart[b];
+    int k = std::max(1, std::min(nseg, (BS_WAVES + nstrip - 1) / nstrip));
+    while (k < nseg && (long long)rows * ((nseg + k - 1) / k) > (long long)BS_GROUP_ROWS * nseg * 9 / 10) k++;
+    gps[b] = k;
+  }
   std::vector<Part> parts((size_t)nstrip * nseg);
   parallel_for(nstrip, [&](long long b0, long long b1) {
+    std::vector<int> uc, up;             // a unit's columns, descending; its entries
     for (long long b = b0; b < b1; b++) {
       const int a = I.bstart[b], e = I.bstart[b + 1];
       // units of the strip (runs of one node's rows in one segment, at most 3)
@@ -1529,188 +1583,247 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, hipStream_t s)
         uof[i - a] = (int)ustart.size() - 1;
       }
       auto inblock = [&](int i, int c) { return c >= a && c < e && segof(c) == segof(i); };
-      // entry pairs of a row (at least one) when its unit starts at u0 and ends before u1
-      auto row_pairs = [&](int i, int u0, int u1, bool lower) {
-        int w = 0;
-        for (int q = rp[i] + 1; q < rp[i + 1]; q++) {
-          const int c = cl[q];
-          w += (lower ? c < i : c > i) && inblock(i, c) && (c < u0 || c >= u1);
-        }
-        return std::max(1, (w + 1) / 2);
+      // rows [u0, u1) with one set of columns (the rows of a node): row u0 stands for them
+      auto one_set = [&](int u0, int u1) {
+        for (int i = u0 + 1; i < u1; i++)
+          if (rp[i + 1] - rp[i] != rp[u0 + 1] - rp[u0] ||
+              !std::equal(scol.begin() + rp[u0], scol.begin() + rp[u0 + 1], scol.begin() + rp[i]))
+            return false;
+        return true;
       };
-      // a unit whose rows need more pairs than a level holds becomes single-row units (a
-      // row has at most 127 entries, 64 pairs)
+      // columns of rows [u0, u1) outside them, in the block, on one side
+      auto unit_cols = [&](int u0, int u1, bool lower, bool one) {
+        uc.clear();
+        for (int i = u0; i < (one ? u0 + 1 : u1); i++) {
+          const int* b = scol.data() + rp[i];
+          const int* e = scol.data() + rp[i + 1];
+          if (lower) e = std::lower_bound(b, e, u0); else b = std::lower_bound(b, e, u1);
+          for (const int* c = e; c-- > b;)
+            if (inblock(i, *c)) uc.push_back(*c);
+        }
+        if (!one) {
+          std::sort(uc.begin(), uc.end(), std::greater<int>());
+          uc.erase(std::unique(uc.begin(), uc.end()), uc.end());
+        }
+        return (int)uc.size();
+      };
+      // a unit of more columns than BS_MAXW becomes single-row units (a row has at most 127)
       {
         std::vector<int> us2;
+        bool split = false;
         for (size_t U = 0; U < ustart.size(); U++) {
           const int u0 = ustart[U], u1 = U + 1 < ustart.size() ? ustart[U + 1] : e;
-          int pl = 0, pu = 0;
-          for (int i = u0; i < u1; i++) { pl += row_pairs(i, u0, u1, true); pu += row_pairs(i, u0, u1, false); }
-          if (std::max(pl, pu) <= BS_LPAIRS) us2.push_back(u0);
-          else for (int i = u0; i < u1; i++) us2.push_back(i);
+          if (one_set(u0, u1) || (unit_cols(u0, u1, true, false) <= BS_MAXW &&
+                                  unit_cols(u0, u1, false, false) <= BS_MAXW)) {
+            us2.push_back(u0);
+          } else {
+            split = true;
+            for (int i = u0; i < u1; i++) us2.push_back(i);
+          }
         }
-        ustart.swap(us2);
-        for (size_t U = 0; U < ustart.size(); U++) {
-          const int u1 = U + 1 < ustart.size() ? ustart[U + 1] : e;
-          for (int i = ustart[U]; i < u1; i++) uof[i - a] = (int)U;
+        if (split) {
+          ustart.swap(us2);
+          for (size_t U = 0; U < ustart.size(); U++) {
+            const int u1 = U + 1 < ustart.size() ? ustart[U + 1] : e;
+            for (int i = ustart[U]; i < u1; i++) uof[i - a] = (int)U;
+          }
         }
       }
       const int nu = (int)ustart.size();
       ustart.push_back(e);
-      // unit levels, lower and upper
+      // unit levels and slots (log2), lower and upper
       std::vector<int> ulev[2] = { std::vector<int>(nu, 0), std::vector<int>(nu, 0) };
-      for (int U = 0; U < nu; U++)
-        for (int i = ustart[U]; i < ustart[U + 1]; i++)
-          for (int q = rp[i] + 1; q < rp[i + 1]; q++) {
-            const int c = cl[q];
-            if (c < i && inblock(i, c) && uof[c - a] != U)
-              ulev[0][U] = std::max(ulev[0][U], ulev[0][uof[c - a]] + 1);
-          }
-      for (int U = nu - 1; U >= 0; U--)
-        for (int i = ustart[U]; i < ustart[U + 1]; i++)
-          for (int q = rp[i] + 1; q < rp[i + 1]; q++) {
-            const int c = cl[q];
-            if (c > i && inblock(i, c) && uof[c - a] != U)
-              ulev[1][U] = std::max(ulev[1][U], ulev[1][uof[c - a]] + 1);
-          }
-      // units of every segment
-      std::vector<std::vector<int>> segu(nseg);
-      for (int U = 0; U < nu; U++) segu[segof(ustart[U])].push_back(U);
-      for (int g = 0; g < nseg; g++) {
+      std::vector<unsigned char> ulg[2] = { std::vector<unsigned char>(nu, 0),
+                                            std::vector<unsigned char>(nu, 0) };
+      std::vector<unsigned char> uone(nu);
+      for (int U = 0; U < nu; U++) uone[U] = one_set(ustart[U], ustart[U + 1]);
+      for (int t = 0; t < 2; t++)
+        for (int k = 0; k < nu; k++) {
+          const int U = t == 0 ? k : nu - 1 - k;
+          const int w = unit_cols(ustart[U], ustart[U + 1], t == 0, uone[U]);
+          for (int c : uc) ulev[t][U] = std::max(ulev[t][U], ulev[t][uof[c - a]] + 1);
+          while ((16 << ulg[t][U]) < w) ulg[t][U]++;
+        }
+      // units of every group of segments
+      const int ng = gps[b];
+      std::vector<std::vector<int>> grpu(ng);
+      std::vector<int> segrows(nseg, 0);
+      for (int U = 0; U < nu; U++) {
+        const int g = segof(ustart[U]);
+        grpu[(long long)g * ng / nseg].push_back(U);
+        segrows[g] += ustart[U + 1] - ustart[U];
+      }
+      const bool wide_block = *std::max_element(segrows.begin(), segrows.end()) > BS_ROWS;
+      for (int g = 0; g < ng; g++) {
         Part& P = parts[(size_t)b * nseg + g];
-        std::vector<int>& us = segu[g];
+        std::vector<int>& us = grpu[g];
         if (us.empty()) continue;
         int m = 0;
         for (int U : us) m += ustart[U + 1] - ustart[U];
-        if (m > BS_ROWS) { P.fits = false; continue; }
-        // lower order: by lower level, then unit index; local positions follow it
+        if (wide_block || m > BS_GROUP_ROWS) { P.fits = false; continue; }
+        // by level, then falling slot count, then unit index; local positions follow the
+        // lower order
         std::vector<int> ord[2] = { us, us };
         for (int t = 0; t < 2; t++)
-          std::stable_sort(ord[t].begin(), ord[t].end(),
-                           [&](int x, int y) { return ulev[t][x] < ulev[t][y]; });
-        std::vector<int> upos(nu, -1);
-        for (int U : ord[0]) {
+          std::stable_sort(ord[t].begin(), ord[t].end(), [&](int x, int y) {
+            return ulev[t][x] != ulev[t][y] ? ulev[t][x] < ulev[t][y] : ulg[t][x] > ulg[t][y];
+          });
+        std::vector<int> upos(nu, -1), uidx(nu, -1);
+        for (int k = 0; k < (int)ord[0].size(); k++) {
+          const int U = ord[0][k];
           upos[U] = (int)P.rows.size();
+          uidx[U] = k;
           for (int i = ustart[U]; i < ustart[U + 1]; i++) P.rows.push_back(i);
         }
         auto pos = [&](int c) { return upos[uof[c - a]] + (c - ustart[uof[c - a]]); };
         for (int t = 0; t < 2; t++) {
           const bool lower = t == 0;
-          std::vector<unsigned>& tab = P.tab[t];
-          std::vector<unsigned short>& meta = P.meta[t];
+          std::vector<uint2>& desc = P.desc[t];
+          std::vector<unsigned short>& col = P.col[t];
           std::vector<int>& src = P.src[t];
-          int cur = -1, nrow = 0, npair = 0;
-          for (int k = 0; k < (int)ord[t].size(); k++) {
-            const int U = ord[t][k], r0 = ustart[U], nr = ustart[U + 1] - r0;
-            int pairs = 0;                      // the unit's entry pairs (a row at least one)
-            for (int i = r0; i < r0 + nr; i++) pairs += row_pairs(i, r0, r0 + nr, lower);
-            if (ulev[t][U] != cur || nrow + nr > cap_rows || npair + pairs > cap_pairs) {
-              tab.push_back(((unsigned)k << 21) | (unsigned)meta.size());
-              cur = ulev[t][U]; nrow = 0; npair = 0;
-            }
+          col.assign(4, 0);                    // the zero groups
+          src.assign(12, -1);
+          desc.assign(1, uint2{ 0u, 0u });     // the empty slot
+          int cur = -1, nrow = 0, npair = 0, nslot = 0;
+          P.usrc[t].assign(4 * ord[t].size(), -1);
+          if (!lower) P.dsrc.assign(4 * ord[t].size(), -1);
+          for (int U : ord[t]) {
+            const int r0 = ustart[U], nr = ustart[U + 1] - r0;
+            const int ns = 1 << ulg[t][U];
+            P.lgmax[t] = std::max(P.lgmax[t], (int)ulg[t][U]);
+            const int w = unit_cols(r0, r0 + nr, lower, uone[U]);
+            // CSR positions of the unit's entries, row by row in the order of uc; a row's
+            // entries in pairs, at least one
+            up.assign((size_t)nr * w, -1);
+            int pairs = 0;
             for (int j = 0; j < nr; j++) {
-              const int i = r0 + j;
-              const size_t start = meta.size();
-              for (int q = rp[i] + 1; q < rp[i + 1]; q++) {
-                const int c = cl[q];
-                if ((lower ? c < i : c > i) && inblock(i, c) && uof[c - a] != U) {
-                  meta.push_back((unsigned short)(pos(c) | ((nrow + j) << 11)));
-                  src.push_back(q);
+              const int* b = scol.data() + rp[r0 + j];
+              const int* c = scol.data() + rp[r0 + j + 1];
+              int k = 0;
+              for (int x = 0; x < w; x++) {            // both descending
+                while (c > b && c[-1] > uc[x]) c--;
+                if (c > b && c[-1] == uc[x]) {
+                  up[(size_t)j * w + x] = rp[r0 + j] + (int)spos[c - 1 - scol.data()];
+                  k++;
                 }
               }
-              while (meta.size() - start < 2 || ((meta.size() - start) & 1)) {   // zero entries
-                meta.push_back((unsigned short)(((nrow + j) << 11)));
-                src.push_back(-1);
-              }
+              pairs += std::max(1, (k + 1) / 2);
             }
-            P.unit[t].push_back((unsigned)upos[U] | ((unsigned)nr << 11) | ((unsigned)nrow << 13));
+            if (ulev[t][U] != cur || nslot + ns > BS_SLOTS || nrow + nr > cap_rows ||
+                npair + pairs > cap_pairs) {
+              P.tab[t].push_back((unsigned)desc.size());
+              P.npass[t]++;
+              cur = ulev[t][U]; nrow = 0; npair = 0; nslot = 0;
+            }
+            const int ngroups = (w + 3) / 4;
+            const size_t cg0 = col.size() / 4, vg0 = src.size() / 4;
+            for (int k = 0; k < 4 * ngroups; k++)  // padding: the zero slot, value zero
+              col.push_back((unsigned short)(k < w ? 8 * (pos(uc[k]) + 1) : 0));
+            for (int gq = 0; gq < ngroups; gq++)
+              for (int j = 0; j < nr; j++)
+                for (int k = 4 * gq; k < 4 * gq + 4; k++) src.push_back(k < w ? up[(size_t)j * w + k] : -1);
+            if (col.size() / 4 > BS_CM || src.size() / 4 > BS_VM) P.fits = false;
+            for (int j = 0; j < ns; j++) {
+              // a slot without columns takes the zero groups
+              const int ng = std::max(0, std::min(4, ngroups - 4 * j));
+              const size_t v0 = ng > 0 ? vg0 + (size_t)4 * j * nr : 0, c0 = ng > 0 ? cg0 + 4 * j : 0;
+              desc.push_back(uint2{ (unsigned)(v0 & BS_VM) | (unsigned)upos[U] << 18 |
+                                        (unsigned)std::max(0, ng - 1) << 30,
+                                    (unsigned)(c0 & BS_CM) | (unsigned)uidx[U] << 16 |
+                                        (unsigned)nr << 28 | (unsigned)ulg[t][U] << 30 });
+            }
+            int* us4 = &P.usrc[t][4 * (size_t)uidx[U]];
             const int r1 = r0 + std::min(1, nr - 1), r2 = r0 + std::min(2, nr - 1);
             if (lower) {
-              const int l10 = nr > 1 ? find(r1, r0) : -1, l20 = nr > 2 ? find(r2, r0) : -1;
-              const int l21 = nr > 2 ? find(r2, r1) : -1;
-              for (int v : { l10, l20, l21, -1 }) P.usrc[t].push_back(v);
+              us4[0] = nr > 1 ? find(r1, r0) : -1;
+              us4[1] = nr > 2 ? find(r2, r0) : -1;
+              us4[2] = nr > 2 ? find(r2, r1) : -1;
             } else {
-              const int u01 = nr > 1 ? find(r0, r1) : -1, u02 = nr > 2 ? find(r0, r2) : -1;
-              const int u12 = nr > 2 ? find(r1, r2) : -1;
-              for (int v : { u01, u02, u12, -1 }) P.usrc[t].push_back(v);
-              for (int v : { rp[r0], nr > 1 ? rp[r1] : -1, nr > 2 ? rp[r2] : -1, -1 })
-                P.dsrc.push_back(v);
+              us4[0] = nr > 1 ? find(r0, r1) : -1;
+              us4[1] = nr > 2 ? find(r0, r2) : -1;
+              us4[2] = nr > 2 ? find(r1, r2) : -1;
+              int* ds4 = &P.dsrc[4 * (size_t)uidx[U]];
+              ds4[0] = rp[r0];
+              if (nr > 1) ds4[1] = rp[r1];
+              if (nr > 2) ds4[2] = rp[r2];
             }
             nrow += nr;
             npair += pairs;
+            nslot += ns;
           }
-          tab.push_back(((unsigned)ord[t].size() << 21) | (unsigned)meta.size());
-          tab.push_back(tab.back());         // read by the prefetch past the last level
-          for (int z = 0; z < 2; z++) {      // a zero pair, loaded by the levels past the last
-            meta.push_back(0);
-            src.push_back(-1);
-          }
-          if (meta.size() > BS_EM) P.fits = false;
+          // the end, repeated for the entries read past the last pass
+          P.tab[t].resize(P.tab[t].size() + 4 * BS_DEPTH, (unsigned)desc.size());
         }
       }
     }
   });
-  long long nb = 0, ent[2] = {0, 0}, nlev = 0, nunit = 0;
+  long long nb = 0, ncg[2] = {0, 0}, nvg[2] = {0, 0}, npass = 0, nunit = 0, nslots = 0, ntab = 0;
   size_t lds = 0;
   for (const Part& P : parts) {
     if (!P.fits) return;
     if (P.rows.empty()) continue;
     nb++;
-    for (int t = 0; t < 2; t++) ent[t] += P.meta[t].size();
-    nlev += P.tab[0].size() + P.tab[1].size();
-    nunit += P.unit[0].size();
-    const size_t m = P.rows.size();
-    lds = std::max(lds, 8 * (m + BS_LROWS + 2) + 4 * (P.tab[0].size() + P.tab[1].size()));
+    for (int t = 0; t < 2; t++) {
+      ncg[t] += P.col[t].size() / 4;
+      nvg[t] += P.src[t].size() / 4;
+      nslots += P.desc[t].size();
+      npass += P.npass[t];
+      ntab += P.tab[t].size();
+    }
+    nunit += P.usrc[0].size() / 4;
+    lds = std::max(lds, 8 * (P.rows.size() + 3));
   }
-  if (nb == 0 || ent[0] + BS_PAD > INT_MAX || ent[1] + BS_PAD > INT_MAX) return;
-  std::vector<int4> info(2 * nb);
+  const long long lim = INT_MAX - BS_PAD;
+  if (nb == 0 || std::max({ 4 * ncg[0], 4 * ncg[1], nvg[0], nvg[1], nslots, ntab }) > lim) return;
+  std::vector<int4> info(4 * nb);
   std::vector<int> gidx(n);
-  std::vector<int> src[2], usrc[2];
-  std::vector<unsigned short> meta[2];
-  std::vector<unsigned> unit[2];
+  std::vector<int> src[2], usrc[2], dsrc((size_t)4 * nunit, -1);
+  std::vector<unsigned short> col[2];
+  std::vector<uint2> desc(nslots);
+  std::vector<unsigned> tab(ntab + 64, 0u);
   for (int t = 0; t < 2; t++) {
-    src[t].assign(ent[t] + BS_PAD, -1);
-    meta[t].assign(ent[t] + BS_PAD, 0);
-    unit[t].assign(nunit + 64, 1u << 11);
-    usrc[t].assign((size_t)4 * (nunit + 64), -1);
+    src[t].assign(4 * ((size_t)nvg[t] + BS_PAD), -1);
+    col[t].assign(4 * ((size_t)ncg[t] + BS_PAD), 0);
+    usrc[t].assign((size_t)4 * nunit, -1);
   }
-  std::vector<int> dsrc((size_t)4 * (nunit + 64), -1);
-  std::vector<unsigned> lev(nlev);
-  long long k = 0, rb = 0, lb = 0, eo[2] = {0, 0}, ub = 0;
+  long long k = 0, rb = 0, sb = 0, tb = 0, ub = 0, cg[2] = {0, 0}, vg[2] = {0, 0};
   for (const Part& P : parts) {
     if (P.rows.empty()) continue;
     const int m = (int)P.rows.size();
-    const int nl = (int)P.tab[0].size() - 2, nu = (int)P.tab[1].size() - 2;
-    info[2 * k] = int4{ (int)rb, m, (int)lb, nl };
-    info[2 * k + 1] = int4{ nu, (int)ub, (int)eo[0], (int)eo[1] };
-    std::copy(P.tab[0].begin(), P.tab[0].end(), lev.begin() + lb);
-    std::copy(P.tab[1].begin(), P.tab[1].end(), lev.begin() + lb + nl + 2);
+    const int su = (int)(sb + P.desc[0].size());
+    info[4 * k] = int4{ (int)rb, m, (int)ub, (int)tb };
+    info[4 * k + 1] = int4{ P.npass[0], (int)sb, P.npass[1], su };
+    info[4 * k + 2] = int4{ (int)vg[0], (int)cg[0], (int)vg[1], (int)cg[1] };
+    info[4 * k + 3] = int4{ P.lgmax[0], P.lgmax[1], 0, 0 };
     std::copy(P.rows.begin(), P.rows.end(), gidx.begin() + rb);
     for (int t = 0; t < 2; t++) {
-      std::copy(P.meta[t].begin(), P.meta[t].end(), meta[t].begin() + eo[t]);
-      std::copy(P.src[t].begin(), P.src[t].end(), src[t].begin() + eo[t]);
-      std::copy(P.unit[t].begin(), P.unit[t].end(), unit[t].begin() + ub);
+      std::copy(P.tab[t].begin(), P.tab[t].end(), tab.begin() + tb);
+      tb += P.tab[t].size();
+      std::copy(P.desc[t].begin(), P.desc[t].end(), desc.begin() + sb);
+      sb += P.desc[t].size();
+      std::copy(P.col[t].begin(), P.col[t].end(), col[t].begin() + 4 * cg[t]);
+      std::copy(P.src[t].begin(), P.src[t].end(), src[t].begin() + 4 * vg[t]);
       std::copy(P.usrc[t].begin(), P.usrc[t].end(), usrc[t].begin() + 4 * ub);
-      eo[t] += P.meta[t].size();
+      cg[t] += P.col[t].size() / 4;
+      vg[t] += P.src[t].size() / 4;
     }
     std::copy(P.dsrc.begin(), P.dsrc.end(), dsrc.begin() + 4 * ub);
-    k++; rb += m; lb += nl + nu + 4; ub += P.unit[0].size();
+    k++; rb += m; ub += P.usrc[0].size() / 4;
   }
   B.nb = (int)nb; B.lds = (lds + 15) & ~(size_t)15;
   B.ne_lo = std::count_if(src[0].begin(), src[0].end(), [](int q) { return q >= 0; });
   B.ne_up = std::count_if(src[1].begin(), src[1].end(), [](int q) { return q >= 0; });
-  B.nlev = nlev; B.nunit = nunit;
-  B.info.upload(info, s); B.gidx.upload(gidx, s); B.lev.upload(lev, s);
-  B.mlo.upload(meta[0], s); B.mup.upload(meta[1], s);
+  B.npass = npass; B.nunit = nunit; B.nslot = nslots; B.ncol = 4 * (ncg[0] + ncg[1]);
+  B.info.upload(info, s); B.gidx.upload(gidx, s); B.tab.upload(tab, s); B.desc.upload(desc, s);
+  B.clo.upload(col[0], s); B.cup.upload(col[1], s);
   B.slo.upload(src[0], s); B.sup.upload(src[1], s);
-  B.ulo.upload(unit[0], s); B.uup.upload(unit[1], s);
   B.sulo.upload(usrc[0], s); B.suup.upload(usrc[1], s); B.sdg.upload(dsrc, s);
   HIPCHECK(hipStreamSynchronize(s));
   B.on = true;
   if (getenv("RMX_DEBUG"))
-    fprintf(stderr, "[rmx] block sweeps: %lld blocks, %lld nodes, %lld + %lld entries (%lld + "
-            "%lld padded), %.1f levels per block, %zu bytes LDS\n", nb, nunit, B.ne_lo, B.ne_up,
-            ent[0], ent[1], (double)nlev / nb - 4.0, B.lds);
+    fprintf(stderr, "[rmx] block sweeps: %lld groups of blocks, %lld nodes, %lld + %lld entries (%lld + "
+            "%lld padded), %.1f passes per group, %zu bytes LDS\n", nb, nunit, B.ne_lo, B.ne_up,
+            4 * nvg[0], 4 * nvg[1], (double)npass / nb, B.lds);
 }
 
 // Segment of every row: each strip [bstart[b], bstart[b+1]) is cut into nseg parts of
@@ -1853,7 +1966,7 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   std::vector<int> olo, oup;
   build_sweep(I.lo, I, true, olo, s, cap);
   build_sweep(I.up, I, false, oup, s, cap);
-  build_blocks(I, group, s);
+  build_blocks(I, group, scol, spos, s);
   // forward position (global, concatenated) of the row at each backward position
   std::vector<int> fpos(n), f2b(n);
   for (int r = 0; r < n; r++) fpos[olo[r]] = r;
@@ -2078,15 +2191,16 @@ static void launch_blocks(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t
   BlockSweep& B = I.bs;
   const BSvals<VT> V = bsvals<VT>(B);
   if (ev) HIPCHECK(hipEventRecord(ev[0], c.stream));
-  // algorithmic bytes: entries (value + 2-byte column), per node its two records, 8 coupling
-  // values and 3 FP64 reciprocal diagonals (stored as 4), per row the gather index,
-  // right-hand side and result, per level its table entry, and the folded prolongation
+  // algorithmic bytes: entry values, a 2-byte column per node and column, per node 8 coupling
+  // values and 3 FP64 reciprocal diagonals (stored as 4), per row the gather index, right-hand
+  // side and result, per slot its descriptor, per pass its table entry, the folded prolongation
   const double v = (double)sizeof(VT);
-  const double bytes = (double)(B.ne_lo + B.ne_up) * (v + 2.0) + (double)B.nunit * (32.0 + 8.0 * v) +
-                       20.0 * I.n + 4.0 * B.nlev + (aidx ? 12.0 * I.n : 0.0);
+  const double bytes = (double)(B.ne_lo + B.ne_up) * v + 2.0 * B.ncol + (double)B.nunit * (32.0 + 8.0 * v) +
+                       8.0 * B.nslot + 20.0 * I.n + 4.0 * B.npass + (aidx ? 12.0 * I.n : 0.0);
   const int kt = kt_begin(c, KT_SWEEP_BLK, bytes);
-  k_block_sweep<VT><<<B.nb, 64, B.lds, c.stream>>>(B.info.p, B.gidx.p, B.lev.p,
-      V.vlo->p, B.mlo.p, B.ulo.p, V.wlo->p, V.vup->p, B.mup.p, B.uup.p, V.wup->p,
+  k_block_sweep<VT><<<B.nb, 64, B.lds, c.stream>>>(B.info.p, B.gidx.p, B.tab.p, B.desc.p,
+      V.vlo->p, reinterpret_cast<const uint2*>(B.clo.p), V.wlo->p, V.vup->p,
+      reinterpret_cast<const uint2*>(B.cup.p), V.wup->p,
       reinterpret_cast<const double4*>(V.rdg->p), b, x, aidx, aval);
   kt_end(c, kt);
   if (ev) {

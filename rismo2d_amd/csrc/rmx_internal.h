@@ -138,23 +138,25 @@ struct SweepSet {
 
 // Block sweeps of the strip ILU(0): one wave per block (a segment of a strip), the lower
 // and the upper sweep of the block in one launch with the block's values in LDS.  The unit
-// of a sweep level is a node (the run of its rows in the block, up to 3): the entries that
-// couple a node's rows are solved by one lane in registers, so a node adds one level, not
-// three.  Local positions are the rows in lower-sweep order.  A level holds at most 32 rows
-// and 64 entry pairs (a row's entries are padded to an even count, so no lane holds two
-// rows' entries).
+// of a sweep is a node (the run of its rows in the block, up to 3): the entries that couple
+// a node's rows are solved in registers, so a node adds one level, not three.  Local
+// positions are the rows in lower-sweep order.  A node's columns outside it are stored once,
+// in groups of 4, with the values of its rows group by group (4 values a row); passes,
+// slots and descriptors as k_block_sweep takes them.
 struct BlockSweep {
   bool on = false;
   int nb = 0;                      // blocks
   size_t lds = 0;                  // dynamic LDS bytes of the largest block
-  long long ne_lo = 0, ne_up = 0, nlev = 0, nunit = 0;
-  DBuf<int4> info;                 // [2 nb] {row base, rows, level table, lower levels},
-                                   //        {upper levels, unit base, lower / upper entry base}
+  long long ne_lo = 0, ne_up = 0, npass = 0, nunit = 0, nslot = 0, ncol = 0;
+  DBuf<int4> info;                 // [4 nb] {row base, rows, unit base, pass table},
+                                   //        {lower passes, descriptors, upper ...},
+                                   //        {lower row group, column group, upper ...},
+                                   //        {log2 of the most slots of a node, lower, upper}
   DBuf<int> gidx;                  // [n] equation at every local position
-  DBuf<unsigned> lev;              // per level: first unit (<< 21) | first entry in the block
-  DBuf<unsigned short> mlo, mup;   // per entry: local column | row in its level << 11
-  DBuf<unsigned> ulo, uup;         // per unit: position | rows << 11 | first row in level << 13
-  DBuf<int> slo, sup;              // CSR position of every entry value (-1: zero)
+  DBuf<unsigned> tab;              // pass tables (lower, upper of every block)
+  DBuf<uint2> desc;                // slot descriptors (lower, upper of every block)
+  DBuf<unsigned short> clo, cup;   // columns: LDS byte offset (0: the zero slot)
+  DBuf<int> slo, sup;              // CSR position of every value (-1: zero)
   DBuf<int> sulo, suup, sdg;       // per unit: CSR positions of its lower / upper couplings
                                    // and of its diagonals (4 each; -1: none)
   DBuf<float> vlo32, vup32, wlo32, wup32;       // packed values (entries, unit couplings)

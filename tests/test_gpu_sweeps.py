@@ -1,0 +1,89 @@
+"""Triangular sweeps on the GPU at the edges of their layouts, against the oracle's ILU(0)
+factors and triangular solves.
+
+The sweeps sum a row's products in another order than the oracle, in FP64: each sum of w
+products is off by at most about w 1.1e-16 of its terms' magnitude, and the systems here are
+diagonally dominant (or the channel's, whose sweeps the other tests hold to the same bound),
+so results agree within 1e-12 of the largest.
+"""
+import numpy as np
+import pytest
+
+from helpers import golden_deck, load_golden
+from oracle import pyoracle as po
+from rismo2d_amd import rmx
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = rmx.Context(0)
+    yield c
+    c.close()
+
+
+def _band_csr(n, offsets, seed):
+    """n rows, row i coupled to i - o and i + o for every offset o (a symmetric pattern), in
+    random order after the diagonal; diagonally dominant."""
+    rng = np.random.default_rng(seed)
+    rp, cols, vals = [0], [], []
+    for i in range(n):
+        js = np.asarray([j for o in offsets for j in (i - o, i + o) if 0 <= j < n], int)
+        js = rng.permutation(js)
+        v = rng.standard_normal(len(js))
+        cols += [i] + js.tolist()
+        vals += [np.abs(v).sum() + 1.0] + v.tolist()
+        rp.append(len(cols))
+    return np.asarray(rp, np.int32), np.asarray(cols, np.int32), np.asarray(vals)
+
+
+# one block: entries per row and triangle at the edges of a lane's group (4), of a slot (16)
+# and of 2, 4 and 8 slots (32, 64, 127), chains and independent rows
+@pytest.mark.parametrize("n,width,stride", [(1, 0, 1), (2, 1, 1), (3, 2, 1), (17, 4, 3), (64, 0, 1),
+                                            (65, 5, 7), (200, 16, 2), (300, 17, 11), (513, 32, 3),
+                                            (700, 33, 5), (900, 63, 1), (65, 64, 1), (128, 127, 1),
+                                            (2047, 13, 31)])
+def test_single_block_of_single_rows(ctx, n, width, stride):
+    print(f"[gpu] one block, {n} rows, {width} entries a side", flush=True)
+    rp, cols, vals = _band_csr(n, [1 + stride * k for k in range(width)], 11)
+    b = np.random.default_rng(12).standard_normal(n)
+    ctx.csr_upload(rp, cols, vals, b)
+    for prec, dt in ((rmx.F64, np.float64), (rmx.F32, np.float32)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        ctx.ilu0_factor(prec)
+        L, r = po.ilu0_factor(rp, cols, vals.astype(dt))
+        assert r == 0
+        ref = po.ilu0_solve(rp, cols, L, b)
+        ctx.kernel_stats(True)
+        y = ctx.ilu0_apply(b, prec)
+        assert ctx.kernel_stats(False)["sweeps_block"][2] == 1
+        assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
+
+
+# 61 and 256 waves for 128 and 300 segments: one to three blocks of a strip share a wave
+@pytest.mark.parametrize("strips,segments", [(17, 128), (4, 300)])
+def test_blocks_that_share_a_wave(ctx, strips, segments):
+    print(f"[gpu] {strips} strips x {segments} segments, blocks sharing waves", flush=True)
+    g = load_golden("channel200x20")
+    ctx.upload_mesh(golden_deck(g))
+    ctx.prepare()
+    ctx.set_strips(strips, segments)
+    ctx.assemble(rmx.F64)
+    ctx.scale_l2()
+    rp, cols = ctx.pattern()
+    A, B = ctx.matrix(rmx.F64)
+    block = ctx.blocks()
+    rows = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+    keep = block[rows] == block[cols]
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=len(rp) - 1))])
+    for prec, dt in ((rmx.F64, np.float64), (rmx.F32, np.float32)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        ctx.silu0_factor(prec)
+        L, _ = po.ilu0_factor(rp, cols, A.astype(dt))
+        ref = po.ilu0_solve(rp2.astype(np.int32), cols[keep], L[keep], B)
+        y = ctx.silu0_apply(B, prec)
+        assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
+    ctx.set_strips(0, 0)
