@@ -419,7 +419,7 @@ rmx_status rmx_profile_kernels(rmx_ctx* ctx, int prec, int reps, rmx_kernel_time
  * in one launch (block sweeps: one wave per block).  bytes: the algorithmic bytes of each
  * launch summed (factorisation 3 nnz (v + 4); sweep: kept entries (v + 4) + 20 or 24 bytes
  * per row; block sweeps: kept entries of both triangles v bytes, 2 bytes per column of a
- * node and triangle, 32 + 8 v per node, 8 per slot descriptor, 4 per pass, 20 per row, + 12
+ * node and triangle, 32 + 16 v per node, 8 per slot descriptor, 4 per pass, 20 per row, + 12
  * per row with the folded prolongation; SpMV: the bytes of the layout it ran on;
  * Gram-Schmidt: the basis vectors read, FP32 or FP64, and the vector read and written;
  * coarse: the vectors, maps and A P entries it reads). */

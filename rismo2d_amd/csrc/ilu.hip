@@ -1,15 +1,14 @@
 // ILU(0) preconditioner on gfx950: factorisation and triangular sweeps
 // (PRECO_ILU0::Factor / Solve, Preco_ilu0.cpp:64-186, 497-530, 958-980).
 //
-// An Ilu object holds one ILU(0) system: the CSR pattern, the level sets of its
-// factorisation, the packed sweep layouts, and FP64 / FP32 factors.  Both instances of a
-// context factor the whole matrix in the reference's equation order (its FP32 factors are
-// bit-identical to the reference's); they differ in the sweeps:
-//  * the reference sweeps: one workgroup walks the level sets of the whole lower / upper
-//    factor (the plain FP64 path);
+// An Ilu object holds one ILU(0) system: the CSR pattern, the schedule of its factorisation,
+// the packed sweep layouts, and FP64 / FP32 factors.  Both instances of a context factor the
+// whole matrix in the reference's equation order (its FP32 factors are bit-identical to the
+// reference's); they differ in the sweeps:
+//  * the reference sweeps: the whole lower / upper factor (the plain FP64 path);
 //  * strip sweeps: rows are cut into contiguous ranges (the frontal order runs along the
-//    channel, so a range is a strip of cross-sections) and the factor entries that couple
-//    two strips are left out of the sweeps, so each strip is swept by its own workgroup.
+//    channel, so a range is a strip of cross-sections), strips into blocks, and the factor
+//    entries that couple two blocks are left out of the sweeps, so blocks are swept apart.
 //    The pivots stay those of the full factorisation (factoring the strips separately
 //    loses the upstream couplings at each strip start and leaves near-zero pivots).
 //    It preconditions the FP32 solve inside the FP64 refinement, where the FP64 residual,
@@ -20,17 +19,16 @@
 // updates in the reference's order and, with FMA contraction off, the reference's
 // rounding.  Multipliers are stored negated as in the reference.
 //
-// Sweeps: one workgroup per strip walks its level sets.  Rows are stored in processing
-// order with each row's off-diagonal entries contiguous and columns replaced by
-// processing positions.  Solved values go to an LDS ring (slot = position & (RING-1)) and
-// to a position-ordered global copy; a level reads a dependency from the ring while its
-// slot has not been reused (position >= P + nr - RING for a level of nr rows starting at
-// P) and from the global copy otherwise, which is safe because a full barrier (global
-// release / acquire) is taken whenever the position crosses a multiple of FENCE, and any
-// value that has left the ring is older than the last such barrier (nr <= RING/4).
-// Wider levels read everything from the global copy between full barriers.  Other levels
-// are separated by LDS-only barriers, so the next level's rows, loaded into registers
-// while the current level finishes, stay in flight across the barrier.
+// Sweeps: blocks of at most BS_ROWS rows by a wave each with their values in LDS
+// (k_block_sweep); others by a workgroup per strip that walks the levels of nodes, LDS holding
+// the rows that later levels still read (k_node_sweep); where those do not fit LDS, the staged
+// level sweep (k_sweep_stage), whose values go through an LDS ring of RING positions and a
+// global copy in processing order: a level reads a dependency from the ring while its slot has
+// not been reused (position >= P + nr - RING for a level of nr rows starting at P) and from the
+// global copy otherwise, which is safe because a full barrier (global release / acquire) is
+// taken whenever the position crosses a multiple of FENCE, and any value that has left the ring
+// is older than the last such barrier (nr <= RING/4).  Wider levels read everything from the
+// global copy between full barriers.
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -43,9 +41,6 @@
 namespace rmx {
 
 constexpr int FW = 128;         // maximum row width handled by the factorisation
-constexpr int PW = 6;           // entries per lane held in registers (more are read on)
-constexpr int SG = 8;           // lanes per row in the sweeps
-constexpr int SKR = 2;          // row-rounds per level held in registers
 constexpr int LPC = 1024;       // level offsets staged in LDS at a time
 constexpr int FENCE = 2048;     // positions between full barriers
 constexpr int WIDE = RING / 4;  // levels wider than this use the global copy only
@@ -733,6 +728,15 @@ __global__ void k_pack_rcp(long long ne, const int* __restrict__ psrc, const VT*
     out[t] = psrc[t] >= 0 ? 1.0 / (double)LU[psrc[t]] : 1.0;
 }
 
+// Reciprocal diagonals in equation order.
+template <class VT>
+__global__ void k_rcp_diag(int n, const int* __restrict__ rowptr, const VT* __restrict__ LU,
+                           double* __restrict__ out)
+{
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < n) out[r] = 1.0 / (double)LU[rowptr[r]];
+}
+
 template <class VT>
 __global__ void k_pack_diag(int n, const int* __restrict__ prow, const int* __restrict__ rowptr,
                             const VT* __restrict__ LU, VT* __restrict__ pdiag)
@@ -749,14 +753,6 @@ __device__ __forceinline__ void lds_barrier()
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-__device__ __forceinline__ double ring_or_global(const double* ring, const double* xp, int c, int lim)
-{
-  double v;
-  if (c >= lim) v = ring[c & (RING - 1)];
-  else v = __builtin_nontemporal_load(xp + c);
-  return v;
 }
 
 // One lane's share of a row's sum over entries q0, q0 + G, ... below q1, each solved value
@@ -781,136 +777,6 @@ __device__ __noinline__ double lane_sum(const VT* __restrict__ pval, const int* 
 // The right-hand side of position r is gsrc[gidx[r]] (the input vector gathered into
 // processing order on the fly); with oidx the solution of position r is also written to
 // odst[oidx[r]] (scattered back to equation order).
-template <class VT, bool LOWER, int G, int KR>
-__global__ void __launch_bounds__(1024) k_sweep(const int* __restrict__ blev,
-                                                const int* __restrict__ bpos,
-                                                const int* __restrict__ lev_ptr_all,
-                                                const int* __restrict__ prs_all,
-                                                const int* __restrict__ pcol,
-                                                const VT* __restrict__ pval,
-                                                const VT* __restrict__ pdiag_all,
-                                                const int* __restrict__ gidx_all,
-                                                const double* __restrict__ gsrc,
-                                                const int* __restrict__ oidx_all,
-                                                double* __restrict__ odst,
-                                                double* __restrict__ xp_all)
-{
-  __shared__ double ring[RING];
-  __shared__ int s_lp[LPC + 2];
-  const int b = blockIdx.x;
-  const int lb = blev[b];
-  const int nlev = blev[b + 1] - lb;
-  const int* lev_ptr = lev_ptr_all + lb + 2 * b;   // nlev + 2 local offsets
-  const int base = bpos[b];
-  const int* prs = prs_all + base;
-  const VT* pdiag = LOWER ? nullptr : pdiag_all + base;
-  const int* gidx = gidx_all + base;
-  const int* oidx = oidx_all ? oidx_all + base : nullptr;
-  double* xp = xp_all + base;
-  const int t = threadIdx.x;
-  const int grp = t / G, lane = t % G, ngr = blockDim.x / G;
-  auto load_lp = [&](int l0) {
-    for (int k = t; k < LPC + 2; k += blockDim.x) s_lp[k] = lev_ptr[min(l0 + k, nlev + 1)];
-  };
-  load_lp(0);
-  __syncthreads();
-  if (nlev <= 0) return;
-  int lbase = 0;
-  int cr[KR][PW];
-  VT vr[KR][PW];
-  int qar[KR], qbr[KR];
-  double inr[KR];
-  VT dgr[KR];
-  int P = s_lp[0], nr = s_lp[1] - s_lp[0];
-  auto fetch = [&](int P_, int nr_) {
-#pragma unroll
-    for (int k = 0; k < KR; k++) {
-      const int g = grp + k * ngr;
-      if (g < nr_) {
-        const int r = P_ + g;
-        inr[k] = gsrc[gidx[r]];
-        if (!LOWER) dgr[k] = pdiag[r];
-        qar[k] = prs[r];
-        qbr[k] = prs[r + 1];
-#pragma unroll
-        for (int j = 0; j < PW; j++) {
-          const int q = qar[k] + lane + j * G;
-          if (q < qbr[k]) { cr[k][j] = pcol[q]; vr[k][j] = pval[q]; }
-          else { cr[k][j] = -1; vr[k][j] = (VT)0; }
-        }
-      }
-    }
-  };
-  fetch(P, nr);
-  for (int l = 0; l < nlev; l++) {
-    // positions >= lim are still in the ring; a wide level reads the global copy only
-    const int lim = nr > WIDE ? INT_MAX : P + nr - RING;
-    const int rounds = (nr + ngr - 1) / ngr;
-    for (int k = 0; k < rounds; k++) {
-      const int g = grp + k * ngr;
-      const bool act = g < nr;
-      double s = 0.0;
-      double in = 0.0;
-      VT dg = (VT)1;
-      if (act) {
-        if (k < KR) {
-          const int kk = k < KR ? k : 0;
-          in = inr[kk];
-          dg = dgr[kk];
-          bool old = false;
-#pragma unroll
-          for (int j = 0; j < PW; j++) {
-            const int c = cr[kk][j];
-            if (c >= 0) {
-              old |= c < lim;
-              s += (double)vr[kk][j] * ring[c & (RING - 1)];
-            }
-          }
-          if (old) {                         // a dependency has left the ring: redo the row
-            s = 0.0;
-            for (int j = 0; j < PW; j++) {
-              const int c = cr[kk][j];
-              if (c >= 0) s += (double)vr[kk][j] * ring_or_global(ring, xp, c, lim);
-            }
-          }
-          for (int q = qar[kk] + lane + PW * G; q < qbr[kk]; q += G)
-            s += (double)pval[q] * ring_or_global(ring, xp, pcol[q], lim);
-        } else {
-          const int r = P + g;
-          in = gsrc[gidx[r]];
-          if (!LOWER) dg = pdiag[r];
-          for (int q = prs[r] + lane; q < prs[r + 1]; q += G)
-            s += (double)pval[q] * ring_or_global(ring, xp, pcol[q], lim);
-        }
-      }
-#pragma unroll
-      for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, G);
-      if (act && lane == 0) {
-        const double xi = LOWER ? in + s : (in - s) / (double)dg;
-        ring[(P + g) & (RING - 1)] = xi;
-        xp[P + g] = xi;
-        if (oidx) odst[oidx[P + g]] = xi;
-      }
-    }
-    const int Pn = P + nr;
-    bool full = Pn / FENCE != P / FENCE || nr > WIDE;
-    if (l + 1 < nlev) {
-      if (l + 2 - lbase > LPC) {            // next chunk of level offsets (rare)
-        __syncthreads();
-        lbase = l + 1;
-        load_lp(lbase);
-        __syncthreads();
-      }
-      P = s_lp[l + 1 - lbase];
-      nr = s_lp[l + 2 - lbase] - P;
-      full |= nr > WIDE;                    // a wide level starts after a full barrier
-      fetch(P, nr);                         // next level's registers, in flight across the barrier
-    }
-    if (full) __syncthreads();
-    else lds_barrier();
-  }
-}
-
 // Sweep with a two-stage load pipeline and no global stores inside a level.  Level l
 // computes from registers loaded during level l - 1 (stage 2: columns, values, right-hand
 // side, diagonal); during level l the stage-2 loads of level l + 1 and the stage-1 loads
@@ -1149,10 +1015,9 @@ constexpr int BS_DEPTH = 4;        // passes whose loads are in flight ahead
 // empty.
 constexpr unsigned BS_VM = (1u << 18) - 1, BS_CM = (1u << 16) - 1, BS_PM = (1u << 12) - 1;
 
-template <class T> struct Triple { T x, y, z; };   // loaded without the padding's register
 template <class VT> struct VQuad;
-template <> struct VQuad<float> { using T = float4; };
-template <> struct VQuad<double> { using T = double4; };
+template <> struct VQuad<float> { using T = float4; using P = float2; };
+template <> struct VQuad<double> { using T = double4; using P = double2; };
 
 template <int C>
 __device__ __forceinline__ double dpp_get(double v)
@@ -1172,15 +1037,56 @@ typedef __attribute__((address_space(3))) double lds_double;
 __device__ __forceinline__ double ld_lds(unsigned off) { return *(const lds_double*)off; }
 __device__ __forceinline__ void st_lds(unsigned off, double v) { *(lds_double*)off = v; }
 
+// Row q's sum of a node in lane q of the node's first quad, from every lane's shares s0, s1,
+// s2 of the three rows: two exchanges that halve the rows a lane carries, then, for nodes of
+// more slots (lg: log2 of their number), the other quads' sums by row rotations and shuffles.
+// M: the block has no such node, none of more than 2 slots, any.
+template <int M>
+__device__ __forceinline__ double node_sum(unsigned q, double s0, double s1, double s2, unsigned lg)
+{
+  const bool hi = q >= 2u, odd = q & 1u;
+  double a = (hi ? s2 : s0) + dpp_get<0x4E>(hi ? s0 : s2);          // lane ^ 2
+  double b = (hi ? 0.0 : s1) + dpp_get<0x4E>(hi ? s1 : 0.0);
+  double s = (odd ? b : a) + dpp_get<0xB1>(odd ? a : b);            // lane ^ 1
+  if (M > 0) {
+    const double e = dpp_get<0x12C>(s);                             // the next quad's
+    s += lg >= 1u ? e : 0.0;
+    if (M > 1) {
+      if (__any(lg > 1u)) {
+        const double f = dpp_get<0x128>(s);                         // two quads on
+        s += lg >= 2u ? f : 0.0;
+        const double g = __shfl_xor(s, 16, 64);
+        s += lg >= 3u ? g : 0.0;
+      }
+    }
+  }
+  return s;
+}
+
+// The node's rows solved across its first quad: row q in lane q from its right-hand side x
+// and sum s.  Lower sweep (factors stored negated): x_q + s_q + l_q0 y_0 + l_q1 y_1, w the
+// row's two couplings; upper sweep, last row first: (x_q - s_q - u_q2 y_2 - u_q1 y_1) rd, w =
+// (u_q1, u_q2), rd the reciprocal diagonal.  Couplings a row does not have are zero.
+template <bool LOWER, class W2>
+__device__ __forceinline__ double node_solve(double x, double s, const W2& w, double rd)
+{
+  if (LOWER) {
+    double t = x + s;
+    t += (double)w.x * dpp_get<0x00>(t);
+    t += (double)w.y * dpp_get<0x55>(t);
+    return t;
+  }
+  double t = x - s;
+  t -= (double)w.y * dpp_get<0xAA>(t * rd);
+  t -= (double)w.x * dpp_get<0x55>(t * rd);
+  return t * rd;
+}
+
 // The passes of one triangle of one block.  A pass holds up to 16 slots of 4 lanes; a slot
 // holds up to 16 columns of one node, a node takes 1, 2, 4 or 8 neighbouring slots, and the
 // nodes of a pass do not depend on each other.  Lane q of a slot multiplies column group q
-// into the node's (at most 3) row sums; two DPP exchanges add them over the quad (nodes of
-// more slots: row mirrors and a shuffle; M: none in the block, at most 2 slots, any), so every
-// lane of the node has them and solves the node's rows in registers: the lower sweep x_r +=
-// sum_r + sum of l_rs x_s (factors stored negated), the upper sweep (rows in reverse) x_r =
-// (x_r - sum_r - sum of u_rs x_s) / u_rr; lane r of the node's first slot writes row r.
-// Column groups that a slot does not have read the block's zero group and the zero slot
+// into the node's row sums; every lane of the node gets them and solves the node's rows in
+// registers; lane r of its first slot writes row r.  Column groups that a slot does not have read the block's zero group and the zero slot
 // before x; rows that a node does not have read what follows and are not used.
 // The chain from one pass to the next is one LDS read, four products, two exchanges, the
 // node's solve and one LDS write, and a wave working alone is bound by its instructions
@@ -1194,17 +1100,18 @@ __device__ __forceinline__ void block_passes(int np, const unsigned* __restrict_
                                              const VT* __restrict__ vals,
                                              const uint2* __restrict__ cols,
                                              const VT* __restrict__ uval,
-                                             const double4* __restrict__ rdg, int lane)
+                                             const double* __restrict__ rdg, int lane)
 {
   using V4 = typename VQuad<VT>::T;
+  using V2 = typename VQuad<VT>::P;
   constexpr unsigned VB = sizeof(V4);
   const unsigned slot = lane >> 2, q = lane & 3;
   V4 va[D], vb[D], vc[D];
-  Triple<VT> wu[D];
-  Triple<double> rd[D];
+  V2 wu[D];
+  double rd[D];
   uint2 ca[D], dr[D];
-  unsigned xo[D], wo[D], fl[D];            // byte offsets: first row, result (0: none); rows
-                                           // and log2 of the slots << 2
+  unsigned xo[D], fl[D];                   // LDS offset of row q (0: none); the lane writes it,
+                                           // log2 of the node's slots << 1
   // descriptors of D passes from the table's entries (one per lane)
   auto fetch = [&](unsigned t, uint2* d) {
 #pragma unroll
@@ -1221,9 +1128,9 @@ __device__ __forceinline__ void block_passes(int np, const unsigned* __restrict_
   for (int k = 0; k < D; k++) {             // the first D passes are empty
     ca[k] = make_uint2(0u, 0u);
     va[k] = vb[k] = vc[k] = V4{};
-    wu[k] = Triple<VT>{};
-    rd[k] = Triple<double>{};
-    xo[k] = wo[k] = fl[k] = 0u;
+    wu[k] = V2{};
+    rd[k] = 0.0;
+    xo[k] = fl[k] = 0u;
     // waited for here: pending at the loop's entry, they would be waited for in every round,
     // with the loads in flight behind them
     asm volatile("" : "+v"(dr[k].x), "+v"(dr[k].y));
@@ -1238,60 +1145,29 @@ __device__ __forceinline__ void block_passes(int np, const unsigned* __restrict_
     va[k] = ld_off<V4>(vals, ov);
     vb[k] = ld_off<V4>(vals, ov + VB);
     vc[k] = ld_off<V4>(vals, ov + 2u * VB);
-    const unsigned u = d.y >> 16 & BS_PM;
-    wu[k] = ld_off<Triple<VT>>(uval, u * VB);
-    if (!LOWER) rd[k] = ld_off<Triple<double>>(rdg, u * 32u);
-    xo[k] = ((d.x >> 18 & BS_PM) + 1u) * 8u;
-    wo[k] = q < R && (M == 0 || (slot & ((1u << lg) - 1u)) == 0u) ? xo[k] + 8u * q : 0u;
-    fl[k] = d.y >> 28;
+    const unsigned u = 4u * (d.y >> 16 & BS_PM) + q;
+    wu[k] = ld_off<V2>(uval, u * (unsigned)sizeof(V2));
+    if (!LOWER) rd[k] = ld_off<double>(rdg, u * 8u);
+    xo[k] = q < R ? ((d.x >> 18 & BS_PM) + 1u + q) * 8u : 0u;
+    fl[k] = (q < R && (M == 0 || (slot & ((1u << lg) - 1u)) == 0u) ? 1u : 0u) | lg << 1;
   };
-  double h0 = 0.0, h1 = 0.0, h2 = 0.0;      // right-hand sides of the next pass's nodes
+  double h0 = 0.0;                          // right-hand side of the next pass's row
   auto pass = [&](int k) {
     const double xa = ld_lds(ca[k].x & 0xffffu), xc = ld_lds(ca[k].x >> 16);
     const double xd = ld_lds(ca[k].y & 0xffffu), xe = ld_lds(ca[k].y >> 16);
-    // read a pass ahead (no other pass writes them), behind the reads that this pass waits for
-    const double x0 = h0, x1 = h1, x2 = h2;
-    const int kn = (k + 1) % D;
-    h0 = ld_lds(xo[kn]); h1 = ld_lds(xo[kn] + 8u); h2 = ld_lds(xo[kn] + 16u);
+    // read a pass ahead (no other pass writes it), behind the reads that this pass waits for
+    const double x0 = h0;
+    h0 = ld_lds(xo[(k + 1) % D]);
     __builtin_amdgcn_sched_barrier(0);
     double s0 = (double)va[k].x * xa, s1 = (double)vb[k].x * xa, s2 = (double)vc[k].x * xa;
     s0 += (double)va[k].y * xc; s1 += (double)vb[k].y * xc; s2 += (double)vc[k].y * xc;
     s0 += (double)va[k].z * xd; s1 += (double)vb[k].z * xd; s2 += (double)vc[k].z * xd;
     s0 += (double)va[k].w * xe; s1 += (double)vb[k].w * xe; s2 += (double)vc[k].w * xe;
-    s0 += dpp_get<0xB1>(s0); s1 += dpp_get<0xB1>(s1); s2 += dpp_get<0xB1>(s2);   // lane ^ 1
-    s0 += dpp_get<0x4E>(s0); s1 += dpp_get<0x4E>(s1); s2 += dpp_get<0x4E>(s2);   // lane ^ 2
-    if (M > 0) {                                            // nodes of 2 or more slots
-      const unsigned lg = fl[k] >> 2;
-      double e0 = dpp_get<0x141>(s0), e1 = dpp_get<0x141>(s1), e2 = dpp_get<0x141>(s2);
-      s0 += lg >= 1u ? e0 : 0.0; s1 += lg >= 1u ? e1 : 0.0; s2 += lg >= 1u ? e2 : 0.0;
-      if (M > 1) {
-        if (__any(lg > 1u)) {
-          e0 = dpp_get<0x140>(s0); e1 = dpp_get<0x140>(s1); e2 = dpp_get<0x140>(s2);
-          s0 += lg >= 2u ? e0 : 0.0; s1 += lg >= 2u ? e1 : 0.0; s2 += lg >= 2u ? e2 : 0.0;
-          e0 = __shfl_xor(s0, 16, 64); e1 = __shfl_xor(s1, 16, 64); e2 = __shfl_xor(s2, 16, 64);
-          s0 += lg >= 3u ? e0 : 0.0; s1 += lg >= 3u ? e1 : 0.0; s2 += lg >= 3u ? e2 : 0.0;
-        }
-      }
-    }
-    double y0, y1, y2;
-    if (LOWER) {
-      // couplings l10, l20, l21 (zero where absent)
-      y0 = x0 + s0;
-      y1 = x1 + s1 + (double)wu[k].x * y0;
-      y2 = x2 + s2 + (double)wu[k].y * y0 + (double)wu[k].z * y1;
-    } else {
-      // couplings u01, u02, u12 (zero where absent), reciprocal diagonals; last row first,
-      // rows past the node's zero
-      const unsigned R = fl[k] & 3u;
-      y2 = (R > 2u ? x2 - s2 : 0.0) * rd[k].z;
-      y1 = (R > 1u ? x1 - s1 - (double)wu[k].z * y2 : 0.0) * rd[k].y;
-      y0 = (x0 - s0 - (double)wu[k].x * y1 - (double)wu[k].y * y2) * rd[k].x;
-    }
-    asm volatile("" : "+v"(y0), "+v"(y1), "+v"(y2));        // selected, not branched around
-    const double y = q == 0u ? y0 : (q == 1u ? y1 : y2);
+    const double s = node_sum<M>(q, s0, s1, s2, fl[k] >> 1);
+    const double y = node_solve<LOWER>(x0, s, wu[k], rd[k]);
     // a wave's LDS operations complete in order: the compiler must keep the order, no wait
     asm volatile("" ::: "memory");
-    if (wo[k]) st_lds(wo[k], y);
+    if (fl[k] & 1u) st_lds(xo[k], y);
     asm volatile("" ::: "memory");
   };
   // no branch around a stage, so that every pass issues the same loads and the wait before
@@ -1332,7 +1208,7 @@ __global__ void __launch_bounds__(64) k_block_sweep(const int4* __restrict__ inf
                                                     const VT* __restrict__ vup,
                                                     const uint2* __restrict__ cup,
                                                     const VT* __restrict__ wup,
-                                                    const double4* __restrict__ rdg,
+                                                    const double* __restrict__ rdg,
                                                     const double* rhs, double* out,
                                                     const int* __restrict__ aidx,
                                                     const double* __restrict__ aval)
@@ -1361,12 +1237,12 @@ __global__ void __launch_bounds__(64) k_block_sweep(const int4* __restrict__ inf
   auto lower = [&](auto mode) {
     block_passes<VT, true, decltype(mode)::value, BS_DEPTH>(
         i1.x, tab + tb, desc + i1.y, vlo + 4 * (long long)i2.x, clo + i2.y,
-        wlo + 4 * (long long)ub, nullptr, lane);
+        wlo + 8 * (long long)ub, nullptr, lane);
   };
   auto upper = [&](auto mode) {
     block_passes<VT, false, decltype(mode)::value, BS_DEPTH>(
         i1.z, tab + tb + i1.x + 4 * BS_DEPTH, desc + i1.w, vup + 4 * (long long)i2.z, cup + i2.w,
-        wup + 4 * (long long)ub, rdg + ub, lane);
+        wup + 8 * (long long)ub, rdg + 4 * (long long)ub, lane);
   };
   if (i3.x == 0) lower(std::integral_constant<int, 0>());
   else if (i3.x == 1) lower(std::integral_constant<int, 1>());
@@ -1396,7 +1272,140 @@ __global__ void __launch_bounds__(64) k_block_sweep(const int4* __restrict__ inf
 }
 
 // ---------------------------------------------------------------------------------------
+// node sweeps: one workgroup of several waves per block of any size
+
+constexpr int NS_DEPTH = 4;        // passes whose loads are in flight ahead
+constexpr int NS_WAVES = 4;        // waves per workgroup at most
+constexpr int NS_LDS = 160 * 1024; // LDS of a workgroup at most (a double per live row)
+
+// One triangle of one block by a workgroup of blockDim.x / 64 waves, as block_passes works
+// it, with passes of up to blockDim.x / 4 slots (16 a wave) between LDS barriers.  A row's
+// solved value lives in LDS from its pass to the last pass that reads it: the set-up gives
+// every node LDS places as a linear scan allocates registers (place 0 holds the zero of
+// absent columns), so a block may have far more rows than LDS holds values.  Right-hand
+// sides are read and results written in equation order (a node's rows are consecutive
+// equations); every row has its two couplings inside the node and its reciprocal diagonal.
+// Descriptor: x = first row group of the slot's values | rows << 30 (0: empty); y = first
+// column group | column groups in the slot - 1 << 30; z = the node's first equation | log2 of
+// the node's slots << 30; w = its LDS place.  Group 0 of the streams is zero.
+// What bounds it: one pass per level of nodes, about 1,100 cycles with four waves: the chain
+// through LDS and a barrier, and every wave's loads through one CU's cache (64 bytes a cycle,
+// empty slots included: eight waves take twice as long as four).  FP64, lower + upper sweep: a
+// 200 x 20-cell channel (36,262 rows, 519 levels) 3.9 ms with the staged level sweeps, 0.51 ms
+// here; a dried 80 x 320-cell meander (207,553 rows, 2,145 levels) 16.6 -> 3.2 ms.
+template <class VT, bool LOWER, int M>
+__global__ void __launch_bounds__(64 * NS_WAVES) k_node_sweep(const int4* __restrict__ info,
+                                                              const unsigned* __restrict__ tabs,
+                                                              const uint4* __restrict__ descs,
+                                                              const VT* __restrict__ vals,
+                                                              const uint2* __restrict__ cols,
+                                                              const VT* __restrict__ wcp,
+                                                              const double* __restrict__ rdg,
+                                                              const double* rhs, double* out)
+{
+  using V4 = typename VQuad<VT>::T;
+  using V2 = typename VQuad<VT>::P;
+  constexpr unsigned IM = (1u << 30) - 1;
+  constexpr int D = NS_DEPTH;
+  extern __shared__ double smem[];
+  const int4 in = info[blockIdx.x];                // passes, table, descriptors
+  const int np = in.x;
+  const unsigned* tab = tabs + in.y;
+  const uint4* desc = descs + in.z;
+  const int lane = threadIdx.x & 63;
+  const unsigned slot = threadIdx.x >> 2, q = lane & 3;
+  if (threadIdx.x == 0) smem[0] = 0.0;
+  V4 va[D], vb[D], vc[D];
+  V2 wu[D];
+  double rd[D], hx[D];
+  uint2 ca[D];
+  uint4 dr[D];
+  unsigned wo[D], fl[D], eo[D];            // LDS offset of the result (0: none), log2 of the
+                                           // node's slots, equation of row q
+  auto fetch = [&](unsigned t, uint4* d) {
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+      const unsigned s0 = __builtin_amdgcn_readlane(t, k), s1 = __builtin_amdgcn_readlane(t, k + 1);
+      d[k] = desc[slot < s1 - s0 ? s0 + slot : 0u];
+    }
+  };
+  const unsigned tl = min(lane, D);
+  fetch(tab[tl], dr);
+  tab += D;
+  unsigned tv = tab[tl];
+#pragma unroll
+  for (int k = 0; k < D; k++) {             // the first D passes are empty
+    ca[k] = make_uint2(0u, 0u);
+    va[k] = vb[k] = vc[k] = V4{};
+    wu[k] = V2{};
+    rd[k] = hx[k] = 0.0;
+    wo[k] = fl[k] = eo[k] = 0u;
+    // waited for here (see block_passes)
+    asm volatile("" : "+v"(dr[k].x), "+v"(dr[k].y), "+v"(dr[k].z), "+v"(dr[k].w));
+  }
+  asm volatile("" : "+v"(tv));
+  auto stage = [&](int k) {
+    const uint4 d = dr[k];
+    const unsigned R = d.x >> 30, lg = d.z >> 30, e = d.z & IM;
+    const bool has = q <= d.y >> 30;
+    ca[k] = cols[has ? (d.y & IM) + q : 0u];
+    const V4* v = reinterpret_cast<const V4*>(vals) + (has ? (d.x & IM) + q * R : 0u);
+    va[k] = v[0];
+    vb[k] = v[1];
+    vc[k] = v[2];
+    const unsigned eq = e + (q < R ? q : 0u);      // rows past the node's: its first again
+    wu[k] = reinterpret_cast<const V2*>(wcp)[eq];
+    if (!LOWER) rd[k] = rdg[eq];
+    hx[k] = rhs[eq];
+    wo[k] = q < R && (M == 0 || (slot & ((1u << lg) - 1u)) == 0u) ? (d.w + q) * 8u : 0u;
+    eo[k] = eq;
+    fl[k] = lg;
+  };
+  auto pass = [&](int k) {
+    const double xa = ld_lds((ca[k].x & 0xffffu) * 8u), xc = ld_lds((ca[k].x >> 16) * 8u);
+    const double xd = ld_lds((ca[k].y & 0xffffu) * 8u), xe = ld_lds((ca[k].y >> 16) * 8u);
+    double s0 = (double)va[k].x * xa, s1 = (double)vb[k].x * xa, s2 = (double)vc[k].x * xa;
+    s0 += (double)va[k].y * xc; s1 += (double)vb[k].y * xc; s2 += (double)vc[k].y * xc;
+    s0 += (double)va[k].z * xd; s1 += (double)vb[k].z * xd; s2 += (double)vc[k].z * xd;
+    s0 += (double)va[k].w * xe; s1 += (double)vb[k].w * xe; s2 += (double)vc[k].w * xe;
+    const double s = node_sum<M>(q, s0, s1, s2, fl[k]);
+    const double y = node_solve<LOWER>(hx[k], s, wu[k], rd[k]);
+    if (wo[k]) {
+      st_lds(wo[k], y);
+      out[eo[k]] = y;
+    }
+    lds_barrier();
+  };
+  lds_barrier();
+  for (int l0 = -D; l0 < np; l0 += D) {
+    uint4 dn[D];
+    fetch(tv, dn);
+    tab += D;
+    const unsigned tn = tab[tl];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < D; k++) {
+      pass(k);
+      stage(k);
+    }
+#pragma unroll
+    for (int k = 0; k < D; k++) dr[k] = dn[k];
+    tv = tn;
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // host set-up
+
+// RMX_SWEEP selects the sweep kernels (tuning and comparison), read when a system is set up
+// and at every application: 1 the staged level sweeps, 2 (default) the block sweeps where
+// every block has at most BS_ROWS rows, else the node sweeps where the rows alive at a time
+// fit LDS, else 1.
+static int sweep_variant()
+{
+  const char* e = getenv("RMX_SWEEP");
+  return e ? atoi(e) : 2;
+}
 
 // Level sets of the lower or upper dependency graph of rows [a, e), entries with a column
 // outside [a, e) or (with `seg`) in another segment ignored.
@@ -1432,9 +1441,10 @@ static void levels(int a, int e, const std::vector<int>& rp, const std::vector<i
   else { for (int i = e - 1; i >= a; i--) rows[fill[lev[i]]++] = i; }
 }
 
-// Packed layout of one sweep over all blocks.
+// Packed layout of one sweep over all blocks; without `full` only its counts (the block or
+// node sweeps run).
 static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>& order,
-                        hipStream_t s, int cap)
+                        hipStream_t s, int cap, bool full)
 {
   const int n = I.n, nb = I.nblk;
   const std::vector<int>& rp = I.h_rp;
@@ -1477,15 +1487,18 @@ static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>&
            (!sg || I.seg[c] == I.seg[i]);
   };
   std::vector<int> prs(n + 1, 0);
-  for (int r = 0; r < n; r++) {
-    const int i = prow[r];
-    int k = 0;
-    for (int q = rp[i] + 1; q < rp[i + 1]; q++) k += keep(i, cl[q]);
-    prs[r + 1] = prs[r] + k;
-  }
-  const long long ne = prs[n];
-  std::vector<int> pcol(ne), psrc(ne);
   parallel_for(n, [&](long long a, long long b) {
+    for (long long r = a; r < b; r++) {
+      const int i = prow[r];
+      int k = 0;
+      for (int q = rp[i] + 1; q < rp[i + 1]; q++) k += keep(i, cl[q]);
+      prs[r + 1] = k;
+    }
+  });
+  for (int r = 0; r < n; r++) prs[r + 1] += prs[r];
+  const long long ne = prs[n];
+  std::vector<int> pcol(full ? ne : 0), psrc(full ? ne : 0);
+  if (full) parallel_for(n, [&](long long a, long long b) {
     for (long long r = a; r < b; r++) {
       const int i = prow[r];
       int j = prs[r];
@@ -1502,9 +1515,13 @@ static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>&
     fprintf(stderr, "[rmx] %s sweep, %d strip(s) x %d segment(s): %d levels (longest strip), "
             "%.1f rows/level, max %d, %lld entries\n", lower ? "lower" : "upper", nb, I.nseg,
             nlev_tot, (double)n / std::max(1, blev[nb]), maxnr, ne);
-  S.blev.upload(blev, s); S.bpos.upload(bpos, s); S.lev_ptr.upload(levp, s);
-  S.prs.upload(prs, s); S.prow.upload(prow, s); S.pcol.upload(pcol, s); S.psrc.upload(psrc, s);
   S.xp.alloc(n);
+  S.packed = full;
+  if (full) {
+    S.blev.upload(blev, s); S.bpos.upload(bpos, s); S.lev_ptr.upload(levp, s);
+    S.prs.upload(prs, s); S.prow.upload(prow, s); S.pcol.upload(pcol, s); S.psrc.upload(psrc, s);
+    HIPCHECK(hipStreamSynchronize(s));
+  }
   order = prow;
 }
 
@@ -1554,7 +1571,7 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
     int npass[2] = {0, 0}, lgmax[2] = {0, 0};   // lgmax: log2 of the most slots of a node
     std::vector<unsigned short> col[2];  // columns, LDS byte offsets, 4 per group
     std::vector<int> src[2];             // CSR position of every value (4 per row group)
-    std::vector<int> usrc[2];            // unit coupling sources (4 per unit)
+    std::vector<int> usrc[2];            // unit coupling sources (2 per row, 4 rows per unit)
     std::vector<int> dsrc;               // unit diagonal sources (4 per unit)
     bool fits = true;
   };
@@ -1685,7 +1702,7 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
           src.assign(12, -1);
           desc.assign(1, uint2{ 0u, 0u });     // the empty slot
           int cur = -1, nrow = 0, npair = 0, nslot = 0;
-          P.usrc[t].assign(4 * ord[t].size(), -1);
+          P.usrc[t].assign(8 * ord[t].size(), -1);
           if (!lower) P.dsrc.assign(4 * ord[t].size(), -1);
           for (int U : ord[t]) {
             const int r0 = ustart[U], nr = ustart[U + 1] - r0;
@@ -1732,21 +1749,15 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
                                     (unsigned)(c0 & BS_CM) | (unsigned)uidx[U] << 16 |
                                         (unsigned)nr << 28 | (unsigned)ulg[t][U] << 30 });
             }
-            int* us4 = &P.usrc[t][4 * (size_t)uidx[U]];
-            const int r1 = r0 + std::min(1, nr - 1), r2 = r0 + std::min(2, nr - 1);
-            if (lower) {
-              us4[0] = nr > 1 ? find(r1, r0) : -1;
-              us4[1] = nr > 2 ? find(r2, r0) : -1;
-              us4[2] = nr > 2 ? find(r2, r1) : -1;
-            } else {
-              us4[0] = nr > 1 ? find(r0, r1) : -1;
-              us4[1] = nr > 2 ? find(r0, r2) : -1;
-              us4[2] = nr > 2 ? find(r1, r2) : -1;
-              int* ds4 = &P.dsrc[4 * (size_t)uidx[U]];
-              ds4[0] = rp[r0];
-              if (nr > 1) ds4[1] = rp[r1];
-              if (nr > 2) ds4[2] = rp[r2];
-            }
+            // row q's couplings inside the unit: lower (l_q0, l_q1), upper (u_q1, u_q2)
+            int* us = &P.usrc[t][8 * (size_t)uidx[U]];
+            for (int j = 0; j < nr; j++)
+              for (int k = 0; k < 2; k++) {
+                const int o = lower ? k : k + 1;
+                if (o < nr && (lower ? o < j : o > j)) us[2 * j + k] = find(r0 + j, r0 + o);
+              }
+            if (!lower)
+              for (int j = 0; j < nr; j++) P.dsrc[4 * (size_t)uidx[U] + j] = rp[r0 + j];
             nrow += nr;
             npair += pairs;
             nslot += ns;
@@ -1770,7 +1781,7 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
       npass += P.npass[t];
       ntab += P.tab[t].size();
     }
-    nunit += P.usrc[0].size() / 4;
+    nunit += P.usrc[0].size() / 8;
     lds = std::max(lds, 8 * (P.rows.size() + 3));
   }
   const long long lim = INT_MAX - BS_PAD;
@@ -1784,7 +1795,7 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
   for (int t = 0; t < 2; t++) {
     src[t].assign(4 * ((size_t)nvg[t] + BS_PAD), -1);
     col[t].assign(4 * ((size_t)ncg[t] + BS_PAD), 0);
-    usrc[t].assign((size_t)4 * nunit, -1);
+    usrc[t].assign((size_t)8 * nunit, -1);
   }
   long long k = 0, rb = 0, sb = 0, tb = 0, ub = 0, cg[2] = {0, 0}, vg[2] = {0, 0};
   for (const Part& P : parts) {
@@ -1803,12 +1814,12 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
       sb += P.desc[t].size();
       std::copy(P.col[t].begin(), P.col[t].end(), col[t].begin() + 4 * cg[t]);
       std::copy(P.src[t].begin(), P.src[t].end(), src[t].begin() + 4 * vg[t]);
-      std::copy(P.usrc[t].begin(), P.usrc[t].end(), usrc[t].begin() + 4 * ub);
+      std::copy(P.usrc[t].begin(), P.usrc[t].end(), usrc[t].begin() + 8 * ub);
       cg[t] += P.col[t].size() / 4;
       vg[t] += P.src[t].size() / 4;
     }
     std::copy(P.dsrc.begin(), P.dsrc.end(), dsrc.begin() + 4 * ub);
-    k++; rb += m; ub += P.usrc[0].size() / 4;
+    k++; rb += m; ub += P.usrc[0].size() / 8;
   }
   B.nb = (int)nb; B.lds = (lds + 15) & ~(size_t)15;
   B.ne_lo = std::count_if(src[0].begin(), src[0].end(), [](int q) { return q >= 0; });
@@ -1824,6 +1835,251 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
     fprintf(stderr, "[rmx] block sweeps: %lld groups of blocks, %lld nodes, %lld + %lld entries (%lld + "
             "%lld padded), %.1f passes per group, %zu bytes LDS\n", nb, nunit, B.ne_lo, B.ne_up,
             4 * nvg[0], 4 * nvg[1], (double)npass / nb, B.lds);
+}
+
+// Node sweep layout (k_node_sweep) of one triangle over all strips.  Units are those of
+// build_blocks (runs of rows of one node in one segment, at most 3); a unit's columns lie in
+// its rows' strip and segment.  Units are scheduled by levels, as early or as late as their
+// dependencies allow, whichever keeps fewer rows alive; a unit's LDS places are free again
+// after the last level that reads them.  Off when a strip's live rows do not fit LDS.
+static void build_nodes(NodeSweep& S, const Ilu& I, bool lower, const std::vector<int>* group,
+                        const std::vector<int>& scol, const std::vector<unsigned char>& spos,
+                        hipStream_t s)
+{
+  S.on = false;
+  const int n = I.n, nstrip = I.nblk;
+  const std::vector<int>& rp = I.h_rp;
+  if (I.nnz >= (1LL << 29) || n >= (1 << 30) - 64) return;
+  const bool sg = !I.seg.empty();
+  auto segof = [&](int i) { return sg ? I.seg[i] : 0; };
+  // units, ascending rows; the strip of every unit
+  std::vector<int> ustart, uof(n), ustrip, ub(nstrip + 1, 0);
+  auto one_set = [&](int u0, int u1) {          // one set of columns: row u0 stands for all
+    for (int i = u0 + 1; i < u1; i++)
+      if (rp[i + 1] - rp[i] != rp[u0 + 1] - rp[u0] ||
+          !std::equal(scol.begin() + rp[u0], scol.begin() + rp[u0 + 1], scol.begin() + rp[i]))
+        return false;
+    return true;
+  };
+  for (int b = 0; b < nstrip; b++) {
+    ub[b] = (int)ustart.size();
+    for (int i = I.bstart[b]; i < I.bstart[b + 1];) {
+      int j = i + 1;
+      while (j < I.bstart[b + 1] && group && (*group)[j] == (*group)[i] && segof(j) == segof(i) &&
+             j < i + 3) j++;
+      // rows of different columns, which could be more than a unit takes: single rows
+      if (j > i + 1 && !one_set(i, j)) {
+        int w = 0;
+        for (int k = i; k < j; k++) w += rp[k + 1] - rp[k];
+        if (w > BS_MAXW) j = i + 1;
+      }
+      ustart.push_back(i);
+      ustrip.push_back(b);
+      i = j;
+    }
+  }
+  const int nu = (int)ustart.size();
+  ub[nstrip] = nu;
+  ustart.push_back(n);
+  std::vector<unsigned char> uone(nu), ulg(nu, 0);
+  std::vector<int> uw(nu, 0);
+  // columns of a unit, descending (uc), and the units they belong to
+  auto cols_of = [&](int U, std::vector<int>& uc) {
+    const int u0 = ustart[U], u1 = ustart[U + 1], a = I.bstart[ustrip[U]], e = I.bstart[ustrip[U] + 1];
+    uc.clear();
+    for (int i = u0; i < (uone[U] ? u0 + 1 : u1); i++) {
+      const int* b = scol.data() + rp[i];
+      const int* z = scol.data() + rp[i + 1];
+      if (lower) { z = std::lower_bound(b, z, u0); b = std::lower_bound(b, z, a); }
+      else { b = std::lower_bound(b, z, u1); z = std::lower_bound(b, z, e); }
+      for (const int* c = z; c-- > b;)
+        if (!sg || segof(*c) == segof(i)) uc.push_back(*c);
+    }
+    if (!uone[U]) {
+      std::sort(uc.begin(), uc.end(), std::greater<int>());
+      uc.erase(std::unique(uc.begin(), uc.end()), uc.end());
+    }
+  };
+  parallel_for(nu, [&](long long u0, long long u1) {
+    std::vector<int> uc;
+    for (long long U = u0; U < u1; U++) {
+      uone[U] = one_set(ustart[U], ustart[U + 1]);
+      for (int i = ustart[U]; i < ustart[U + 1]; i++) uof[i] = (int)U;
+      cols_of((int)U, uc);
+      uw[U] = (int)uc.size();
+      while ((16 << ulg[U]) < uw[U]) ulg[U]++;
+    }
+  });
+  // units that every unit reads
+  std::vector<long long> dp(nu + 1, 0);
+  std::vector<int> dep;
+  {
+    std::vector<int> cnt(nu, 0);
+    auto units = [&](int U, std::vector<int>& uc, int* out) {
+      cols_of(U, uc);
+      int last = -1, k = 0;
+      for (int c : uc)
+        if (uof[c] != last) { last = uof[c]; if (out) out[k] = last; k++; }
+      return k;
+    };
+    parallel_for(nu, [&](long long u0, long long u1) {
+      std::vector<int> uc;
+      for (long long U = u0; U < u1; U++) cnt[U] = units((int)U, uc, nullptr);
+    });
+    for (int U = 0; U < nu; U++) dp[U + 1] = dp[U] + cnt[U];
+    dep.resize(dp[nu]);
+    parallel_for(nu, [&](long long u0, long long u1) {
+      std::vector<int> uc;
+      for (long long U = u0; U < u1; U++) units((int)U, uc, dep.data() + dp[U]);
+    });
+  }
+  std::vector<int> place(nu, 0), order(nu), nlev(nstrip, 0), live(nstrip, 1), lbeg;
+  std::vector<std::vector<int>> lptr(nstrip);    // level offsets of a strip into its order
+  parallel_for(nstrip, [&](long long b0, long long b1) {
+    for (long long b = b0; b < b1; b++) {
+      const int a = ub[b], e = ub[b + 1], m = e - a;
+      if (m == 0) { lptr[b].assign(1, 0); continue; }
+      std::vector<int> lev[2] = { std::vector<int>(m, 0), std::vector<int>(m, INT_MAX) };
+      int L = 0;
+      for (int k = 0; k < m; k++) {
+        const int U = lower ? a + k : e - 1 - k;
+        int l = 0;
+        for (long long q = dp[U]; q < dp[U + 1]; q++) l = std::max(l, lev[0][dep[q] - a] + 1);
+        lev[0][U - a] = l;
+        L = std::max(L, l + 1);
+      }
+      for (int k = m - 1; k >= 0; k--) {
+        const int U = lower ? a + k : e - 1 - k;
+        int& l = lev[1][U - a];
+        if (l == INT_MAX) l = lev[0][U - a];     // nothing reads it
+        for (long long q = dp[U]; q < dp[U + 1]; q++)
+          lev[1][dep[q] - a] = std::min(lev[1][dep[q] - a], l - 1);
+      }
+      // order by level, a level's units by falling slot count (aligned to their number); LDS
+      // places as a linear scan gives them
+      std::vector<int> best, bplace, bptr;
+      for (int t = 0; t < 2; t++) {
+        const std::vector<int>& lv = lev[t];
+        std::vector<int> last(lv), ptr(4 * (size_t)L + 1, 0), ord(m), dptr(L + 1, 0), dl(m), pl(m);
+        for (int U = a; U < e; U++)
+          for (long long q = dp[U]; q < dp[U + 1]; q++)
+            last[dep[q] - a] = std::max(last[dep[q] - a], lv[U - a]);
+        for (int k = 0; k < m; k++) { ptr[4 * lv[k] + 3 - ulg[a + k] + 1]++; dptr[last[k] + 1]++; }
+        for (int l = 0; l < 4 * L; l++) ptr[l + 1] += ptr[l];
+        for (int l = 0; l < L; l++) dptr[l + 1] += dptr[l];
+        std::vector<int> lp(L + 1);
+        for (int l = 0; l <= L; l++) lp[l] = ptr[4 * l];
+        {
+          std::vector<int> f(ptr), g(dptr);
+          for (int k = 0; k < m; k++) { ord[f[4 * lv[k] + 3 - ulg[a + k]]++] = k; dl[g[last[k]]++] = k; }
+        }
+        std::vector<int> freed[4];
+        int top = 1;
+        for (int l = 0; l < L; l++) {
+          for (int q = lp[l]; q < lp[l + 1]; q++) {
+            const int k = ord[q], w = ustart[a + k + 1] - ustart[a + k];
+            if (!freed[w].empty()) { pl[k] = freed[w].back(); freed[w].pop_back(); }
+            else { pl[k] = top; top += w; }
+          }
+          for (int q = dptr[l]; q < dptr[l + 1]; q++)
+            freed[ustart[a + dl[q] + 1] - ustart[a + dl[q]]].push_back(pl[dl[q]]);
+        }
+        if (t == 0 || top < live[b]) { live[b] = top; best.swap(ord); bplace.swap(pl); bptr.swap(lp); }
+      }
+      for (int k = 0; k < m; k++) { order[a + k] = a + best[k]; place[a + k] = bplace[k]; }
+      lptr[b].swap(bptr);
+      nlev[b] = L;
+    }
+  });
+  // waves: the fewest that hold an average level in one pass (lower + upper sweep, FP64, 1 / 2 /
+  // 4 / 8 waves: 30 slots a level 842 / 554 / 517 / 816 us, 11 slots 627 / 399 / 575 / 935, 59 and
+  // 54 slots 5.3 / 3.5 / 3.2 / 3.7 ms, 104 slots 21 / 14.3 / 14.6 / 15.3 ms): at most four, past
+  // which a pass takes longer by what it saves in passes
+  long long slots = 0, levels = 0;
+  int lgmax = 0, maxlive = 1;
+  for (int U = 0; U < nu; U++) { slots += 1 << ulg[U]; lgmax = std::max(lgmax, (int)ulg[U]); }
+  for (int b = 0; b < nstrip; b++) { levels += nlev[b]; maxlive = std::max(maxlive, live[b]); }
+  S.lds = 8 * ((size_t)maxlive + 2);
+  if (maxlive > 65533 || S.lds > (size_t)NS_LDS) return;
+  S.waves = 1;
+  while (S.waves < NS_WAVES && 16LL * S.waves * levels < slots) S.waves *= 2;
+  if (const char* e = getenv("RMX_NODE_WAVES")) S.waves = std::max(1, std::min(NS_WAVES, atoi(e)));
+  const int cap = 16 * S.waves;
+  // passes, and where every unit's slots, column groups and row groups start (descriptor 0 of
+  // a strip is empty; column group 0 and row groups 0 to 2 are zero)
+  std::vector<int4> info(nstrip);
+  std::vector<unsigned> tab;
+  std::vector<unsigned> us0(nu), uc0(nu), uv0(nu);
+  long long nd = 0, nc = 1, nv = 3;
+  for (int b = 0; b < nstrip; b++) {
+    const long long d0 = nd++;
+    const size_t t0 = tab.size();
+    for (int l = 0; l < nlev[b]; l++) {
+      int ns = cap;
+      for (int q = lptr[b][l]; q < lptr[b][l + 1]; q++) {
+        const int U = order[ub[b] + q], ng = (uw[U] + 3) / 4;
+        if (ns + (1 << ulg[U]) > cap) { tab.push_back((unsigned)(nd - d0)); ns = 0; }
+        ns += 1 << ulg[U];
+        us0[U] = (unsigned)nd; uc0[U] = (unsigned)nc; uv0[U] = (unsigned)nv;
+        nd += 1 << ulg[U];
+        nc += ng;
+        nv += (long long)ng * (ustart[U + 1] - ustart[U]);
+      }
+    }
+    info[b] = int4{ (int)(tab.size() - t0), (int)t0, (int)d0, 0 };
+    tab.resize(tab.size() + 4 * NS_DEPTH, (unsigned)(nd - d0));   // repeated past the last pass
+  }
+  if (nd >= INT_MAX || nv >= (1 << 30) - BS_PAD) return;
+  const size_t npass = tab.size() - (size_t)nstrip * 4 * NS_DEPTH;
+  tab.resize(tab.size() + 64, 0u);
+  std::vector<uint4> desc(nd, uint4{ 0u, 0u, 0u, 0u });
+  std::vector<unsigned short> col(4 * (size_t)(nc + BS_PAD), 0);
+  std::vector<int> src(4 * (size_t)(nv + BS_PAD), -1), wsrc(2 * (size_t)n, -1);
+  parallel_for(nu, [&](long long a, long long z) {
+    std::vector<int> uc;
+    auto find = [&](int r, int c) {
+      const auto b = scol.begin() + rp[r], e = scol.begin() + rp[r + 1];
+      const auto it = std::lower_bound(b, e, c);
+      return it != e && *it == c ? rp[r] + (int)spos[it - scol.begin()] : -1;
+    };
+    for (long long U = a; U < z; U++) {
+      const int r0 = ustart[U], nr = ustart[U + 1] - r0;
+      cols_of((int)U, uc);
+      const int w = (int)uc.size(), ng = (w + 3) / 4;
+      for (int k = 0; k < w; k++)
+        col[4 * (size_t)uc0[U] + k] = (unsigned short)(place[uof[uc[k]]] + (uc[k] - ustart[uof[uc[k]]]));
+      for (int j = 0; j < nr; j++) {
+        const int* b = scol.data() + rp[r0 + j];
+        const int* c = scol.data() + rp[r0 + j + 1];
+        for (int k = 0; k < w; k++) {              // both descending
+          while (c > b && c[-1] > uc[k]) c--;
+          if (c > b && c[-1] == uc[k])
+            src[4 * (size_t)uv0[U] + ((size_t)(k / 4) * nr + j) * 4 + k % 4] =
+                rp[r0 + j] + (int)spos[c - 1 - scol.data()];
+        }
+      }
+      for (int j = 0; j < (1 << ulg[U]); j++) {
+        const int g = std::max(0, std::min(4, ng - 4 * j));
+        desc[us0[U] + j] = uint4{ (g ? uv0[U] + (unsigned)(4 * j * nr) : 0u) | (unsigned)nr << 30,
+                                  (g ? uc0[U] + (unsigned)(4 * j) : 0u) | (unsigned)std::max(0, g - 1) << 30,
+                                  (unsigned)r0 | (unsigned)ulg[U] << 30, (unsigned)place[U] };
+      }
+      for (int j = 0; j < nr; j++)                 // as in build_blocks
+        for (int k = 0; k < 2; k++) {
+          const int o = lower ? k : k + 1;
+          if (o < nr && (lower ? o < j : o > j)) wsrc[2 * (size_t)(r0 + j) + k] = find(r0 + j, r0 + o);
+        }
+    }
+  });
+  S.lgmax = std::min(2, lgmax);
+  S.info.upload(info, s); S.tab.upload(tab, s); S.desc.upload(desc, s);
+  S.cols.upload(col, s); S.src.upload(src, s); S.wsrc.upload(wsrc, s);
+  HIPCHECK(hipStreamSynchronize(s));
+  S.on = true;
+  if (getenv("RMX_DEBUG"))
+    fprintf(stderr, "[rmx] %s node sweep: %d strip(s), %d nodes, %lld slots, %lld levels, %zu "
+            "passes, %d waves, %d LDS places\n", lower ? "lower" : "upper", nstrip, nu, slots,
+            levels, npass, S.waves, maxlive);
 }
 
 // Segment of every row: each strip [bstart[b], bstart[b+1]) is cut into nseg parts of
@@ -1872,9 +2128,11 @@ std::vector<int> cut_segments(const std::vector<int>& bstart, const std::vector<
 // equation) a cut moves forward to the next row of another node, so the U, V, H equations
 // of one node stay in one strip.  level_cap > 0 splits the sweeps' levels into parts of at
 // most that many rows.
+// `unit`: rows of one unit of the block and node sweeps have one value (the node, or a run of
+// rows with one set of columns).
 void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>& cl, int nblk,
-               const std::vector<int>* group, hipStream_t s, const HostModel* hm, int nseg,
-               int level_cap)
+               const std::vector<int>* group, const std::vector<int>& unit, hipStream_t s,
+               const HostModel* hm, int nseg, int level_cap)
 {
   I.ready = I.fac64 = I.fac32 = false;
   I.n = n;
@@ -1963,15 +2221,25 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   // loaded inside the level instead of one level ahead
   int cap = level_cap;
   if (const char* e = getenv("RMX_LEVEL_CAP")) cap = std::max(0, atoi(e));
+  build_blocks(I, &unit, scol, spos, s);
+  I.nlo.on = I.nup.on = false;
+  if (!I.bs.on) {
+    build_nodes(I.nlo, I, true, &unit, scol, spos, s);
+    if (I.nlo.on) build_nodes(I.nup, I, false, &unit, scol, spos, s);
+  }
+  // the level sweeps where neither runs, or RMX_SWEEP asks for them
+  const bool full = !(I.bs.on || (I.nlo.on && I.nup.on)) || sweep_variant() < 2;
   std::vector<int> olo, oup;
-  build_sweep(I.lo, I, true, olo, s, cap);
-  build_sweep(I.up, I, false, oup, s, cap);
-  build_blocks(I, group, scol, spos, s);
+  build_sweep(I.lo, I, true, olo, s, cap, full);
+  build_sweep(I.up, I, false, oup, s, cap, full);
   // forward position (global, concatenated) of the row at each backward position
-  std::vector<int> fpos(n), f2b(n);
-  for (int r = 0; r < n; r++) fpos[olo[r]] = r;
-  for (int r = 0; r < n; r++) f2b[r] = fpos[oup[r]];
-  I.fwd2bwd.upload(f2b, s);
+  if (full) {
+    std::vector<int> fpos(n), f2b(n);
+    for (int r = 0; r < n; r++) fpos[olo[r]] = r;
+    for (int r = 0; r < n; r++) f2b[r] = fpos[oup[r]];
+    I.fwd2bwd.upload(f2b, s);
+    HIPCHECK(hipStreamSynchronize(s));
+  }
   HIPCHECK(hipStreamSynchronize(s));
   I.ready = true;
 }
@@ -2002,6 +2270,14 @@ template <> BSvals<float> bsvals<float>(BlockSweep& B)
 {
   return { &B.vlo32, &B.vup32, &B.wlo32, &B.wup32, &B.rdg32 };
 }
+// node sweep values of one precision: entries, couplings, reciprocal diagonals (upper)
+template <class VT> struct NSvals {
+  DBuf<VT> *v, *w;
+  DBuf<double>* rdg;
+};
+template <class VT> static NSvals<VT> nsvals(NodeSweep& S);
+template <> NSvals<double> nsvals<double>(NodeSweep& S) { return { &S.v64, &S.w64, &S.rdg64 }; }
+template <> NSvals<float> nsvals<float>(NodeSweep& S) { return { &S.v32, &S.w32, &S.rdg32 }; }
 template <class VT> static DBuf<VT>& PDbuf(Ilu& I);
 template <> DBuf<double>& PDbuf<double>(Ilu& I) { return I.pdg64; }
 template <> DBuf<float>& PDbuf<float>(Ilu& I) { return I.pdg32; }
@@ -2102,15 +2378,29 @@ static void factor_t(Ctx& c, Ilu& I, const VT* A)
   kt_end(c, kt);
   }
   HIPCHECK(hipGetLastError());
-  DBuf<VT>& pl = PLbuf<VT>(I);
-  DBuf<VT>& pu = PUbuf<VT>(I);
-  DBuf<VT>& pd = PDbuf<VT>(I);
-  pl.alloc(std::max<long long>(I.lo.ne, 1));
-  pu.alloc(std::max<long long>(I.up.ne, 1));
-  pd.alloc(I.n);
-  if (I.lo.ne) k_pack<VT><<<4096, 256, 0, c.stream>>>(I.lo.ne, I.lo.psrc.p, LU.p, pl.p);
-  if (I.up.ne) k_pack<VT><<<4096, 256, 0, c.stream>>>(I.up.ne, I.up.psrc.p, LU.p, pu.p);
-  k_pack_diag<VT><<<(I.n + 255) / 256, 256, 0, c.stream>>>(I.n, I.up.prow.p, I.rp.p, LU.p, pd.p);
+  if (I.lo.packed) {                            // level sweeps
+    DBuf<VT>& pl = PLbuf<VT>(I);
+    DBuf<VT>& pu = PUbuf<VT>(I);
+    DBuf<VT>& pd = PDbuf<VT>(I);
+    pl.alloc(std::max<long long>(I.lo.ne, 1));
+    pu.alloc(std::max<long long>(I.up.ne, 1));
+    pd.alloc(I.n);
+    if (I.lo.ne) k_pack<VT><<<4096, 256, 0, c.stream>>>(I.lo.ne, I.lo.psrc.p, LU.p, pl.p);
+    if (I.up.ne) k_pack<VT><<<4096, 256, 0, c.stream>>>(I.up.ne, I.up.psrc.p, LU.p, pu.p);
+    k_pack_diag<VT><<<(I.n + 255) / 256, 256, 0, c.stream>>>(I.n, I.up.prow.p, I.rp.p, LU.p, pd.p);
+  }
+  if (I.nlo.on && I.nup.on) {                   // node sweeps
+    for (NodeSweep* S : { &I.nlo, &I.nup }) {
+      const NSvals<VT> V = nsvals<VT>(*S);
+      V.v->alloc(S->src.n);
+      V.w->alloc(S->wsrc.n);
+      k_pack<VT><<<4096, 256, 0, c.stream>>>((long long)S->src.n, S->src.p, LU.p, V.v->p);
+      k_pack<VT><<<1024, 256, 0, c.stream>>>((long long)S->wsrc.n, S->wsrc.p, LU.p, V.w->p);
+    }
+    DBuf<double>& rd = *nsvals<VT>(I.nup).rdg;
+    rd.alloc(I.n);
+    k_rcp_diag<VT><<<(I.n + 255) / 256, 256, 0, c.stream>>>(I.n, I.rp.p, LU.p, rd.p);
+  }
   if (I.bs.on) {                                // block sweeps: values in their entry order
     BlockSweep& B = I.bs;
     const BSvals<VT> V = bsvals<VT>(B);
@@ -2147,37 +2437,26 @@ void ilu_factor(Ctx& c, Ilu& I, int prec)
   }
 }
 
-template <class VT, int V>
+template <class VT>
 static void launch_sweeps(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t* ev,
                           const int* aidx, const double* aval)
 {
-  // V = 1: staged pipeline, 4 lanes per row with 6 register entries each, 512 threads (two
-  // workgroups per compute unit by registers and LDS); V = 0: one-deep prefetch, 8 lanes
-  // per row, 1024 threads
+  // 4 lanes per row with 12 / 6 register entries each, 512 threads (two workgroups per compute
+  // unit by registers and LDS)
   const int nb = I.nblk;
   const int nt = STAGE_THREADS;
   if (ev) HIPCHECK(hipEventRecord(ev[0], c.stream));
   const double vb = (double)sizeof(VT) + 4.0;
   int kt = kt_begin(c, KT_SWEEP_LO, (double)I.lo.ne * vb + 20.0 * I.n);
-  if constexpr (V == 1)
-    k_sweep_stage<VT, true, 4, 12><<<nb, nt, 0, c.stream>>>(I.lo.blev.p, I.lo.bpos.p,
-        I.lo.lev_ptr.p, I.lo.prs.p, I.lo.pcol.p, PLbuf<VT>(I).p, nullptr, I.lo.prow.p, b, nullptr,
-        nullptr, I.lo.xp.p, nullptr, nullptr);
-  else
-    k_sweep<VT, true, SG, SKR><<<nb, 1024, 0, c.stream>>>(I.lo.blev.p, I.lo.bpos.p,
-        I.lo.lev_ptr.p, I.lo.prs.p, I.lo.pcol.p, PLbuf<VT>(I).p, nullptr, I.lo.prow.p, b, nullptr,
-        nullptr, I.lo.xp.p);
+  k_sweep_stage<VT, true, 4, 12><<<nb, nt, 0, c.stream>>>(I.lo.blev.p, I.lo.bpos.p,
+      I.lo.lev_ptr.p, I.lo.prs.p, I.lo.pcol.p, PLbuf<VT>(I).p, nullptr, I.lo.prow.p, b, nullptr,
+      nullptr, I.lo.xp.p, nullptr, nullptr);
   kt_end(c, kt);
   if (ev) HIPCHECK(hipEventRecord(ev[1], c.stream));
   kt = kt_begin(c, KT_SWEEP_UP, (double)I.up.ne * vb + 24.0 * I.n);
-  if constexpr (V == 1)
-    k_sweep_stage<VT, false, 4, 6><<<nb, nt, 0, c.stream>>>(I.up.blev.p, I.up.bpos.p,
-        I.up.lev_ptr.p, I.up.prs.p, I.up.pcol.p, PUbuf<VT>(I).p, PDbuf<VT>(I).p, I.fwd2bwd.p,
-        I.lo.xp.p, I.up.prow.p, x, I.up.xp.p, aidx, aval);
-  else
-    k_sweep<VT, false, SG, SKR><<<nb, 1024, 0, c.stream>>>(I.up.blev.p, I.up.bpos.p,
-        I.up.lev_ptr.p, I.up.prs.p, I.up.pcol.p, PUbuf<VT>(I).p, PDbuf<VT>(I).p, I.fwd2bwd.p,
-        I.lo.xp.p, I.up.prow.p, x, I.up.xp.p);
+  k_sweep_stage<VT, false, 4, 6><<<nb, nt, 0, c.stream>>>(I.up.blev.p, I.up.bpos.p,
+      I.up.lev_ptr.p, I.up.prs.p, I.up.pcol.p, PUbuf<VT>(I).p, PDbuf<VT>(I).p, I.fwd2bwd.p,
+      I.lo.xp.p, I.up.prow.p, x, I.up.xp.p, aidx, aval);
   kt_end(c, kt);
   if (ev) HIPCHECK(hipEventRecord(ev[2], c.stream));
   HIPCHECK(hipGetLastError());
@@ -2191,17 +2470,16 @@ static void launch_blocks(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t
   BlockSweep& B = I.bs;
   const BSvals<VT> V = bsvals<VT>(B);
   if (ev) HIPCHECK(hipEventRecord(ev[0], c.stream));
-  // algorithmic bytes: entry values, a 2-byte column per node and column, per node 8 coupling
-  // values and 3 FP64 reciprocal diagonals (stored as 4), per row the gather index, right-hand
+  // algorithmic bytes: entry values, a 2-byte column per node and column, per node 16 coupling
+  // values and 4 FP64 reciprocal diagonals (those of 3 rows used), per row the gather index, right-hand
   // side and result, per slot its descriptor, per pass its table entry, the folded prolongation
   const double v = (double)sizeof(VT);
-  const double bytes = (double)(B.ne_lo + B.ne_up) * v + 2.0 * B.ncol + (double)B.nunit * (32.0 + 8.0 * v) +
+  const double bytes = (double)(B.ne_lo + B.ne_up) * v + 2.0 * B.ncol + (double)B.nunit * (32.0 + 16.0 * v) +
                        8.0 * B.nslot + 20.0 * I.n + 4.0 * B.npass + (aidx ? 12.0 * I.n : 0.0);
   const int kt = kt_begin(c, KT_SWEEP_BLK, bytes);
   k_block_sweep<VT><<<B.nb, 64, B.lds, c.stream>>>(B.info.p, B.gidx.p, B.tab.p, B.desc.p,
       V.vlo->p, reinterpret_cast<const uint2*>(B.clo.p), V.wlo->p, V.vup->p,
-      reinterpret_cast<const uint2*>(B.cup.p), V.wup->p,
-      reinterpret_cast<const double4*>(V.rdg->p), b, x, aidx, aval);
+      reinterpret_cast<const uint2*>(B.cup.p), V.wup->p, V.rdg->p, b, x, aidx, aval);
   kt_end(c, kt);
   if (ev) {
     HIPCHECK(hipEventRecord(ev[1], c.stream));
@@ -2210,12 +2488,24 @@ static void launch_blocks(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t
   HIPCHECK(hipGetLastError());
 }
 
-// RMX_SWEEP selects the sweep kernels (tuning and comparison): 0 the one-deep strip sweep,
-// 1 the staged strip sweep, 2 (default) the block sweeps where the layout exists, else 1.
-static int sweep_variant()
+template <class VT, bool LOWER>
+static void launch_nodes(Ctx& c, Ilu& I, NodeSweep& S, const double* b, double* x)
 {
-  const char* e = getenv("RMX_SWEEP");
-  return e ? atoi(e) : 2;
+  const NSvals<VT> V = nsvals<VT>(S);
+  auto run = [&](auto* kernel) {
+    if (S.lds > 65536)
+      HIPCHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   NS_LDS));
+    kernel<<<I.nblk, 64 * S.waves, S.lds, c.stream>>>(S.info.p, S.tab.p, S.desc.p, V.v->p,
+        reinterpret_cast<const uint2*>(S.cols.p), V.w->p, V.rdg->p, b, x);
+  };
+  const SweepSet& L = LOWER ? I.lo : I.up;
+  const int kt = kt_begin(c, LOWER ? KT_SWEEP_LO : KT_SWEEP_UP,
+                          (double)L.ne * (sizeof(VT) + 4.0) + (LOWER ? 20.0 : 24.0) * I.n);
+  if (S.lgmax == 0) run(k_node_sweep<VT, LOWER, 0>);
+  else if (S.lgmax == 1) run(k_node_sweep<VT, LOWER, 1>);
+  else run(k_node_sweep<VT, LOWER, 2>);
+  kt_end(c, kt);
 }
 
 template <class VT>
@@ -2223,10 +2513,18 @@ static bool apply_t(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t* ev, 
                     const double* aval)
 {
   const int v = sweep_variant();
-  if (v >= 2 && I.bs.on) { launch_blocks<VT>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
-  if (v != 0) { launch_sweeps<VT, 1>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
-  launch_sweeps<VT, 0>(c, I, b, x, ev, nullptr, nullptr);
-  return false;
+  if (I.bs.on && (v >= 2 || !I.lo.packed)) { launch_blocks<VT>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
+  if (I.nlo.on && I.nup.on && (v >= 2 || !I.lo.packed)) {
+    if (ev) HIPCHECK(hipEventRecord(ev[0], c.stream));
+    launch_nodes<VT, true>(c, I, I.nlo, b, I.lo.xp.p);
+    if (ev) HIPCHECK(hipEventRecord(ev[1], c.stream));
+    launch_nodes<VT, false>(c, I, I.nup, I.lo.xp.p, x);
+    if (ev) HIPCHECK(hipEventRecord(ev[2], c.stream));
+    HIPCHECK(hipGetLastError());
+    return false;
+  }
+  launch_sweeps<VT>(c, I, b, x, ev, aidx, aval);
+  return aidx != nullptr;
 }
 
 bool ilu_apply(Ctx& c, Ilu& I, int prec, const double* b, double* x, hipEvent_t* ev,
@@ -2264,20 +2562,33 @@ void setup_ilu_schedule(Ctx& c)
   }
   const std::vector<int>& rp = c.csr_only ? hrp : c.hm.rowptr;
   const std::vector<int>& cl = c.csr_only ? hcols : c.hm.cols;
-  ilu_setup(c.ilu, c.n, rp, cl, 1, nullptr, c.stream, nullptr, 1, 0);
+  std::vector<int> group, unit(c.n);
+  if (!c.csr_only) {
+    group.assign(c.n, -1);
+    for (size_t k = 0; k < c.hm.eqno.size(); k++)
+      if (c.hm.eqno[k] >= 0) group[c.hm.eqno[k]] = (int)(k / 3);
+    unit = group;
+  } else {
+    // rows that follow each other with one set of columns, as the rows of a node have it
+    std::vector<char> mark(c.n, 0);
+    for (int i = 0; i < c.n; i++) {
+      bool same = i > 0 && rp[i + 1] - rp[i] == rp[i] - rp[i - 1];
+      if (same) {
+        for (int q = rp[i - 1]; q < rp[i]; q++) mark[cl[q]] = 1;
+        for (int q = rp[i]; q < rp[i + 1]; q++) same = same && mark[cl[q]];
+        for (int q = rp[i - 1]; q < rp[i]; q++) mark[cl[q]] = 0;
+      }
+      unit[i] = same ? unit[i - 1] : i;
+    }
+  }
+  ilu_setup(c.ilu, c.n, rp, cl, 1, nullptr, unit, c.stream, nullptr, 1, 0);
   // strip ILU: two strips per compute unit (two sweep workgroups fit one CU's LDS), at
   // least a few thousand rows each
   hipDeviceProp_t prop;
   HIPCHECK(hipGetDeviceProperties(&prop, c.device));
   int nblk = c.strips > 0 ? c.strips : 2 * prop.multiProcessorCount;
   nblk = std::max(1, std::min(nblk, c.n / 2048));
-  std::vector<int> group;
-  if (!c.csr_only) {
-    group.assign(c.n, -1);
-    for (size_t k = 0; k < c.hm.eqno.size(); k++)
-      if (c.hm.eqno[k] >= 0) group[c.hm.eqno[k]] = (int)(k / 3);
-  }
-  ilu_setup(c.silu, c.n, rp, cl, nblk, c.csr_only ? nullptr : &group, c.stream,
+  ilu_setup(c.silu, c.n, rp, cl, nblk, c.csr_only ? nullptr : &group, unit, c.stream,
             c.csr_only ? nullptr : &c.hm, strip_segments(c, nblk), STAGE_ROWS);
   c.coarse.ready = c.coarse.fac = false;
   const int cseg = coarse_segments_of(c);

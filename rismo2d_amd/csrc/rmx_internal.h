@@ -126,8 +126,10 @@ struct Params {
 
 constexpr int RING = 8192;     // LDS ring of solved x values in the packed sweeps
 
-// Packed layout of one triangular sweep over all strips of an ILU system.
+// Packed layout of one triangular sweep by levels over all strips of an ILU system (its
+// counts alone unless `packed`).
 struct SweepSet {
+  bool packed = false;
   int nblk = 0, nlev_max = 0, nlev_sum = 0, max_nr = 0;
   long long ne = 0;
   DBuf<int> blev, bpos;         // per strip: first level, first position
@@ -157,11 +159,26 @@ struct BlockSweep {
   DBuf<uint2> desc;                // slot descriptors (lower, upper of every block)
   DBuf<unsigned short> clo, cup;   // columns: LDS byte offset (0: the zero slot)
   DBuf<int> slo, sup;              // CSR position of every value (-1: zero)
-  DBuf<int> sulo, suup, sdg;       // per unit: CSR positions of its lower / upper couplings
-                                   // and of its diagonals (4 each; -1: none)
+  DBuf<int> sulo, suup, sdg;       // per unit, 4 rows: CSR positions of a row's two lower /
+                                   // upper couplings and of its diagonal (-1: none)
   DBuf<float> vlo32, vup32, wlo32, wup32;       // packed values (entries, unit couplings)
   DBuf<double> vlo64, vup64, wlo64, wup64;
   DBuf<double> rdg32, rdg64;       // reciprocal diagonals of the FP32 / FP64 factors
+};
+
+// Node sweep of one triangle (k_node_sweep): one workgroup per strip of any size, a pass per
+// level of nodes.
+struct NodeSweep {
+  bool on = false;
+  int waves = 1, lgmax = 0;        // waves per workgroup; log2 of the most slots of a node (<= 2)
+  size_t lds = 0;                  // dynamic LDS bytes (a double per live row)
+  DBuf<int4> info;                 // per strip {passes, pass table, descriptors}
+  DBuf<unsigned> tab;
+  DBuf<uint4> desc;
+  DBuf<unsigned short> cols;       // LDS places of the columns, 4 per group
+  DBuf<int> src, wsrc;             // CSR positions of the values, of every row's two couplings
+  DBuf<float> v32, w32;            // packed values of the FP32 / FP64 factors
+  DBuf<double> v64, w64, rdg32, rdg64;
 };
 
 // One ILU(0) system: pattern, factorisation schedule, sweeps and factors.
@@ -179,6 +196,7 @@ struct Ilu {
   DBuf<unsigned short> plan;    // per plan entry: pivot index | target position << 8
   SweepSet lo, up;
   BlockSweep bs;
+  NodeSweep nlo, nup;
   DBuf<double> LU64, plo64, pup64, pdg64;
   DBuf<float> LU32, plo32, pup32, pdg32;
   bool fac64 = false, fac32 = false;

@@ -87,3 +87,43 @@ def test_blocks_that_share_a_wave(ctx, strips, segments):
         y = ctx.silu0_apply(B, prec)
         assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
     ctx.set_strips(0, 0)
+
+
+# systems past one block (2,047 rows): chains and wide levels, one to four waves, entries per
+# row and triangle at the edges of a slot (16) and of 2 and 4 slots; rows in units of 3 (one
+# set of columns) and alone; the last keeps 21,000 rows alive, more than LDS holds (the staged
+# level sweeps)
+@pytest.mark.parametrize("n,width,stride,run", [(2048, 1, 1, 1), (2050, 3, 700, 1), (2500, 16, 1, 1),
+                                                (3001, 17, 37, 1), (2100, 33, 2, 1), (6000, 4, 500, 3),
+                                                (2049, 0, 1, 1), (9000, 2, 2000, 3),
+                                                (45000, 2, 21000, 1)])
+def test_single_strip_node_sweeps(ctx, n, width, stride, run):
+    print(f"[gpu] one strip, {n} rows in runs of {run}, {width} entries a side", flush=True)
+    rp, cols, vals = _band_csr(n // run, [1 + stride * k for k in range(width)], 21)
+    if run > 1:                              # every row and column `run` times
+        m, rng = n // run, np.random.default_rng(22)
+        rp0, c0, rp, cols, vals = rp, cols, [0], [], []
+        for i in range(m):
+            js = (run * c0[rp0[i]:rp0[i + 1], None] + np.arange(run)).ravel()
+            for r in range(run * i, run * i + run):
+                o = rng.permutation(js[js != r])
+                v = rng.standard_normal(len(o))
+                cols += [r] + o.tolist()
+                vals += [np.abs(v).sum() + 1.0] + v.tolist()
+                rp.append(len(cols))
+        rp, cols, vals = np.asarray(rp, np.int32), np.asarray(cols, np.int32), np.asarray(vals)
+    n = len(rp) - 1
+    b = np.random.default_rng(12).standard_normal(n)
+    ctx.csr_upload(rp, cols, vals, b)
+    for prec, dt in ((rmx.F64, np.float64), (rmx.F32, np.float32)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        ctx.ilu0_factor(prec)
+        L, r = po.ilu0_factor(rp, cols, vals.astype(dt))
+        assert r == 0
+        ref = po.ilu0_solve(rp, cols, L, b)
+        ctx.kernel_stats(True)
+        y = ctx.ilu0_apply(b, prec)
+        ran = ctx.kernel_stats(False)
+        assert ran["sweep_lower"][2] == 1 and ran["sweep_upper"][2] == 1
+        assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
