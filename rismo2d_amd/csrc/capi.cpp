@@ -708,6 +708,7 @@ rmx_status rmx_precond_apply(rmx_ctx* p, int kind, int prec, const double* b, do
   dev_precond(c, pr, kind, c.w[0].p, c.w[1].p);
   c.w[1].download(x, c.n, c.stream);
   HIPCHECK(hipStreamSynchronize(c.stream));
+  coarse_check(c);
   API_END
 }
 

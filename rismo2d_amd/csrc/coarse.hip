@@ -12,9 +12,11 @@
 // instead of a second SpMV.  R A P is summed on
 // the device in a fixed order (every coarse entry is the sum of the matrix entries whose row
 // and column aggregates match, listed by a permutation built once per pattern).  Aggregates
-// are numbered strip by strip, so R A P is banded; its LU factorisation with partial
-// pivoting (the layout and steps of LAPACK's band LU, gbtf2 / gbtrs) and the per-apply
-// solve of a few thousand unknowns run on the host between two small copies.
+// are numbered strip by strip, so R A P is block tridiagonal in runs of strips: it is factored
+// by block cyclic reduction on the device and solved by one launch per application.  Where a
+// run's aggregates are too many for a block, or a reduced block is singular, R A P is factored
+// as a band with partial pivoting (the layout and steps of LAPACK's band LU, gbtf2 / gbtrs)
+// and solved on the host between two small copies.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -160,89 +162,160 @@ static void band_solve(int n, int kl, int ku, std::vector<double>& ab, const std
 //   apply, back-substitution: w_j <- A_j^-1 (w_j - B_j w_{j-s} - C_j w_{j+s}).
 // After the last level block 0 alone remains: w_0 <- A_0^-1 w_0.  Matrices are stored
 // column-major (entry (r, c) at c * bs + r), so row r of a matrix-vector product reads
-// consecutive entries across the lanes of a wave.
-
-// w[i * bs + r] <- rc[blk_start[i] + r] (0 on padding)
-__global__ void k_cr_in(int nb, int bs, const int* __restrict__ blk_start,
-                        const double* __restrict__ rc, double* __restrict__ w)
-{
-  const int i = blockIdx.x, r = threadIdx.x;
-  if (i >= nb || r >= bs) return;
-  const int a = blk_start[i], m = blk_start[i + 1] - a;
-  w[(long long)i * bs + r] = r < m ? rc[a + r] : 0.0;
-}
-
-__global__ void k_cr_out(int nb, int bs, const int* __restrict__ blk_start,
-                         const double* __restrict__ w, double* __restrict__ zc)
-{
-  const int i = blockIdx.x, r = threadIdx.x;
-  if (i >= nb || r >= bs) return;
-  const int a = blk_start[i], m = blk_start[i + 1] - a;
-  if (r < m) zc[a + r] = w[(long long)i * bs + r];
-}
+// consecutive entries across the lanes of a wave.  The whole apply is one launch (k_cr_solve).
 
 constexpr int CR_MAX = 128;       // rows of a coarse block (a strip's aggregates)
+constexpr int CR_THREADS = 512;   // threads per task of the solve
+constexpr int CR_PRE = 16;        // matrix entries per thread loaded before a wait
 
-// one workgroup (a thread per block row) per kept block k (i = 2 s k) of level s:
-// w_i -= P_i w_{i-s} + Q_i w_{i+s}
-__global__ void __launch_bounds__(CR_MAX) k_cr_fwd(int nb, int bs, int s,
-                                                   const double* __restrict__ M,
-                                                   double* __restrict__ w)
+// The solve in one launch: a workgroup per task, tasks in an order in which each needs only
+// earlier ones (`order`: blocks by elimination level, block 0 last).  Task t < nb reduces
+// block i = order[t]: its levels' updates with the eliminated neighbours' final values, then
+// (block 0) the top block's solution; task nb + u substitutes back into the u-th block from
+// the end of the order.  A workgroup takes its task's number from a counter when it starts, so
+// the tasks it waits for have been started before and every wait ends, in whatever order
+// and number workgroups run; the counter's value also numbers the launch.  A finished block's
+// values are exchanged as two 64-bit words each, half of the value with the launch's number,
+// by agent-scope (sc1) accesses: a reader has a value when both its words carry the number,
+// so there is no flag to write after the values, to poll before them or to clear.
+// Thread (g, r) holds row r's entries of every G-th column, the first CR_PRE of each matrix
+// in registers before it waits; the column groups' shares are summed in LDS in fixed order.
+// Bound: the chain of 2 log2(nb) exchanges, about 3.5 us each.  Against a launch per level (and
+// a copy in and out): 17 blocks of 24 44 -> 34 us, 512 blocks of 42 160 -> 69 us; 51 blocks of
+// 48 41 us and 225 blocks of 48, the coarse systems of 80 x 320 and 320 x 320-cell meanders,
+// whose strips couple two apart, where the host's band LU with its two copies took about 0.2
+// and 0.9 ms.
+__global__ void __launch_bounds__(CR_THREADS) k_cr_solve(int nb, int bs, int levels,
+                                                         const int* __restrict__ order,
+                                                         const int* __restrict__ blk_start,
+                                                         const long long* __restrict__ off_elim,
+                                                         const long long* __restrict__ off_keep,
+                                                         long long off_top,
+                                                         const double* __restrict__ mats,
+                                                         const double* __restrict__ rc,
+                                                         double* __restrict__ zc,
+                                                         unsigned long long* state,
+                                                         unsigned long long* words, int spin_limit)
 {
-  __shared__ double lo[CR_MAX], hi[CR_MAX];
-  const int k = blockIdx.x, r = threadIdx.x;
-  const int i = 2 * s * k;
-  if (i >= nb) return;
-  const bool hl = i - s >= 0, hh = i + s < nb;
-  if (r < bs) {
-    lo[r] = hl ? w[(long long)(i - s) * bs + r] : 0.0;
-    hi[r] = hh ? w[(long long)(i + s) * bs + r] : 0.0;
+  __shared__ double v0[CR_MAX], v1[CR_MAX], own[CR_MAX], red[CR_THREADS];
+  __shared__ unsigned long long s_ticket;
+  __shared__ int s_ok;
+  const int t = threadIdx.x;
+  const int rp = (bs + 31) & ~31;                // threads per column group
+  const int G = CR_THREADS / rp, g = t / rp, r = t - g * rp;
+  const bool on = g < G && r < bs;
+  const long long b2 = (long long)bs * bs;
+  const unsigned long long total = 2ull * nb - 1;
+  if (t == 0) {
+    s_ticket = __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_ok = 1;
   }
   __syncthreads();
-  if (r >= bs) return;
-  const long long b2 = (long long)bs * bs;
-  const double* P = M + 2 * b2 * k;
-  const double* Q = P + b2;
-  double acc = 0.0;
-  for (int c = 0; c < bs; c++) acc += P[c * bs + r] * lo[c] + Q[c * bs + r] * hi[c];
-  w[(long long)i * bs + r] -= acc;
-}
-
-// one workgroup per eliminated block k (j = s + 2 s k):
-// w_j <- A_j^-1 (w_j - B_j w_{j-s} - C_j w_{j+s}); with s = 0 the top block, w_0 <- A^-1 w_0
-__global__ void __launch_bounds__(CR_MAX) k_cr_bwd(int nb, int bs, int s,
-                                                   const double* __restrict__ M,
-                                                   double* __restrict__ w)
-{
-  __shared__ double lo[CR_MAX], hi[CR_MAX], t[CR_MAX];
-  const int k = blockIdx.x, r = threadIdx.x;
-  const int j = s + 2 * s * k;
-  if (j >= nb) return;
-  const long long b2 = (long long)bs * bs;
-  const double* Ai = M + (s ? 3 * b2 * k : 0);
-  double v = 0.0;
-  if (s) {
-    const bool hl = j - s >= 0, hh = j + s < nb;
-    if (r < bs) {
-      lo[r] = hl ? w[(long long)(j - s) * bs + r] : 0.0;
-      hi[r] = hh ? w[(long long)(j + s) * bs + r] : 0.0;
+  const unsigned long long tag = (s_ticket / total + 1) << 32;
+  const int task = (int)(s_ticket % total);
+  const bool fwd = task < nb;
+  const int i = fwd ? order[task] : order[2 * nb - 2 - task];
+  const int e = i ? __builtin_ctz((unsigned)i) : levels;      // level it is eliminated at
+  const int m = blk_start[i + 1] - blk_start[i];
+  // list f (0 reduced, 1 solved) values of blocks lo and hi (below 0 or from nb on: absent, zero)
+  // into v0 and v1; false (the same in every thread) past the spin limit or after another's
+  auto gather = [&](int f, int lo, double* dlo, int hi, double* dhi) {
+    const int q = t & (CR_MAX - 1), k = t < CR_MAX ? lo : hi;
+    double* dst = t < CR_MAX ? dlo : dhi;
+    if (t < 2 * CR_MAX && q < bs && dst) {
+      double v = 0.0;
+      if (k >= 0 && k < nb) {
+        const unsigned long long* p = words + 2 * (((long long)f * nb + k) * bs + q);
+        unsigned long long a = 0, b = 0;
+        for (int polls = 0;;) {
+          a = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          b = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if ((a & ~0xffffffffull) == tag && (b & ~0xffffffffull) == tag) break;
+          if (++polls > spin_limit ||
+              ((polls & 255) == 0 && __hip_atomic_load(state + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+            __hip_atomic_store(state + 1, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_ok = 0;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        v = __hiloint2double((int)(unsigned)a, (int)(unsigned)b);
+      }
+      dst[q] = v;
     }
     __syncthreads();
-    if (r < bs) {
-      const double* B = Ai + b2;
-      const double* C = B + b2;
-      v = w[(long long)j * bs + r];
-      for (int c = 0; c < bs; c++) v -= B[c * bs + r] * lo[c] + C[c * bs + r] * hi[c];
+    return s_ok != 0;
+  };
+  // entries of a column-major matrix that this thread holds: columns g, g + G, ...
+  auto load = [&](const double* M, double* pre) {
+#pragma unroll
+    for (int k = 0; k < CR_PRE; k++) {
+      const int c = g + k * G;
+      pre[k] = on && c < bs ? M[(long long)c * bs + r] : 0.0;
     }
-  } else if (r < bs) {
-    v = w[(long long)j * bs + r];
+  };
+  auto dot = [&](const double* M, const double* pre, const double* v) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < CR_PRE; k++) {
+      const int c = g + k * G;
+      if (c < bs) s += pre[k] * v[c];
+    }
+    if (on)
+      for (int c = g + CR_PRE * G; c < bs; c += G) s += M[(long long)c * bs + r] * v[c];
+    return s;
+  };
+  auto total_of = [&](double s) {                // row r's sum over the groups, in group 0
+    if (on) red[g * rp + r] = s;
+    __syncthreads();
+    double a = 0.0;
+    if (g == 0 && r < bs)
+      for (int k = 0; k < G; k++) a += red[k * rp + r];
+    __syncthreads();
+    return a;
+  };
+  auto publish = [&](int f) {                    // own[] as block i's values
+    if (t < bs) {
+      unsigned long long* p = words + 2 * (((long long)f * nb + i) * bs + t);
+      const double v = own[t];
+      __hip_atomic_store(p, tag | (unsigned)__double2hiint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(p + 1, tag | (unsigned)__double2loint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  };
+  double pa[CR_PRE], pb[CR_PRE], pc[CR_PRE];
+  if (fwd) {
+    if (t < bs) own[t] = t < m ? rc[blk_start[i] + t] : 0.0;
+    for (int l = 0; l < e; l++) {
+      const int s = 1 << l;
+      const double* P = mats + off_keep[l] + 2 * b2 * (i >> (l + 1));
+      load(P, pa);
+      load(P + b2, pb);
+      if (!gather(0, i - s, v0, i + s, v1)) return;
+      const double a = total_of(dot(P, pa, v0) + dot(P + b2, pb, v1));
+      if (t < bs) own[t] -= a;
+    }
+    if (i != 0) { publish(0); return; }
+    const double* A = mats + off_top;
+    load(A, pa);
+    __syncthreads();
+    const double a = total_of(dot(A, pa, own));
+    if (t < bs) own[t] = a;
+  } else {
+    const int s = 1 << e;
+    const double* A = mats + off_elim[e] + 3 * b2 * (i >> (e + 1));
+    load(A + b2, pb);
+    load(A + 2 * b2, pc);
+    load(A, pa);
+    if (!gather(0, i, own, -1, nullptr)) return;
+    if (!gather(1, i - s, v0, i + s, v1)) return;
+    const double a = total_of(dot(A + b2, pb, v0) + dot(A + 2 * b2, pc, v1));
+    if (t < bs) own[t] -= a;
+    __syncthreads();
+    const double y = total_of(dot(A, pa, own));
+    if (t < bs) own[t] = y;
   }
-  if (r < bs) t[r] = v;
-  __syncthreads();
-  if (r >= bs) return;
-  double x = 0.0;
-  for (int c = 0; c < bs; c++) x += Ai[c * bs + r] * t[c];
-  w[(long long)j * bs + r] = x;
+  if (t < m) zc[blk_start[i] + t] = own[t];
+  publish(1);
 }
 
 // ---- factorisation of the reduction on the device (column-major bs x bs blocks) ----
@@ -458,19 +531,24 @@ static void dense_mm(int n, const double* a, const double* b, double alpha, bool
   }
 }
 
-// Block structure of the coarse matrix: usable when every slot couples aggregates of one
-// strip or of neighbouring strips and no strip holds more than CR_MAX aggregates.
-static void cr_setup(Coarse& C, const std::vector<int>& agg_strip, int nstrips)
+// Block structure of the coarse matrix: a block is the aggregates of as many neighbouring
+// strips as apart a slot couples (two where a strip holds less than the rows of a column of
+// cells), so that every slot couples one block or neighbouring ones; usable when no block
+// holds more than CR_MAX aggregates.
+static void cr_setup(Coarse& C, std::vector<int> agg_strip, int nstrips)
 {
   C.cr_ok = C.cr_fac = false;
   if (getenv("RMX_COARSE_HOST")) return;
+  int reach = 1;
+  for (long long k = 0; k < C.nslot; k++)
+    reach = std::max(reach, std::abs(agg_strip[C.slot_row[k]] - agg_strip[C.slot_col[k]]));
+  for (int& v : agg_strip) v /= reach;
+  nstrips = (nstrips + reach - 1) / reach;
   std::vector<int> cnt(nstrips, 0);
   for (int v : agg_strip) cnt[v]++;
   int bs = 0;
   for (int v : cnt) bs = std::max(bs, v);
   if (bs < 1 || bs > CR_MAX) return;
-  for (long long k = 0; k < C.nslot; k++)
-    if (std::abs(agg_strip[C.slot_row[k]] - agg_strip[C.slot_col[k]]) > 1) return;
   const int nb = nstrips;
   C.nb = nb; C.bs = bs;
   C.blk_start.assign(nb + 1, 0);
@@ -501,8 +579,18 @@ static void cr_setup(Coarse& C, const std::vector<int>& agg_strip, int nstrips)
   C.mats_n = off;
   C.h_mats.assign(off, 0.0);
   C.mats.alloc(off);
-  C.w.alloc((size_t)nb * bs);
   C.d_blk_start.upload(C.blk_start, nullptr);
+  // blocks by elimination level (the number of times 2 divides them), block 0 last
+  std::vector<int> order;
+  for (int l = 0; l < levels; l++)
+    for (int i = 1 << l; i < nb; i += 2 << l) order.push_back(i);
+  order.push_back(0);
+  C.d_order.upload(order, nullptr);
+  std::vector<long long> offs(C.lev_elim);
+  offs.insert(offs.end(), C.lev_keep.begin(), C.lev_keep.end());
+  offs.push_back(0);
+  C.d_off.upload(offs, nullptr);
+  C.d_state.release();
   C.d_slot_dst.upload(C.slot_dst, nullptr);
   HIPCHECK(hipDeviceSynchronize());
   C.cr_ok = true;
@@ -615,23 +703,28 @@ static bool cr_factor_device(Ctx& c, Coarse& C)
 
 static void cr_apply(Ctx& c, Coarse& C)
 {
-  const int nb = C.nb, bs = C.bs;
-  const int nt = (bs + 63) / 64 * 64;           // a thread per block row, whole waves
-  hipStream_t st = c.stream;
-  k_cr_in<<<nb, nt, 0, st>>>(nb, bs, C.d_blk_start.p, C.rc.p, C.w.p);
-  int lev = 0;
-  for (int s = 1; s < nb; s *= 2, lev++) {
-    const int nk = (nb + 2 * s - 1) / (2 * s);
-    k_cr_fwd<<<nk, nt, 0, st>>>(nb, bs, s, C.mats.p + C.lev_keep[lev], C.w.p);
-  }
-  k_cr_bwd<<<1, nt, 0, st>>>(nb, bs, 0, C.mats.p + C.top_off, C.w.p);
-  for (int l = C.levels - 1; l >= 0; l--) {
-    const int s = 1 << l;
-    const int ne = (nb - s + 2 * s - 1) / (2 * s);
-    k_cr_bwd<<<ne, nt, 0, st>>>(nb, bs, s, C.mats.p + C.lev_elim[l], C.w.p);
-  }
-  k_cr_out<<<nb, nt, 0, st>>>(nb, bs, C.d_blk_start.p, C.w.p, C.zc.p);
+  int spin = 1 << 22;
+  if (const char* e = getenv("RMX_COARSE_SPIN")) spin = std::max(1, atoi(e));
+  k_cr_solve<<<2 * C.nb - 1, CR_THREADS, 0, c.stream>>>(C.nb, C.bs, C.levels, C.d_order.p,
+      C.d_blk_start.p, C.d_off.p, C.d_off.p + C.levels, C.top_off, C.mats.p, C.rc.p, C.zc.p,
+      C.d_state.p, C.d_state.p + 2, spin);
   HIPCHECK(hipGetLastError());
+}
+
+// Whether a coarse solve gave up a wait (the stream must have synchronised).
+void coarse_check(Ctx& c)
+{
+  Coarse& C = c.coarse;
+  if (!C.fac || !C.cr_fac || !C.applied) return;
+  C.applied = false;
+  unsigned long long st[2] = { 0, 0 };
+  HIPCHECK(hipMemcpyAsync(st, C.d_state.p, sizeof(st), hipMemcpyDeviceToHost, c.stream));
+  HIPCHECK(hipStreamSynchronize(c.stream));
+  if (st[1]) {
+    C.d_state.release();                         // words and numbers start again
+    C.fac = false;
+    fail(RMX_ERR_HIP, "coarse space: a block's wait for its neighbours exceeded its bound");
+  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -795,6 +888,10 @@ void coarse_factor(Ctx& c, int prec)
   HIPCHECK(hipGetLastError());
   C.fac = false;
   C.cr_fac = false;
+  if (C.cr_ok && !C.d_state.p) {                 // task counter, abort flag, exchanged words
+    C.d_state.alloc(2 + 4 * (size_t)C.nb * C.bs);
+    HIPCHECK(hipMemsetAsync(C.d_state.p, 0, sizeof(unsigned long long) * C.d_state.n, c.stream));
+  }
   // the block cyclic reduction factored on the device (RMX_COARSE_HOST_FACTOR: on the host)
   if (C.cr_ok && !getenv("RMX_COARSE_HOST_FACTOR") && cr_factor_device(c, C)) {
     C.cr_fac = true;
@@ -837,6 +934,7 @@ void coarse_apply(Ctx& c, int prec, const double* r, double* z)
   k_restrict<<<(C.nc * 64 + 255) / 256, 256, 0, c.stream>>>(C.nc, C.agg_ptr.p, C.agg_rows.p, r, C.rc.p);
   if (C.cr_fac) {
     cr_apply(c, C);
+    C.applied = true;
   } else {
     HIPCHECK(hipMemcpyAsync(C.h_buf, C.rc.p, sizeof(double) * C.nc, hipMemcpyDeviceToHost, c.stream));
     HIPCHECK(hipStreamSynchronize(c.stream));

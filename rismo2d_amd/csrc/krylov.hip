@@ -685,6 +685,7 @@ void dev_solve(Ctx& c, const rmx_krylov_opts& o0, rmx_krylov_out& out)
   out.solvers = solvers;
   HIPCHECK(hipStreamSynchronize(c.stream));
   kt_collect(c);
+  coarse_check(c);
   out.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
 

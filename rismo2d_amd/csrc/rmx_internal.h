@@ -245,10 +245,9 @@ struct Coarse {
   std::vector<double> band;                   // LU factors, band storage (LAPACK layout)
   std::vector<int> ipiv;
   double* h_buf = nullptr;                    // pinned, max(nc, nslot) doubles
-  // Block cyclic reduction of R A P on the device, when it is block tridiagonal in strips
-  // (every coarse entry couples aggregates of one strip or of neighbouring strips): block
-  // i = the aggregates of strip i, padded to bs; factored on the host per factorisation,
-  // applied by level kernels.  Off (or a singular reduced block): the host band LU.
+  // Block cyclic reduction of R A P on the device, block tridiagonal in runs of strips: block
+  // i = the aggregates of one run, padded to bs; applied by one launch.  Off (blocks too
+  // large), or a singular reduced block: the host band LU.
   bool cr_ok = false, cr_fac = false;
   int nb = 0, bs = 0, levels = 0;
   std::vector<int> blk_start;                 // [nb + 1] first aggregate of every block
@@ -256,7 +255,11 @@ struct Coarse {
   std::vector<long long> lev_elim, lev_keep;  // per level: offset of its matrices in mats
   long long top_off = 0, mats_n = 0;
   std::vector<double> h_mats;
-  DBuf<double> mats, w;                       // factor matrices; padded work vector
+  DBuf<double> mats;                          // factor matrices
+  DBuf<int> d_order;                          // blocks in elimination order
+  DBuf<long long> d_off;                      // lev_elim, lev_keep
+  DBuf<unsigned long long> d_state;           // task counter, abort flag, exchanged words
+  bool applied = false;                       // applied since the abort flag was read
   DBuf<int> d_blk_start;
   DBuf<long long> d_slot_dst;
   DBuf<double> d_blocks, d_inv, d_tmp;        // device factorisation: B, A, C blocks; inverses
@@ -441,6 +444,7 @@ void coarse_setup(Ctx& c, const std::vector<int>& rp, const std::vector<int>& cl
 int coarse_segments_of(const Ctx& c);          // coarse segments per strip in effect
 void coarse_factor(Ctx& c, int prec);
 void coarse_apply(Ctx& c, int prec, const double* r, double* z);   // device pointers
+void coarse_check(Ctx& c);                     // fails if a coarse solve gave up a wait
 void dev_precond(Ctx& c, int prec, int kind, const double* in, double* out);
 void spmv_setup(Ctx& c, const int* rowptr, const int* cols);   // host pattern
 double spmv_f32_bytes(const Ctx& c);          // algorithmic bytes of one FP32 SpMV

@@ -127,3 +127,53 @@ def test_single_strip_node_sweeps(ctx, n, width, stride, run):
         ran = ctx.kernel_stats(False)
         assert ran["sweep_lower"][2] == 1 and ran["sweep_upper"][2] == 1
         assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
+
+
+def _two_level_reference(ctx, prec, dt, r):
+    """z = z1 + M^-1 (r - A z1), z1 = P (R A P)^-1 R r, in numpy with the oracle's ILU(0)."""
+    import scipy.sparse as sp
+    n = ctx.n
+    rp, cols = ctx.pattern()
+    A, _ = ctx.matrix(rmx.F64)
+    agg, nc = ctx.aggregates()
+    block = ctx.blocks()
+    P = sp.csr_matrix((np.ones(n), (np.arange(n), agg)), shape=(n, nc))
+    Ap = A.astype(dt)
+    M = sp.csr_matrix((Ap.astype(np.float64), cols, rp), shape=(n, n))
+    z1 = P @ np.linalg.solve((P.T @ M @ P).toarray(), P.T @ r)
+    rows = np.repeat(np.arange(n), np.diff(rp))
+    keep = block[rows] == block[cols]
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=n))])
+    L, _ = po.ilu0_factor(rp, cols, Ap)
+    return z1 + po.ilu0_solve(rp2.astype(np.int32), cols[keep], L[keep], r - M @ z1)
+
+
+# strips of less than a column of cells (the coarse matrix couples strips two apart), with few
+# and many coarse unknowns a strip; one strip; a number of blocks that is no power of two.
+# The same 1e-9 as the two-level test on the channel.
+@pytest.mark.parametrize("nx,ny,strips,cseg", [(14, 250, 0, 2), (14, 250, 0, 20), (6, 60, 0, 5),
+                                               (14, 250, 3, 8), (30, 130, 0, 6)])
+def test_two_level_on_thin_strips(ctx, nx, ny, strips, cseg):
+    from rismo2d_amd import deck as dk
+    d = dk.meander(nx, ny, reach=3.125 * nx)
+    ctx.set_coarse(cseg)
+    ctx.set_strips(strips, 0)
+    ctx.upload_mesh(d)
+    ctx.time_step(30.0, 0.7, first=True)
+    n = ctx.prepare()
+    print(f"[gpu] two-level apply on a {nx} x {ny} meander, {n} equations, "
+          f"{ctx.aggregates()[1]} coarse unknowns", flush=True)
+    ctx.assemble(rmx.F64)
+    ctx.scale_l2()
+    r = np.random.default_rng(3).standard_normal(n)
+    for prec, dt in ((rmx.F64, np.float64), (rmx.F32, np.float32)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        ctx.silu0_factor(prec)
+        ctx.coarse_factor(prec)
+        ref = _two_level_reference(ctx, prec, dt, r)
+        for _ in range(3):                   # the second and third apply meet used words
+            y = ctx.precond_apply(rmx.PREC_SILU0C, r, prec)
+            assert np.abs(y - ref).max() <= 1e-9 * np.abs(ref).max(), prec
+    ctx.set_coarse(-1)
+    ctx.set_strips(0, 0)
