@@ -162,7 +162,8 @@ static void band_solve(int n, int kl, int ku, std::vector<double>& ab, const std
 //   apply, back-substitution: w_j <- A_j^-1 (w_j - B_j w_{j-s} - C_j w_{j+s}).
 // After the last level block 0 alone remains: w_0 <- A_0^-1 w_0.  Matrices are stored
 // column-major (entry (r, c) at c * bs + r), so row r of a matrix-vector product reads
-// consecutive entries across the lanes of a wave.  The whole apply is one launch (k_cr_solve).
+// consecutive entries across the lanes of a wave.  The whole apply is one launch (k_cr_solve), or
+// for a small system one product with the inverse (k_cr_dense).
 
 constexpr int CR_MAX = 128;       // rows of a coarse block (a strip's aggregates)
 constexpr int CR_THREADS = 512;   // threads per task of the solve
@@ -316,6 +317,109 @@ __global__ void __launch_bounds__(CR_THREADS) k_cr_solve(int nb, int bs, int lev
   }
   if (t < m) zc[blk_start[i] + t] = own[t];
   publish(1);
+}
+
+// ---- inverse of a small coarse matrix from its reduction ----
+//
+// Up to CR_DENSE rows (with the blocks' padding) the apply is one product with the inverse, a
+// read of 8 nc^2 bytes spread over the chip, in place of the chain of exchanges: the unit
+// vectors are taken through the reduction's steps together, W row-major (row i * bs + r: block
+// i's row r; column J: the unit vector of aggregate J), and W is the inverse.
+
+constexpr int CR_DENSE = 3072;
+constexpr int CR_TILE = 64;       // columns of W per workgroup
+
+__global__ void k_cr_units(long long count, int ld, int nc, const int* __restrict__ prow,
+                           double* __restrict__ W)
+{
+  for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < count;
+       k += (long long)gridDim.x * blockDim.x) {
+    const int row = (int)(k / ld), J = (int)(k % ld);
+    W[k] = J < nc && prow[J] == row ? 1.0 : 0.0;
+  }
+}
+
+// acc[a] += sum over k of M[k * bs + r0 + a] * X[k * ld]: RA rows of a column-major block times
+// one column of W's rows (M's entries are the same in a wave)
+template <int RA>
+__device__ __forceinline__ void rows_mac(int bs, int r0, const double* __restrict__ M,
+                                         const double* __restrict__ X, int ld, double* acc)
+{
+  for (int k = 0; k < bs; k++) {
+    const double x = X[(long long)k * ld];
+#pragma unroll
+    for (int a = 0; a < RA; a++) acc[a] += M[k * bs + min(r0 + a, bs - 1)] * x;
+  }
+}
+
+// kept blocks of level s (i = 2 s k): W_i -= P W_{i-s} + Q W_{i+s}; four waves of RA rows each
+template <int RA>
+__global__ void __launch_bounds__(256) k_cr_unit_fwd(int nb, int bs, int s,
+                                                     const double* __restrict__ M, double* W, int ld)
+{
+  const int i = 2 * s * blockIdx.x;
+  const int c = blockIdx.y * CR_TILE + (threadIdx.x & 63);
+  const int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * RA;
+  if (i >= nb || r0 >= bs) return;
+  const long long b2 = (long long)bs * bs;
+  const double* P = M + 2 * b2 * blockIdx.x;
+  double acc[RA];
+#pragma unroll
+  for (int a = 0; a < RA; a++) acc[a] = 0.0;
+  if (i - s >= 0) rows_mac<RA>(bs, r0, P, W + (long long)(i - s) * bs * ld + c, ld, acc);
+  if (i + s < nb) rows_mac<RA>(bs, r0, P + b2, W + (long long)(i + s) * bs * ld + c, ld, acc);
+#pragma unroll
+  for (int a = 0; a < RA; a++)
+    if (r0 + a < bs) W[((long long)i * bs + r0 + a) * ld + c] -= acc[a];
+}
+
+// eliminated blocks of level s (j = s + 2 s k; s = 0: block 0): W_j <- A_j^-1 (W_j - B_j W_{j-s}
+// - C_j W_{j+s})
+template <int RA>
+__global__ void __launch_bounds__(256) k_cr_unit_bwd(int nb, int bs, int s,
+                                                     const double* __restrict__ M, double* W, int ld)
+{
+  extern __shared__ double tile[];               // [bs][CR_TILE]
+  const int j = s + 2 * s * blockIdx.x;
+  const int l = threadIdx.x & 63, c = blockIdx.y * CR_TILE + l;
+  const int r0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * RA;
+  if (j >= nb) return;
+  const long long b2 = (long long)bs * bs;
+  const double* A = M + (s ? 3 * b2 * blockIdx.x : 0);
+  double acc[RA];
+#pragma unroll
+  for (int a = 0; a < RA; a++) acc[a] = 0.0;
+  if (r0 < bs && s) {
+    if (j - s >= 0) rows_mac<RA>(bs, r0, A + b2, W + (long long)(j - s) * bs * ld + c, ld, acc);
+    if (j + s < nb) rows_mac<RA>(bs, r0, A + 2 * b2, W + (long long)(j + s) * bs * ld + c, ld, acc);
+  }
+#pragma unroll
+  for (int a = 0; a < RA; a++)
+    if (r0 + a < bs) tile[(r0 + a) * CR_TILE + l] = W[((long long)j * bs + r0 + a) * ld + c] - acc[a];
+  __syncthreads();
+  if (r0 >= bs) return;
+#pragma unroll
+  for (int a = 0; a < RA; a++) acc[a] = 0.0;
+  rows_mac<RA>(bs, r0, A, tile + l, CR_TILE, acc);
+#pragma unroll
+  for (int a = 0; a < RA; a++)
+    if (r0 + a < bs) W[((long long)j * bs + r0 + a) * ld + c] = acc[a];
+}
+
+// zc = W rc: a wave per aggregate, its row of W (ld a multiple of 64, zero past nc)
+__global__ void __launch_bounds__(256) k_cr_dense(int nc, int ld, const int* __restrict__ prow,
+                                                  const double* __restrict__ W,
+                                                  const double* __restrict__ rc,
+                                                  double* __restrict__ zc)
+{
+  const int I = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+  if (I >= nc) return;
+  const double* row = W + (long long)prow[I] * ld;
+  double s = 0.0;
+#pragma unroll 8
+  for (int k = lane; k < ld; k += 64) s += row[k] * (k < nc ? rc[k] : 0.0);
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) zc[I] = s;
 }
 
 // ---- factorisation of the reduction on the device (column-major bs x bs blocks) ----
@@ -590,6 +694,13 @@ static void cr_setup(Coarse& C, std::vector<int> agg_strip, int nstrips)
   offs.insert(offs.end(), C.lev_keep.begin(), C.lev_keep.end());
   offs.push_back(0);
   C.d_off.upload(offs, nullptr);
+  std::vector<int> prow(C.nc);
+  for (int i = 0; i < nb; i++)
+    for (int I = C.blk_start[i]; I < C.blk_start[i + 1]; I++) prow[I] = i * bs + (I - C.blk_start[i]);
+  C.d_prow.upload(prow, nullptr);
+  C.dense = nb * bs <= CR_DENSE;
+  C.ld = (C.nc + CR_TILE - 1) / CR_TILE * CR_TILE;
+  C.winv.release();
   C.d_state.release();
   C.d_slot_dst.upload(C.slot_dst, nullptr);
   HIPCHECK(hipDeviceSynchronize());
@@ -701,8 +812,45 @@ static bool cr_factor_device(Ctx& c, Coarse& C)
   return bad == 0;
 }
 
+template <int RA>
+static void cr_units(Ctx& c, Coarse& C)
+{
+  const int nb = C.nb, bs = C.bs, ld = C.ld;
+  const unsigned tiles = (unsigned)(ld / CR_TILE);
+  const size_t lds = sizeof(double) * bs * CR_TILE;
+  double* W = C.winv.p;
+  k_cr_units<<<2048, 256, 0, c.stream>>>((long long)nb * bs * ld, ld, C.nc, C.d_prow.p, W);
+  for (int l = 0; l < C.levels; l++) {
+    const int s = 1 << l;
+    k_cr_unit_fwd<RA><<<dim3((nb + 2 * s - 1) / (2 * s), tiles), 256, 0, c.stream>>>(
+        nb, bs, s, C.mats.p + C.lev_keep[l], W, ld);
+  }
+  k_cr_unit_bwd<RA><<<dim3(1, tiles), 256, lds, c.stream>>>(nb, bs, 0, C.mats.p + C.top_off, W, ld);
+  for (int l = C.levels - 1; l >= 0; l--) {
+    const int s = 1 << l;
+    k_cr_unit_bwd<RA><<<dim3((nb - s + 2 * s - 1) / (2 * s), tiles), 256, lds, c.stream>>>(
+        nb, bs, s, C.mats.p + C.lev_elim[l], W, ld);
+  }
+  HIPCHECK(hipGetLastError());
+}
+
+// The inverse of a small coarse matrix, after its reduction has been factored.
+static void cr_invert(Ctx& c, Coarse& C)
+{
+  if (!C.dense) return;
+  C.winv.alloc((size_t)C.nb * C.bs * C.ld);
+  if (C.bs <= 32) cr_units<8>(c, C);
+  else if (C.bs <= 64) cr_units<16>(c, C);
+  else cr_units<32>(c, C);
+}
+
 static void cr_apply(Ctx& c, Coarse& C)
 {
+  if (C.dense) {
+    k_cr_dense<<<(C.nc + 3) / 4, 256, 0, c.stream>>>(C.nc, C.ld, C.d_prow.p, C.winv.p, C.rc.p, C.zc.p);
+    HIPCHECK(hipGetLastError());
+    return;
+  }
   int spin = 1 << 22;
   if (const char* e = getenv("RMX_COARSE_SPIN")) spin = std::max(1, atoi(e));
   k_cr_solve<<<2 * C.nb - 1, CR_THREADS, 0, c.stream>>>(C.nb, C.bs, C.levels, C.d_order.p,
@@ -894,6 +1042,7 @@ void coarse_factor(Ctx& c, int prec)
   }
   // the block cyclic reduction factored on the device (RMX_COARSE_HOST_FACTOR: on the host)
   if (C.cr_ok && !getenv("RMX_COARSE_HOST_FACTOR") && cr_factor_device(c, C)) {
+    cr_invert(c, C);
     C.cr_fac = true;
     C.fac = true;
     C.fac_prec = prec;
@@ -905,6 +1054,7 @@ void coarse_factor(Ctx& c, int prec)
     HIPCHECK(hipMemcpyAsync(C.mats.p, C.h_mats.data(), sizeof(double) * C.mats_n,
                             hipMemcpyHostToDevice, c.stream));
     HIPCHECK(hipStreamSynchronize(c.stream));
+    cr_invert(c, C);
     C.cr_fac = true;
     C.fac = true;
     C.fac_prec = prec;
@@ -929,12 +1079,12 @@ void coarse_apply(Ctx& c, int prec, const double* r, double* z)
   // bytes: restriction (row lists, r), coarse solve (its matrices), A P residual (A P
   // entries and aggregates, r, t)
   const int kt = kt_begin(c, KT_COARSE, 4.0 * (C.nc + 1) + 12.0 * n + 8.0 * C.nc +
-                                        (C.cr_fac ? 8.0 * (double)C.mats_n : 0.0) +
+                                        (C.cr_fac ? 8.0 * (C.dense ? (double)C.nc * C.nc : (double)C.mats_n) : 0.0) +
                                         12.0 * (double)C.nap + 4.0 * (n + 1) + 16.0 * n);
   k_restrict<<<(C.nc * 64 + 255) / 256, 256, 0, c.stream>>>(C.nc, C.agg_ptr.p, C.agg_rows.p, r, C.rc.p);
   if (C.cr_fac) {
     cr_apply(c, C);
-    C.applied = true;
+    C.applied = !C.dense;
   } else {
     HIPCHECK(hipMemcpyAsync(C.h_buf, C.rc.p, sizeof(double) * C.nc, hipMemcpyDeviceToHost, c.stream));
     HIPCHECK(hipStreamSynchronize(c.stream));

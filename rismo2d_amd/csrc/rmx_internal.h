@@ -260,6 +260,10 @@ struct Coarse {
   DBuf<long long> d_off;                      // lev_elim, lev_keep
   DBuf<unsigned long long> d_state;           // task counter, abort flag, exchanged words
   bool applied = false;                       // applied since the abort flag was read
+  bool dense = false;                         // small: applied as the inverse winv
+  int ld = 0;
+  DBuf<int> d_prow;                           // row of winv of every aggregate
+  DBuf<double> winv;                          // [nb * bs][ld]
   DBuf<int> d_blk_start;
   DBuf<long long> d_slot_dst;
   DBuf<double> d_blocks, d_inv, d_tmp;        // device factorisation: B, A, C blocks; inverses

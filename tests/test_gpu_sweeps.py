@@ -177,3 +177,11 @@ def test_two_level_on_thin_strips(ctx, nx, ny, strips, cseg):
             assert np.abs(y - ref).max() <= 1e-9 * np.abs(ref).max(), prec
     ctx.set_coarse(-1)
     ctx.set_strips(0, 0)
+
+
+# blocks of up to 32, 64 and more coarse unknowns in the product with the inverse; the largest
+# system that takes it (3,060 of 3,072 rows) and the next one (3,264), which takes the chain
+@pytest.mark.parametrize("ny,strips,cseg", [(130, 6, 6), (130, 5, 15), (130, 7, 30), (260, 0, 15),
+                                            (260, 0, 16)])
+def test_two_level_inverse_and_chain(ctx, ny, strips, cseg):
+    test_two_level_on_thin_strips(ctx, 60, ny, strips, cseg)
