@@ -14,7 +14,8 @@
 //    It preconditions the FP32 solve inside the FP64 refinement, where the FP64 residual,
 //    not the preconditioner, decides the answer.
 //
-// Factorisation: row-wise, one wave per row, the rows of one level in one launch; row i
+// Factorisation: one persistent launch, one wave per unit of up to three rows (k_unit_flow), or
+// per row where the pattern does not allow that and after a pivot repair (k_ilu_flow); row i
 // eliminates its lower entries in increasing column order, so every factor entry gets its
 // updates in the reference's order and, with FMA contraction off, the reference's
 // rounding.  Multipliers are stored negated as in the reference.
@@ -616,6 +617,294 @@ __global__ void __launch_bounds__(64) k_ilu_flow(const int4* __restrict__ desc, 
       }
     }
     wave_sync();                                   // LDS reused by the next row
+  }
+}
+
+// ---- dataflow factorisation by units ----
+//
+// A unit is a node's rows (up to 3, one column set), and one wave factors it: lane l holds
+// column l (and l + 64) of each row in registers, so that an entry of a pivot row is read once
+// for all rows of the unit, a multiplier's way is two lane reads and one division (the rows'
+// numerators side by side in its lanes), and the rows hand on to each other without leaving
+// the wave.  What bounds the factorisation is the chain from a row to the next that needs it
+// (store, flag, poll, load: some 3.4 us); the chain has a third of the links of the row-by-row
+// kernel.  Pivot units are taken in ascending order as far as their flags are set; a finished
+// unit's rows go out column by column (U: 3 words a column, from the unit's first row's own
+// column on), and a plan (per pivot unit and lane: the column's place there, 255: none) makes
+// the read of a pivot unit one load per lane.  Updates, order and rounding are those of
+// k_ilu_flow.  FP32 at 200 x 20, 80 x 320, 640 x 320 cells: 1.25, 6.4, 17.5 ms, row by row 4.4,
+// 19.5, 48; FP64 at 80 x 320 7.9 ms, row by row 21.8.
+
+constexpr int FU = 3;             // rows of a unit
+constexpr int FP = 64;            // pivot units of a unit
+
+// desc: {first row, its CSR start, width | rows << 8 | pivot units << 16, own columns' place},
+// {pivot list, plan (64-byte lines), place in U (columns), 0}; a pivot unit's entry: {place in
+// U, place of its columns | its rows << 8, its last row, its position in desc}
+struct FlowUnit { int r0, p0, w, rows, np, sd, list, line, ub; };
+__device__ __forceinline__ FlowUnit flow_unit(const int4* __restrict__ desc, int k)
+{
+  const int4 a = desc[2 * k], b = desc[2 * k + 1];
+  return { a.x, a.y, a.z & 255, (a.z >> 8) & 255, a.z >> 16, a.w, b.x, b.y, b.z };
+}
+
+__global__ void __launch_bounds__(64) k_unit_plan(const int4* __restrict__ desc,
+                                                  const int4* __restrict__ list,
+                                                  const int* __restrict__ srt_cols,
+                                                  unsigned char* __restrict__ plan)
+{
+  const FlowUnit u = flow_unit(desc, blockIdx.x);
+  const int slots = u.w > 64 ? 2 : 1;
+  for (int t = 0; t < u.np; t++) {
+    const FlowUnit v = flow_unit(desc, list[u.list + t].w);
+    for (int c = 0; c < slots; c++) {
+      const int l = threadIdx.x + 64 * c;
+      int pos = 255;
+      if (l < u.w) {
+        const int cc = srt_cols[u.p0 + l];
+        int lo = v.sd, hi = v.w - 1;
+        while (lo <= hi) {
+          const int mid = (lo + hi) >> 1;
+          const int x = srt_cols[v.p0 + mid];
+          if (x == cc) { pos = mid - v.sd; break; }
+          if (x < cc) lo = mid + 1; else hi = mid - 1;
+        }
+      }
+      plan[64LL * (u.line + t * slots + c) + threadIdx.x] = (unsigned char)pos;
+    }
+  }
+}
+
+__device__ __forceinline__ float lane_of(float x, int l)
+{
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
+}
+__device__ __forceinline__ double lane_of(double x, int l)
+{
+  const u32x2 w = __builtin_bit_cast(u32x2, x);
+  u32x2 r;
+  r.x = (unsigned)__builtin_amdgcn_readlane((int)w.x, l);
+  r.y = (unsigned)__builtin_amdgcn_readlane((int)w.y, l);
+  return __builtin_bit_cast(double, r);
+}
+// column p of a row held in C registers a lane
+template <class VT, int C>
+__device__ __forceinline__ VT col_of(const VT* x, int p)
+{
+  if (C == 1) return lane_of(x[0], p);
+  return p < 64 ? lane_of(x[0], p) : lane_of(x[C - 1], p - 64);
+}
+
+typedef unsigned u32x3 __attribute__((ext_vector_type(3)));
+// the 3 words of column m (of a pivot unit's rows), sc1
+__device__ __forceinline__ void ld_col(__amdgpu_buffer_rsrc_t r, unsigned m, float* v)
+{
+  const u32x3 w = __builtin_amdgcn_raw_buffer_load_b96(r, m * 12u, 0, 16);
+  const unsigned x[3] = { w.x, w.y, w.z };
+#pragma unroll
+  for (int q = 0; q < 3; q++) v[q] = __builtin_bit_cast(float, x[q]);
+}
+__device__ __forceinline__ void ld_col(__amdgpu_buffer_rsrc_t r, unsigned m, double* v)
+{
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+    v[q] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, m * 24u + 8u * q, 0, 16));
+}
+__device__ __forceinline__ void st_col(__amdgpu_buffer_rsrc_t r, unsigned m, float a, float b, float c)
+{
+  const u32x3 w = { __builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                    __builtin_bit_cast(unsigned, c) };
+  __builtin_amdgcn_raw_buffer_store_b96(w, r, m * 12u, 0, 16);
+}
+__device__ __forceinline__ void st_col(__amdgpu_buffer_rsrc_t r, unsigned m, double a, double b, double c)
+{
+  const double x[3] = { a, b, c };
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x[q]), r, m * 24u + 8u * q, 0, 16);
+}
+
+// rows FROM.. of a unit minus their multiples of pivot row v (pivot dk, column place p): the
+// rows' numerators go through one division
+template <class VT, int C, int FROM>
+__device__ __forceinline__ void unit_step(VT (&a)[FU][C], const VT* v, const bool* has, int p, VT dk)
+{
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x;
+  VT num = col_of<VT, C>(a[FU - 1], p);
+#pragma unroll
+  for (int r = FU - 2; r >= FROM; r--) {
+    const VT x = col_of<VT, C>(a[r], p);
+    num = lane == r ? x : num;
+  }
+  const VT f = -num / dk;
+#pragma unroll
+  for (int r = FROM; r < FU; r++) {
+    const VT fr = lane_of(f, r);
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      const int l = lane + 64 * c;
+      const VT prod = fr * v[c];
+      const VT sum = a[r][c] + prod;
+      a[r][c] = has[c] && l > p ? sum : a[r][c];
+      a[r][c] = l == p ? fr : a[r][c];
+    }
+  }
+}
+
+// One unit; false: a wait was given up.
+template <class VT, int C, class Wait>
+__device__ __forceinline__ bool factor_unit(const FlowUnit& u, const int4* __restrict__ list,
+                                            const unsigned char* __restrict__ plan,
+                                            const unsigned char* __restrict__ srt_pos,
+                                            VT* __restrict__ LU, VT* __restrict__ U, int* done,
+                                            int epoch, int* state, unsigned char* s_plan,
+                                            Wait wait_row)
+{
+  constexpr int B = sizeof(VT) == 4 ? 4 : 2;     // pivot units whose loads are in flight together
+  const int lane = threadIdx.x;
+  int pos[FU][C];
+  VT a[FU][C];
+#pragma unroll
+  for (int r = 0; r < FU; r++)
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      const int l = lane + 64 * c;
+      pos[r][c] = r < u.rows && l < u.w ? (int)srt_pos[u.p0 + r * u.w + l] : 0;
+    }
+  int4 pv = {0, 0, 0, 0};
+  if (lane < u.np) pv = list[u.list + lane];
+  {
+    const unsigned* src = reinterpret_cast<const unsigned*>(plan) + 16LL * u.line;
+    unsigned* dst = reinterpret_cast<unsigned*>(s_plan);
+    for (int k = lane; k < 16 * C * u.np; k += 64) dst[k] = src[k];
+  }
+#pragma unroll
+  for (int r = 0; r < FU; r++)
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      const int l = lane + 64 * c;
+      a[r][c] = r < u.rows && l < u.w ? LU[u.p0 + r * u.w + pos[r][c]] : (VT)0;
+    }
+  wave_sync();
+  int ta = 0;
+  while (ta < u.np) {
+    const bool ok = lane < ta || lane >= u.np || ld_flag(done + pv.z) == epoch;
+    const unsigned long long pend = __ballot(!ok);
+    int tb = pend ? (int)__builtin_ctzll(pend) : u.np;
+    if (tb == ta) {                              // its flag was read last: it alone
+      if (!wait_row(__builtin_amdgcn_readlane(pv.z, ta))) return false;
+      tb = ta + 1;
+    }
+    // loads of the pivot units' rows only after their flags
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    for (int t0 = ta; t0 < tb; t0 += B) {
+      VT v[B][C][FU];
+      bool has[B][C];
+#pragma unroll
+      for (int b = 0; b < B; b++) {
+        const int t = min(t0 + b, tb - 1);
+        const __amdgpu_buffer_rsrc_t ru =
+            sc1_rsrc(U + 3LL * __builtin_amdgcn_readlane(pv.x, t));
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+          const unsigned m = s_plan[64 * (t * C + c) + lane];
+          has[b][c] = m != 255;
+          ld_col(ru, m == 255 ? 0u : m, v[b][c]);
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < B; b++)
+        if (t0 + b < tb) {
+          const int y = __builtin_amdgcn_readlane(pv.y, t0 + b);
+          const int s0 = y & 255, rows = y >> 8;
+#pragma unroll
+          for (int q = 0; q < FU; q++)
+            if (q < rows) {
+              VT x[C];
+#pragma unroll
+              for (int c = 0; c < C; c++) x[c] = v[b][c][q];
+              unit_step<VT, C, 0>(a, x, has[b], s0 + q, col_of<VT, C>(x, s0 + q));
+            }
+        }
+    }
+    ta = tb;
+  }
+  bool has[C];
+#pragma unroll
+  for (int c = 0; c < C; c++) has[c] = true;
+  if (u.rows > 1) unit_step<VT, C, 1>(a, a[0], has, u.sd, col_of<VT, C>(a[0], u.sd));
+  if (u.rows > 2) unit_step<VT, C, 2>(a, a[1], has, u.sd + 1, col_of<VT, C>(a[1], u.sd + 1));
+  const __amdgpu_buffer_rsrc_t ro = sc1_rsrc(U + 3LL * u.ub);
+#pragma unroll
+  for (int c = 0; c < C; c++) {
+    const int l = lane + 64 * c;
+    if (l >= u.sd && l < u.w) st_col(ro, (unsigned)(l - u.sd), a[0][c], a[1][c], a[2][c]);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);            // vmcnt(0): the rows are performed
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  if (lane < u.rows) st_flag(done + u.r0 + lane, epoch);
+#pragma unroll
+  for (int r = 0; r < FU; r++)
+    if (r < u.rows) {
+#pragma unroll
+      for (int c = 0; c < C; c++) {
+        const int l = lane + 64 * c;
+        if (l < u.w) LU[u.p0 + r * u.w + pos[r][c]] = a[r][c];
+      }
+      const VT d = col_of<VT, C>(a[r], u.sd + r);
+      if (lane == 0 && fabs((double)d) < 1.0e-20) {
+        atomicOr(state + FLOW_ERR, 1);
+        atomicMin(state + FLOW_BADROW, u.r0 + r);
+      }
+    }
+  return true;
+}
+
+template <class VT>
+__global__ void __launch_bounds__(64) k_unit_flow(const int4* __restrict__ desc, int nu,
+                                                  const int4* __restrict__ list,
+                                                  const unsigned char* __restrict__ plan,
+                                                  const unsigned char* __restrict__ srt_pos,
+                                                  VT* __restrict__ LU, VT* __restrict__ U,
+                                                  int* __restrict__ done, int epoch,
+                                                  int* __restrict__ state, int spin_limit)
+{
+  __shared__ __attribute__((aligned(16))) unsigned char s_plan[FP * 128];
+  const int lane = threadIdx.x;
+  int polls = 0;
+  auto wait_row = [&](int k) -> bool {
+    for (;;) {
+      int v = 0;
+      if (lane == 0) v = ld_flag(done + k);
+      if (__builtin_amdgcn_readfirstlane(v) == epoch) return true;
+      if ((++polls & 31) == 0) {
+        int ab = 0;
+        if (lane == 0) ab = ld_flag(state + FLOW_ABORT);
+        if (__builtin_amdgcn_readfirstlane(ab) != 0 || polls > spin_limit) return false;
+      }
+      __builtin_amdgcn_s_sleep(8);
+    }
+  };
+  auto ticket = [&]() {
+    int w = 0;
+    if (lane == 0) w = __hip_atomic_fetch_add(state + FLOW_COUNTER, 1, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_amdgcn_readfirstlane(w);
+  };
+  for (;;) {
+    const int w = ticket();
+    if (w >= nu) break;
+    const FlowUnit u = flow_unit(desc, w);
+    polls = 0;
+    const bool ok = u.w > 64
+        ? factor_unit<VT, 2>(u, list, plan, srt_pos, LU, U, done, epoch, state, s_plan, wait_row)
+        : factor_unit<VT, 1>(u, list, plan, srt_pos, LU, U, done, epoch, state, s_plan, wait_row);
+    if (!ok) {
+      if (lane == 0) st_flag(state + FLOW_ABORT, 1);
+      break;
+    }
+    wave_sync();                                   // LDS reused by the next unit
   }
 }
 
@@ -2124,6 +2413,119 @@ std::vector<int> cut_segments(const std::vector<int>& bstart, const std::vector<
   return seg;
 }
 
+// Schedule of the row-by-row factorisation: rows by lower level of the whole pattern, per
+// level position {row, start, width, lower entries}, per sorted lower entry the start and
+// length (after the diagonal) of its pivot row, and the plan.
+static void build_rows(Ilu& I, const std::vector<int>& scol, hipStream_t s)
+{
+  const int n = I.n;
+  std::vector<int> lev(n, 0), fptr, frows;
+  levels(0, n, I.h_rp, I.h_cols, true, std::vector<int>(), lev, fptr, frows);
+  I.flev = fptr;
+  std::vector<int4> desc(n);
+  std::vector<int2> piv(I.nnz, int2{0, 0});
+  parallel_for(n, [&](long long a, long long e) {
+    for (long long w = a; w < e; w++) {
+      const int i = frows[w];
+      const int p0 = I.h_rp[i], wi = I.h_rp[i + 1] - p0;
+      int nk = 0;
+      while (nk < wi && scol[p0 + nk] < i) {
+        const int k = scol[p0 + nk];
+        piv[p0 + nk] = int2{ I.h_rp[k], I.h_rp[k + 1] - I.h_rp[k] - 1 };
+        nk++;
+      }
+      desc[w] = int4{ i, p0, wi, nk };
+    }
+  });
+  // plan offsets: every row's concatenated pivot-row entries
+  std::vector<long long> pbase(n + 1, 0);
+  for (int w = 0; w < n; w++) {
+    long long tot = 0;
+    for (int t = 0; t < desc[w].w; t++) tot += piv[desc[w].y + t].y;
+    pbase[w + 1] = pbase[w] + tot;
+  }
+  I.fdesc.upload(desc, s);
+  I.fpiv.upload(piv, s);
+  I.fpbase.upload(pbase, s);
+  I.plan.alloc(std::max<long long>(pbase[n], 1));
+  k_ilu_plan<<<n, 64, 0, s>>>(I.fdesc.p, n, I.cols.p, I.srt_cols.p, I.srt_pos.p, I.fpiv.p,
+                              I.fpbase.p, I.plan.p);
+  HIPCHECK(hipGetLastError());
+  HIPCHECK(hipStreamSynchronize(s));
+}
+
+// Schedule of the factorisation by units of up to `rows_max` rows.  False: a unit of more than
+// FP pivot units, or a pattern that couples a unit to some rows of another.
+static bool build_units(Ilu& I, const std::vector<int>& unit, int rows_max,
+                        const std::vector<int>& scol, hipStream_t s)
+{
+  FlowUnits& F = I.fu;
+  F.nu = 0;
+  F.desc.release(); F.list.release(); F.plan.release(); F.u32.release(); F.u64.release();
+  const int n = I.n;
+  const std::vector<int>& rp = I.h_rp;
+  std::vector<int> start, of(n);
+  for (int i = 0; i < n; i++) {
+    const int w = rp[i + 1] - rp[i];
+    const bool same = i > 0 && unit[i] == unit[i - 1] && i - start.back() < rows_max &&
+                      w == rp[i] - rp[i - 1] &&
+                      std::equal(&scol[rp[i]], &scol[rp[i]] + w, &scol[rp[i - 1]]);
+    if (!same) start.push_back(i);
+    of[i] = (int)start.size() - 1;
+  }
+  const int nu = (int)start.size();
+  start.push_back(n);
+  // pivot units, places, levels
+  std::vector<int> lst(nu + 1, 0), sd(nu), lev(nu, 0);
+  std::vector<int4> piv;
+  piv.reserve(rp[n] / 4);
+  std::vector<long long> ub(nu + 1, 0);
+  int top = 0;
+  for (int g = 0; g < nu; g++) {
+    const int r0 = start[g], rows = start[g + 1] - r0, p0 = rp[r0], w = rp[r0 + 1] - p0;
+    int t = 0;
+    while (t < w && scol[p0 + t] < r0) {
+      const int K = of[scol[p0 + t]], R = start[K + 1] - start[K];
+      for (int q = 0; q < R; q++)
+        if (t + q >= w || scol[p0 + t + q] != start[K] + q) return false;
+      piv.push_back(int4{ (int)ub[K], t | R << 8, start[K + 1] - 1, K });
+      lev[g] = std::max(lev[g], lev[K] + 1);
+      t += R;
+    }
+    for (int q = 0; q < rows; q++)
+      if (t + q >= w || scol[p0 + t + q] != r0 + q) return false;
+    sd[g] = t;
+    top = std::max(top, lev[g]);
+    lst[g + 1] = (int)piv.size();
+    if (lst[g + 1] - lst[g] > FP) return false;
+    ub[g + 1] = ub[g] + (w - t);
+  }
+  std::vector<int> ptr(top + 2, 0), at(nu);
+  for (int g = 0; g < nu; g++) ptr[lev[g] + 1]++;
+  for (int l = 0; l <= top; l++) ptr[l + 1] += ptr[l];
+  for (int g = 0; g < nu; g++) at[g] = ptr[lev[g]]++;
+  std::vector<int4> desc(2 * (size_t)nu);
+  long long lines = 0;
+  for (int g = 0; g < nu; g++) {
+    const int r0 = start[g], p0 = rp[r0], w = rp[r0 + 1] - p0, np = lst[g + 1] - lst[g];
+    desc[2 * (size_t)at[g]] = int4{ r0, p0, w | (start[g + 1] - r0) << 8 | np << 16, sd[g] };
+    desc[2 * (size_t)at[g] + 1] = int4{ lst[g], (int)lines, (int)ub[g], 0 };
+    lines += (long long)np * (w > 64 ? 2 : 1);
+  }
+  if (lines > INT_MAX || ub[nu] > INT_MAX) return false;
+  for (int4& e : piv) e.w = at[e.w];
+  if (piv.empty()) piv.push_back(int4{ 0, 0, 0, 0 });
+  F.nu = nu;
+  F.cols = ub[nu];
+  F.desc.upload(desc, s);
+  F.list.upload(piv, s);
+  F.plan.alloc(64 * (size_t)std::max(lines, 1LL));
+  k_unit_plan<<<nu, 64, 0, s>>>(F.desc.p, F.list.p, I.srt_cols.p, F.plan.p);
+  HIPCHECK(hipGetLastError());
+  HIPCHECK(hipStreamSynchronize(s));
+  return true;
+}
+
 // Strips: contiguous row ranges of about equal size.  With `group` (the node of every
 // equation) a cut moves forward to the next row of another node, so the U, V, H equations
 // of one node stay in one strip.  level_cap > 0 splits the sweeps' levels into parts of at
@@ -2159,11 +2561,6 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   I.h_rp = rp;
   I.h_cols = cl;
   I.nnz = I.h_rp[n];
-  // factorisation schedule: lower levels of the whole pattern
-  std::vector<int> lev(n, 0), fptr, frows;
-  levels(0, n, I.h_rp, I.h_cols, true, std::vector<int>(), lev, fptr, frows);
-  I.flev = fptr;
-  I.flev_rows.upload(frows, s);
   // per-row sorted columns for the factorisation lookups
   std::vector<int> scol(I.nnz);
   std::vector<unsigned char> spos(I.nnz);
@@ -2183,39 +2580,13 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   });
   I.rp.upload(I.h_rp, s); I.cols.upload(I.h_cols, s);
   I.srt_cols.upload(scol, s); I.srt_pos.upload(spos, s);
-  // factorisation metadata: per level position {row, start, width, lower entries}; per
-  // sorted lower entry the start and length (after the diagonal) of its pivot row
-  {
-    std::vector<int4> desc(n);
-    std::vector<int2> piv(I.nnz, int2{0, 0});
-    parallel_for(n, [&](long long a, long long e) {
-      for (long long w = a; w < e; w++) {
-        const int i = frows[w];
-        const int p0 = I.h_rp[i], wi = I.h_rp[i + 1] - p0;
-        int nk = 0;
-        while (nk < wi && scol[p0 + nk] < i) {
-          const int k = scol[p0 + nk];
-          piv[p0 + nk] = int2{ I.h_rp[k], I.h_rp[k + 1] - I.h_rp[k] - 1 };
-          nk++;
-        }
-        desc[w] = int4{ i, p0, wi, nk };
-      }
-    });
-    // plan offsets: every row's concatenated pivot-row entries
-    std::vector<long long> pbase(n + 1, 0);
-    for (int w = 0; w < n; w++) {
-      long long tot = 0;
-      for (int t = 0; t < desc[w].w; t++) tot += piv[desc[w].y + t].y;
-      pbase[w + 1] = pbase[w] + tot;
-    }
-    I.fdesc.upload(desc, s);
-    I.fpiv.upload(piv, s);
-    I.fpbase.upload(pbase, s);
-    I.plan.alloc(std::max<long long>(pbase[n], 1));
-    k_ilu_plan<<<n, 64, 0, s>>>(I.fdesc.p, n, I.cols.p, I.srt_cols.p, I.srt_pos.p, I.fpiv.p,
-                                I.fpbase.p, I.plan.p);
-    HIPCHECK(hipGetLastError());
-  }
+  I.flev.clear();
+  I.fdesc.release();
+  // units, of single rows where the pattern couples parts of runs, else row by row (single
+  // rows, FP64, 36,000 in a band of 8 a side, 4,000 in one of 30: 54 and 6.2 ms, row by row 78
+  // and 8.6)
+  if (!build_units(I, unit, FU, scol, s) && !build_units(I, unit, 1, scol, s))
+    build_rows(I, scol, s);
   // strip sweeps: a level of more rows than the staged sweep's row groups (512 threads, 4
   // lanes per row) is split, so that no level needs a second round, whose entries would be
   // loaded inside the level instead of one level ahead
@@ -2282,6 +2653,10 @@ template <class VT> static DBuf<VT>& PDbuf(Ilu& I);
 template <> DBuf<double>& PDbuf<double>(Ilu& I) { return I.pdg64; }
 template <> DBuf<float>& PDbuf<float>(Ilu& I) { return I.pdg32; }
 
+template <class VT> static DBuf<VT>& FUbuf(Ilu& I);
+template <> DBuf<double>& FUbuf<double>(Ilu& I) { return I.fu.u64; }
+template <> DBuf<float>& FUbuf<float>(Ilu& I) { return I.fu.u32; }
+
 template <class VT>
 static void factor_t(Ctx& c, Ilu& I, const VT* A)
 {
@@ -2290,9 +2665,16 @@ static void factor_t(Ctx& c, Ilu& I, const VT* A)
   HIPCHECK(hipMemcpyAsync(LU.p, A, sizeof(VT) * I.nnz, hipMemcpyDeviceToDevice, c.stream));
   int* err = reinterpret_cast<int*>(c.red.p + 8);
   HIPCHECK(hipMemsetAsync(err, 0, sizeof(int), c.stream));
-  const long long plan_n = (long long)I.plan.n;
+  auto need_rows = [&]() {
+    if (I.fdesc.p) return;
+    std::vector<int> scol(I.nnz);
+    I.srt_cols.download(scol.data(), I.nnz, c.stream);
+    HIPCHECK(hipStreamSynchronize(c.stream));
+    build_rows(I, scol, c.stream);
+  };
   const char* lv = getenv("RMX_ILU_LEVELS");
   if (!(lv && atoi(lv) == 1)) {
+    if (!I.fu.nu) need_rows();
     // one persistent launch: rows in level order, pivot rows awaited by completion flags
     if (I.done.n != (size_t)I.n) {
       I.done.alloc(I.n);
@@ -2316,6 +2698,12 @@ static void factor_t(Ctx& c, Ilu& I, const VT* A)
     per_cu = std::max(1, std::min(per_cu, 3));
     int nwg = (int)std::min<long long>(I.n, (long long)per_cu * prop.multiProcessorCount);
     if (const char* e = getenv("RMX_ILU_WAVES")) nwg = std::max(1, std::min(nwg, atoi(e)));
+    // by units three waves on two CUs: a wave that waits polls, and the polls slow the others'
+    // loads (FP32, ms at 200 x 20, 80 x 320, 640 x 320 cells: 192 waves 1.2, 6.5, 25; 384 1.3,
+    // 6.4, 17; 768 1.5, 7.8, 26; with the row-by-row kernel's pause between polls 384 waves
+    // take 1.4, 7.4, 19)
+    int nwu = 3 * prop.multiProcessorCount / 2;
+    if (const char* e = getenv("RMX_ILU_WAVES")) nwu = std::max(1, std::min(4096, atoi(e)));
     int spin = 1 << 22;
     if (const char* e = getenv("RMX_ILU_SPIN")) spin = std::max(32, atoi(e));
     // a pass factors every row after skip; a pivot below 1e-20 is repaired as the
@@ -2328,9 +2716,18 @@ static void factor_t(Ctx& c, Ilu& I, const VT* A)
       HIPCHECK(hipMemcpyAsync(I.flow_state.p, st, sizeof(int) * 4, hipMemcpyHostToDevice,
                               c.stream));
       const int kt = kt_begin(c, KT_FACTOR, 3.0 * (double)I.nnz * (sizeof(VT) + 4));
-      k_ilu_flow<VT><<<nwg, 64, 0, c.stream>>>(I.fdesc.p, I.n, I.cols.p, I.srt_cols.p,
-                                               I.srt_pos.p, I.fpiv.p, I.fpbase.p, I.plan.p, LU.p,
-                                               I.done.p, I.epoch, I.flow_state.p, spin, skip);
+      if (I.fu.nu && skip < 0) {
+        DBuf<VT>& U = FUbuf<VT>(I);
+        U.alloc(FU * (size_t)I.fu.cols);
+        k_unit_flow<VT><<<std::min(I.fu.nu, nwu), 64, 0, c.stream>>>(
+            I.fu.desc.p, I.fu.nu, I.fu.list.p, I.fu.plan.p, I.srt_pos.p, LU.p, U.p, I.done.p,
+            I.epoch, I.flow_state.p, spin);
+      } else {
+        k_ilu_flow<VT><<<nwg, 64, 0, c.stream>>>(I.fdesc.p, I.n, I.cols.p, I.srt_cols.p,
+                                                 I.srt_pos.p, I.fpiv.p, I.fpbase.p, I.plan.p,
+                                                 LU.p, I.done.p, I.epoch, I.flow_state.p, spin,
+                                                 skip);
+      }
       kt_end(c, kt);
       HIPCHECK(hipGetLastError());
       HIPCHECK(hipMemcpyAsync(st, I.flow_state.p, sizeof(int) * 4, hipMemcpyDeviceToHost,
@@ -2362,8 +2759,11 @@ static void factor_t(Ctx& c, Ilu& I, const VT* A)
         k_flags_clear<<<(I.n - bad - 1 + 255) / 256, 256, 0, c.stream>>>(bad + 1, I.n, I.done.p);
       HIPCHECK(hipGetLastError());
       skip = bad;
+      need_rows();
     }
   } else {
+  need_rows();
+  const long long plan_n = (long long)I.plan.n;
   const int kt = kt_begin(c, KT_FACTOR, 3.0 * (double)I.nnz * (sizeof(VT) + 4));
   for (size_t l = 0; l + 1 < I.flev.size(); l++) {
     const int a = I.flev[l], cnt = I.flev[l + 1] - a;

@@ -182,15 +182,27 @@ struct NodeSweep {
 };
 
 // One ILU(0) system: pattern, factorisation schedule, sweeps and factors.
+// Factorisation by units (the rows of a node): schedule, and the finished rows as its waves
+// hand them on.
+struct FlowUnits {
+  int nu = 0;                   // units (0: the pattern takes the row-by-row kernel)
+  long long cols = 0;           // columns of the units from their first row on
+  DBuf<int4> desc, list;        // two per unit in level order; one per pivot unit of a unit
+  DBuf<unsigned char> plan;     // per pivot unit and column of a unit: the column's place there
+  DBuf<float> u32;              // [cols][3]
+  DBuf<double> u64;
+};
+
 struct Ilu {
   bool ready = false;
   int n = 0, nblk = 1, nseg = 1;
   std::vector<int> seg;         // segment of every row (empty: one segment per strip)
   long long nnz = 0;
   std::vector<int> bstart, h_rp, h_cols, flev;
-  DBuf<int> rp, cols, srt_cols, flev_rows, fwd2bwd;
+  DBuf<int> rp, cols, srt_cols, fwd2bwd;
   DBuf<unsigned char> srt_pos;
-  DBuf<int4> fdesc;             // factorisation: per level position {row, start, width, lower}
+  FlowUnits fu;
+  DBuf<int4> fdesc;             // row-by-row factorisation: per level position {row, start, width, lower}
   DBuf<int2> fpiv;              // per sorted lower entry: pivot row start, entries after diag
   DBuf<long long> fpbase;       // per level position: offset of its plan entries
   DBuf<unsigned short> plan;    // per plan entry: pivot index | target position << 8

@@ -185,3 +185,42 @@ def test_two_level_on_thin_strips(ctx, nx, ny, strips, cseg):
                                             (260, 0, 16)])
 def test_two_level_inverse_and_chain(ctx, ny, strips, cseg):
     test_two_level_on_thin_strips(ctx, 60, ny, strips, cseg)
+
+
+# factorisation by units: runs of 2 and 3 rows with one set of columns, longer runs (units of 3
+# and a rest), one dense block; 62 to 68 and 123 to 128 columns (one and two columns a lane);
+# `zero`: rows inside and at the ends of units whose diagonal and lower entries are zero, so
+# that their pivots are repaired.  As for the row-by-row kernel: FP32 factors the oracle's
+# bits, FP64 ones to 1e-12.
+@pytest.mark.parametrize("n,width,stride,run,zero", [
+    (2, 0, 1, 2, ()), (3, 0, 1, 3, ()), (4, 0, 1, 4, ()), (64, 0, 1, 64, ()), (65, 0, 1, 65, ()),
+    (128, 0, 1, 128, ()), (600, 15, 2, 2, ()), (600, 16, 3, 2, ()), (500, 31, 1, 2, ()),
+    (900, 10, 2, 3, ()), (900, 20, 1, 3, ()), (800, 8, 3, 4, ()), (600, 15, 1, 4, ()),
+    (3000, 4, 7, 3, ()), (900, 4, 2, 3, (6, 10, 14, 300, 301, 898)), (600, 16, 1, 2, (1, 100, 598))])
+def test_factorisation_by_units(ctx, n, width, stride, run, zero):
+    print(f"[gpu] factorisation of {n} rows in runs of {run}, {width} runs a side", flush=True)
+    rp0, c0, _ = _band_csr(n // run, [1 + stride * k for k in range(width)], 31)
+    rng = np.random.default_rng(32)
+    rp, cols, vals = [0], [], []
+    for i in range(n // run):
+        js = (run * c0[rp0[i]:rp0[i + 1], None] + np.arange(run)).ravel()
+        for r in range(run * i, run * i + run):
+            o = rng.permutation(js[js != r])
+            v = rng.standard_normal(len(o))
+            d = np.abs(v).sum() + 1.0
+            if r in zero:
+                d, v = 0.0, np.where(o < r, 0.0, v)
+            cols += [r] + o.tolist()
+            vals += [d] + v.tolist()
+            rp.append(len(cols))
+    rp, cols, vals = np.asarray(rp, np.int32), np.asarray(cols, np.int32), np.asarray(vals)
+    ctx.csr_upload(rp, cols, vals, np.ones(len(rp) - 1))
+    L64, rep = po.ilu0_factor(rp, cols, vals)
+    L32, _ = po.ilu0_factor(rp, cols, vals.astype(np.float32))
+    assert (rep > 0) == (len(zero) > 0)
+    ctx.ilu0_factor(rmx.F64)
+    np.testing.assert_allclose(ctx.factors(rmx.F64), L64, rtol=1e-12, atol=1e-14)
+    ctx.convert(rmx.F32)
+    for _ in range(2):                       # the second pass meets flags of the first
+        ctx.ilu0_factor(rmx.F32)
+        np.testing.assert_array_equal(ctx.factors(rmx.F32), L32)
