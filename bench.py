@@ -289,7 +289,7 @@ KERNEL_NAMES = {"ilu_factor": "k_ilu_flow (dataflow ILU(0) factorisation, FP32)"
                 "sweep_upper": "k_sweep_stage upper (strip ILU(0) + coarse prolongation)",
                 "spmv": "k_spmv_grp (FP32 row-group SpMV)",
                 "coarse": "coarse correction (restrict, block cyclic reduction, A P residual)",
-                "gram_schmidt": "k_mdot32 + k_gs_update32 (FP32 basis)",
+                "gram_schmidt": "k_gs_dots + k_gs_update (FP32 basis)",
                 "resid_fp64": "k_spmv<double> (FP64 refinement residual)",
                 "sweeps_block": "k_block_sweep (strip ILU(0), both triangles, one wave per block, "
                                 "+ coarse prolongation)"}

@@ -1071,31 +1071,59 @@ void coarse_factor(Ctx& c, int prec)
   C.fac_prec = prec;
 }
 
+// bytes: restriction (row lists, r), coarse solve (its matrices), A P residual (A P entries and
+// aggregates, r, t)
+static int coarse_bytes(Ctx& c)
+{
+  const Coarse& C = c.coarse;
+  const double n = c.n, mats = C.dense ? (double)C.nc * C.nc : (double)C.mats_n;
+  return kt_begin(c, KT_COARSE, 4.0 * (C.nc + 1) + 12.0 * n + 8.0 * C.nc +
+                                    (C.cr_fac ? 8.0 * mats : 0.0) + 12.0 * (double)C.nap +
+                                    4.0 * (n + 1) + 16.0 * n);
+}
+
+// The coarse part of an apply, the coarse correction zc and t = r - A P zc, without a wait of
+// the host; false: nothing done (the host solves the coarse system).
+bool coarse_begin(Ctx& c, int prec, const double* r)
+{
+  Coarse& C = c.coarse;
+  if (!C.cr_fac || !C.fac || C.fac_prec != prec) return false;
+  const int n = c.n, g = (n + 255) / 256;
+  const int kt = coarse_bytes(c);
+  k_restrict<<<(C.nc * 64 + 255) / 256, 256, 0, c.stream>>>(C.nc, C.agg_ptr.p, C.agg_rows.p, r, C.rc.p);
+  cr_apply(c, C);
+  C.applied = !C.dense;
+  k_ap_resid<<<g, 256, 0, c.stream>>>(n, C.ap_ptr.p, C.ap_agg.p, C.apv.p, C.zc.p, r, C.t.p);
+  kt_end(c, kt);
+  HIPCHECK(hipGetLastError());
+  return true;
+}
+
+// z = P zc + M^-1 t, after coarse_begin.
+void coarse_finish(Ctx& c, int prec, double* z)
+{
+  Coarse& C = c.coarse;
+  if (!ilu_apply(c, c.silu, prec, C.t.p, z, nullptr, C.agg.p, C.zc.p))
+    k_add_prolong<<<(c.n + 255) / 256, 256, 0, c.stream>>>(c.n, C.agg.p, C.zc.p, z);
+  HIPCHECK(hipGetLastError());
+}
+
 void coarse_apply(Ctx& c, int prec, const double* r, double* z)
 {
   Coarse& C = c.coarse;
   if (!C.fac || C.fac_prec != prec) fail(RMX_ERR_ARG, "coarse space not factored in this precision");
-  const int n = c.n, g = (n + 255) / 256;
-  // bytes: restriction (row lists, r), coarse solve (its matrices), A P residual (A P
-  // entries and aggregates, r, t)
-  const int kt = kt_begin(c, KT_COARSE, 4.0 * (C.nc + 1) + 12.0 * n + 8.0 * C.nc +
-                                        (C.cr_fac ? 8.0 * (C.dense ? (double)C.nc * C.nc : (double)C.mats_n) : 0.0) +
-                                        12.0 * (double)C.nap + 4.0 * (n + 1) + 16.0 * n);
-  k_restrict<<<(C.nc * 64 + 255) / 256, 256, 0, c.stream>>>(C.nc, C.agg_ptr.p, C.agg_rows.p, r, C.rc.p);
-  if (C.cr_fac) {
-    cr_apply(c, C);
-    C.applied = !C.dense;
-  } else {
+  if (!coarse_begin(c, prec, r)) {
+    const int n = c.n, g = (n + 255) / 256;
+    const int kt = coarse_bytes(c);
+    k_restrict<<<(C.nc * 64 + 255) / 256, 256, 0, c.stream>>>(C.nc, C.agg_ptr.p, C.agg_rows.p, r, C.rc.p);
     HIPCHECK(hipMemcpyAsync(C.h_buf, C.rc.p, sizeof(double) * C.nc, hipMemcpyDeviceToHost, c.stream));
     HIPCHECK(hipStreamSynchronize(c.stream));
     band_solve(C.nc, C.kl, C.ku, C.band, C.ipiv, C.h_buf);
     HIPCHECK(hipMemcpyAsync(C.zc.p, C.h_buf, sizeof(double) * C.nc, hipMemcpyHostToDevice, c.stream));
+    k_ap_resid<<<g, 256, 0, c.stream>>>(n, C.ap_ptr.p, C.ap_agg.p, C.apv.p, C.zc.p, r, C.t.p);
+    kt_end(c, kt);
   }
-  k_ap_resid<<<g, 256, 0, c.stream>>>(n, C.ap_ptr.p, C.ap_agg.p, C.apv.p, C.zc.p, r, C.t.p);
-  kt_end(c, kt);
-  if (!ilu_apply(c, c.silu, prec, C.t.p, z, nullptr, C.agg.p, C.zc.p))
-    k_add_prolong<<<g, 256, 0, c.stream>>>(n, C.agg.p, C.zc.p, z);
-  HIPCHECK(hipGetLastError());
+  coarse_finish(c, prec, z);
 }
 
 }  // namespace rmx

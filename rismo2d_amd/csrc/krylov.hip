@@ -16,6 +16,8 @@
 namespace rmx {
 
 
+constexpr int HOST_TAG = 63;      // word of the pinned mirror that a kernel's results end with
+
 enum { S_RHO = 0, S_RV = 2, S_TS = 3, S_TT = 4, S_RR = 5, S_B2 = 6 };
 
 __global__ void k_copy3(long long n, const double* __restrict__ b, double* __restrict__ r,
@@ -84,29 +86,14 @@ __global__ void k_axpy(long long n, double a, const double* __restrict__ x, doub
     y[i] += a * x[i];
 }
 
-// x *= 1 / sqrt(sc[slot]) (scale from the device), or x *= a when sc is null; with x32 the
-// scaled vector is also stored in FP32 (the Gram-Schmidt copy of the basis)
-__global__ void k_scal_dev(long long n, const double* __restrict__ sc, int slot, double a,
-                           double* __restrict__ x, float* __restrict__ x32)
+// x *= a; with x32 the scaled vector is also stored in FP32 (the Gram-Schmidt copy of the basis)
+__global__ void k_scal(long long n, double a, double* __restrict__ x, float* __restrict__ x32)
 {
-  const double t = sc ? 1.0 / sqrt(sc[slot]) : a;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
-    const double v = x[i] * t;
+    const double v = x[i] * a;
     x[i] = v;
     if (x32) x32[i] = (float)v;
-  }
-}
-
-// y -= sum_j h[j] * V[j]   (classical Gram-Schmidt update, h on the device)
-__global__ void k_gs_update(long long n, int K, const double* __restrict__ h,
-                            const double* __restrict__ Vb, long long ld, double* __restrict__ y)
-{
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    double v = y[i];
-    for (int j = 0; j < K; j++) v += (-h[j]) * Vb[j * ld + i];
-    y[i] = v;
   }
 }
 
@@ -122,134 +109,198 @@ __global__ void k_comb(long long n, int K, const double* __restrict__ rs,
   }
 }
 
-constexpr int RED_BLOCKS = 512;
+// ---- classical Gram-Schmidt ----
+//
+// Three launches an iteration: the dots of the new vector y with the basis (k_gs_dots), the
+// update and its norm (k_gs_update), the normalisation (k_gs_scale).  A launch that ends a sum
+// would take 4.4 us of its own, so each workgroup of the next kernel sums the partial sums by
+// itself, in one order; GS_BLOCKS bounds what that reads (128 KB of K = 32, 512 workgroups).
+// Four entries a thread (16-byte loads of the FP32 basis: rows padded with zeros to ld, a
+// multiple of 4; of an FP64 basis the entries of a row), four basis vectors' loads together.
+// With some 8 vectors, 36,000 unknowns: 13.7 us, 33 in six launches of a fixed 2,048 workgroups;
+// 1.8 million: 46 us, 63 then.
 
-__device__ __forceinline__ double bsum(double v, double* sh)
-{
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  if (l == 0) sh[w] = v;
-  __syncthreads();
-  double s = 0.0;
-  if (threadIdx.x == 0)
-    for (int i = 0; i < (int)(blockDim.x >> 6); i++) s += sh[i];
-  __syncthreads();
-  return s;
-}
-
-// partial[j*MDOT_BLOCKS + block] = <V[j], y> for j < K <= 32: y read once, K accumulators
-// per thread; enough workgroups for eight waves per SIMD
 constexpr int MDOT_MAX = 32;
-constexpr int MDOT_BLOCKS = 2048;
-__global__ void __launch_bounds__(256) k_mdot(long long n, int K, const double* __restrict__ Vb,
-                                              long long ld, const double* __restrict__ y,
-                                              double* __restrict__ partial)
+constexpr int GS_BLOCKS = 512;
+constexpr int GS_THREADS = 256;
+
+__device__ __forceinline__ void ld4(const float* __restrict__ p, long long i, long long, double* v)
 {
-  __shared__ double sh[4];
-  double acc[MDOT_MAX];
+  const float4 w = *reinterpret_cast<const float4*>(p + i);
+  v[0] = w.x; v[1] = w.y; v[2] = w.z; v[3] = w.w;
+}
+__device__ __forceinline__ void ld4(const double* __restrict__ p, long long i, long long n, double* v)
+{
 #pragma unroll
-  for (int j = 0; j < MDOT_MAX; j++) acc[j] = 0.0;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const double yi = y[i];
+  for (int e = 0; e < 4; e++) v[e] = i + e < n ? p[i + e] : 0.0;
+}
+
+// Sums of KP values a lane over the wave: a step halves the values and the lanes that hold one
+// sum, so a sum of 32 values takes 32 exchanges, not 192.  Lane (j's bits reversed into the top
+// lane bits) holds the sum of value j = sum_of(lane).
+template <int KP>
+__device__ __forceinline__ int sum_of(int lane)
+{
+  int j = 0;
+  for (int h = KP / 2, o = 32; h > 0; h >>= 1, o >>= 1)
+    if (lane & o) j += h;
+  return j;
+}
+template <int H, int O>
+__device__ __forceinline__ double wave_sums(double* acc)
+{
+  if constexpr (H > 0) {
+    const bool up = threadIdx.x & O;
 #pragma unroll
-    for (int j = 0; j < MDOT_MAX; j++)
-      if (j < K) acc[j] += Vb[j * ld + i] * yi;
-  }
-#pragma unroll
-  for (int j = 0; j < MDOT_MAX; j++) {
-    if (j < K) {
-      const double s = bsum(acc[j], sh);
-      if (threadIdx.x == 0) partial[j * MDOT_BLOCKS + blockIdx.x] = s;
+    for (int j = 0; j < H; j++) {
+      const double keep = up ? acc[j + H] : acc[j];
+      const double send = up ? acc[j] : acc[j + H];
+      acc[j] = keep + __shfl_xor(send, O, 64);
     }
+    return wave_sums<H / 2, O / 2>(acc);
+  } else if constexpr (O > 0) {
+    acc[0] += __shfl_xor(acc[0], O, 64);
+    return wave_sums<0, O / 2>(acc);
+  } else {
+    return acc[0];
   }
 }
 
-// FP32 basis (leading dimension ld a multiple of 4, zero padding past n): four entries per
-// thread with 16-byte loads.  k_mdot32: partial[j*MDOT_BLOCKS + block] = <V[j], y>;
-// k_gs_update32: y -= sum_j h[j] V[j] and partial[block] = the block's part of <y, y> (the
-// norm of the updated vector in the same pass).  Both run on exactly MDOT_BLOCKS workgroups.
-__global__ void __launch_bounds__(256) k_mdot32(long long n, int K, const float* __restrict__ Vb,
-                                                long long ld, const double* __restrict__ y,
-                                                double* __restrict__ partial)
+// partial[block * MDOT_MAX + j] = the block's part of <V[j], y>, j < K <= KP
+template <class VT, int KP>
+__global__ void __launch_bounds__(GS_THREADS) k_gs_dots(long long n, int K,
+                                                        const VT* __restrict__ Vb, long long ld,
+                                                        const double* __restrict__ y,
+                                                        double* __restrict__ partial)
 {
-  __shared__ double sh[4];
-  double acc[MDOT_MAX];
+  __shared__ double sh[GS_THREADS / 64][KP];
+  double acc[KP];
 #pragma unroll
-  for (int j = 0; j < MDOT_MAX; j++) acc[j] = 0.0;
+  for (int j = 0; j < KP; j++) acc[j] = 0.0;
   const long long nq = (n + 3) / 4;
-  for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < nq;
-       q += (long long)gridDim.x * blockDim.x) {
+  for (long long q = (long long)blockIdx.x * GS_THREADS + threadIdx.x; q < nq;
+       q += (long long)gridDim.x * GS_THREADS) {
     const long long i = 4 * q;
-    const double y0 = y[i];
-    const double y1 = i + 1 < n ? y[i + 1] : 0.0;
-    const double y2 = i + 2 < n ? y[i + 2] : 0.0;
-    const double y3 = i + 3 < n ? y[i + 3] : 0.0;
+    double ye[4];
+    ld4(y, i, n, ye);
 #pragma unroll
-    for (int j = 0; j < MDOT_MAX; j++)
-      if (j < K) {
-        const float4 v = *reinterpret_cast<const float4*>(Vb + j * ld + i);
-        acc[j] += (double)v.x * y0 + (double)v.y * y1 + (double)v.z * y2 + (double)v.w * y3;
+    for (int j0 = 0; j0 < KP; j0 += 4)
+      if (j0 < K) {
+        double v[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) ld4(Vb + min(j0 + j, K - 1) * ld, i, n, v[j]);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[j0 + j] += v[j][e] * ye[e];
       }
   }
-#pragma unroll
-  for (int j = 0; j < MDOT_MAX; j++) {
-    if (j < K) {
-      const double s = bsum(acc[j], sh);
-      if (threadIdx.x == 0) partial[j * MDOT_BLOCKS + blockIdx.x] = s;
-    }
+  const int lane = threadIdx.x & 63;
+  const double s = wave_sums<KP / 2, 32>(acc);
+  if ((lane & (64 / KP - 1)) == 0) sh[threadIdx.x >> 6][sum_of<KP>(lane)] = s;
+  __syncthreads();
+  if (threadIdx.x < KP) {
+    double v = 0.0;
+    for (int w = 0; w < GS_THREADS / 64; w++) v += sh[w][threadIdx.x];
+    partial[blockIdx.x * MDOT_MAX + threadIdx.x] = v;
   }
 }
 
-__global__ void __launch_bounds__(256) k_gs_update32(long long n, int K, const double* __restrict__ h,
-                                                     const float* __restrict__ Vb, long long ld,
-                                                     double* __restrict__ y,
-                                                     double* __restrict__ partial)
+// y -= sum_j h[j] V[j], h from the partial sums of k_gs_dots (also stored, by block 0);
+// nrm[block] = the block's part of <y, y>
+template <class VT>
+__global__ void __launch_bounds__(GS_THREADS) k_gs_update(long long n, int K, int parts,
+                                                          const double* __restrict__ partial,
+                                                          const VT* __restrict__ Vb, long long ld,
+                                                          double* __restrict__ y,
+                                                          double* __restrict__ h,
+                                                          double* __restrict__ nrm)
 {
-  __shared__ double sh[4];
-  double hr[MDOT_MAX];
-#pragma unroll
-  for (int j = 0; j < MDOT_MAX; j++) hr[j] = j < K ? -h[j] : 0.0;
+  constexpr int S = GS_THREADS / MDOT_MAX;
+  __shared__ double sh[S][MDOT_MAX], hs[MDOT_MAX];
+  {
+    const int j = threadIdx.x % MDOT_MAX, s = threadIdx.x / MDOT_MAX;
+    double v = 0.0;
+    if (j < K) {
+#pragma unroll 8
+      for (int b = s; b < parts; b += S) v += partial[b * MDOT_MAX + j];
+    }
+    sh[s][j] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < MDOT_MAX) {
+    double v = 0.0;
+    for (int s = 0; s < S; s++) v += sh[s][threadIdx.x];
+    hs[threadIdx.x] = threadIdx.x < K ? -v : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x < K) h[threadIdx.x] = v;
+  }
+  __syncthreads();
   double ss = 0.0;
   const long long nq = (n + 3) / 4;
-  for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < nq;
-       q += (long long)gridDim.x * blockDim.x) {
+  for (long long q = (long long)blockIdx.x * GS_THREADS + threadIdx.x; q < nq;
+       q += (long long)gridDim.x * GS_THREADS) {
     const long long i = 4 * q;
-    double v0 = y[i];
-    double v1 = i + 1 < n ? y[i + 1] : 0.0;
-    double v2 = i + 2 < n ? y[i + 2] : 0.0;
-    double v3 = i + 3 < n ? y[i + 3] : 0.0;
+    double ye[4];
+    ld4(y, i, n, ye);
+    for (int j0 = 0; j0 < K; j0 += 4) {
+      double v[4][4];
 #pragma unroll
-    for (int j = 0; j < MDOT_MAX; j++)
-      if (j < K) {
-        const float4 w = *reinterpret_cast<const float4*>(Vb + j * ld + i);
-        v0 += hr[j] * (double)w.x;
-        v1 += hr[j] * (double)w.y;
-        v2 += hr[j] * (double)w.z;
-        v3 += hr[j] * (double)w.w;
+      for (int j = 0; j < 4; j++) ld4(Vb + min(j0 + j, K - 1) * ld, i, n, v[j]);
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) ye[e] += hs[j0 + j] * v[j][e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (i + e < n) {
+        y[i + e] = ye[e];
+        ss += ye[e] * ye[e];
       }
-    if (i + 1 >= n) v1 = 0.0;         // past the end: padding of V, not part of y
-    if (i + 2 >= n) v2 = 0.0;
-    if (i + 3 >= n) v3 = 0.0;
-    y[i] = v0;
-    if (i + 1 < n) y[i + 1] = v1;
-    if (i + 2 < n) y[i + 2] = v2;
-    if (i + 3 < n) y[i + 3] = v3;
-    ss += v0 * v0 + v1 * v1 + v2 * v2 + v3 * v3;
   }
-  const double s = bsum(ss, sh);
-  if (threadIdx.x == 0) partial[blockIdx.x] = s;
+  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) hs[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double v = 0.0;
+    for (int w = 0; w < GS_THREADS / 64; w++) v += hs[w];
+    nrm[blockIdx.x] = v;
+  }
 }
 
-// out[k] = sum of the MDOT_BLOCKS partials of dot k; one workgroup per dot
-__global__ void k_mfinish(const double* __restrict__ partial, double* __restrict__ out)
+// y /= ||y|| (as it is below `tiny`), ||y||^2 from the partial sums; y32: the FP32 copy.
+// Block 0 hands ||y||^2, h and the tag to the host (host[0], host[1 ..], host[tag]).
+__global__ void __launch_bounds__(GS_THREADS) k_gs_scale(long long n, int K, int parts, double tiny,
+                                                         const double* __restrict__ nrm,
+                                                         const double* __restrict__ h,
+                                                         double* __restrict__ y,
+                                                         float* __restrict__ y32, double* host,
+                                                         unsigned long long tag)
 {
-  __shared__ double sh[4];
-  const int k = blockIdx.x;
-  double v = 0.0;
-  for (int i = threadIdx.x; i < MDOT_BLOCKS; i += blockDim.x) v += partial[k * MDOT_BLOCKS + i];
-  const double s = bsum(v, sh);
-  if (threadIdx.x == 0) out[k] = s;
+  __shared__ double sh[GS_THREADS / 64];
+  double s = 0.0;
+  for (int b = threadIdx.x; b < parts; b += GS_THREADS) s += nrm[b];
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  s = 0.0;
+  for (int w = 0; w < GS_THREADS / 64; w++) s += sh[w];
+  if (blockIdx.x == 0 && threadIdx.x < 64) {
+    if (threadIdx.x == 0) host[0] = s;
+    if (threadIdx.x < K) host[1 + threadIdx.x] = h[threadIdx.x];
+    __threadfence_system();
+    if (threadIdx.x == 0)
+      __hip_atomic_store(reinterpret_cast<unsigned long long*>(host) + HOST_TAG, tag,
+                         __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  const double t = fabs(sqrt(s)) > tiny ? 1.0 / sqrt(s) : 1.0;
+  for (long long i = (long long)blockIdx.x * GS_THREADS + threadIdx.x; i < n;
+       i += (long long)gridDim.x * GS_THREADS) {
+    const double v = y[i] * t;
+    y[i] = v;
+    if (y32) y32[i] = (float)v;
+  }
 }
 
 static int vblocks(long long n) { return (int)std::min<long long>(4096, (n + 255) / 256); }
@@ -277,8 +328,30 @@ static void precond(Ctx& c, int prec, int kind, const double* in, double* out)
 void ensure_work(Ctx& c)
 {
   for (int k = 0; k < 10; k++) c.w[k].alloc(c.n);
-  c.red.alloc(64 + 40 * MDOT_BLOCKS);
-  if (!c.h_red) HIPCHECK(hipHostMalloc(&c.h_red, 64 * sizeof(double), hipHostMallocDefault));
+  c.red.alloc(64 + 81920);
+  if (!c.h_red) {
+    HIPCHECK(hipHostMalloc(&c.h_red, 64 * sizeof(double), hipHostMallocDefault));
+    std::fill(c.h_red, c.h_red + 64, 0.0);
+    c.h_tag = 0;
+  }
+}
+
+// Until a kernel of the stream has written `tag` to the pinned mirror (the work queued after it
+// goes on meanwhile); the stream is asked now and then, so that a failed launch ends the wait.
+static void await_tag(Ctx& c, unsigned long long tag)
+{
+  const unsigned long long* word = reinterpret_cast<const unsigned long long*>(c.h_red) + HOST_TAG;
+  for (unsigned polls = 1;; polls++) {
+    if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == tag) return;
+    __builtin_ia32_pause();
+    if (polls % 65536 == 0) {
+      const hipError_t e = hipStreamQuery(c.stream);
+      if (e == hipErrorNotReady) continue;
+      HIPCHECK(e);
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == tag) return;
+      fail(RMX_ERR_HIP, "solve: the Gram-Schmidt sums did not reach the host");
+    }
+  }
 }
 
 static double fetch(Ctx& c, const double* dev, int k = 1)
@@ -366,6 +439,26 @@ static bool bicgstab(Ctx& c, int prec, int pk, const double* b, double* x, int m
   return conv;
 }
 
+// Workgroups of the Gram-Schmidt kernels: as many as have work in every round.
+static int gs_blocks(long long n)
+{
+  const long long nb = ((n + 3) / 4 + GS_THREADS - 1) / GS_THREADS;
+  const long long rounds = (nb + GS_BLOCKS - 1) / GS_BLOCKS;
+  return (int)std::max(1LL, (nb + rounds - 1) / rounds);
+}
+
+// h = V^T y, y -= V h for K basis vectors; h to red + 16, the parts of ||y||^2 after the dots'
+template <class VT>
+static void gram_schmidt(Ctx& c, int K, int gb, const VT* V, long long ld, double* y)
+{
+  double* partial = c.red.p + 64;
+  if (K <= 8) k_gs_dots<VT, 8><<<gb, GS_THREADS, 0, c.stream>>>(c.n, K, V, ld, y, partial);
+  else if (K <= 16) k_gs_dots<VT, 16><<<gb, GS_THREADS, 0, c.stream>>>(c.n, K, V, ld, y, partial);
+  else k_gs_dots<VT, 32><<<gb, GS_THREADS, 0, c.stream>>>(c.n, K, V, ld, y, partial);
+  k_gs_update<VT><<<gb, GS_THREADS, 0, c.stream>>>(c.n, K, gb, partial, V, ld, y, c.red.p + 16,
+                                                   partial + GS_BLOCKS * MDOT_MAX);
+}
+
 // Flexible GMRES(m) on A(prec) x = b, x0 = 0.  In an FP32 solve the Gram-Schmidt dots and
 // updates read an FP32 copy of the basis (written by the normalisation, half the bytes);
 // the preconditioner input, the new vector and the solution update stay FP64.
@@ -389,8 +482,8 @@ static bool fgmres(Ctx& c, int prec, int pk, const double* b, double* x, int m, 
   float* V32 = b32 ? c.V32_basis.p : nullptr;
   double* Zb = c.Z_basis.p;
   double* sc = c.red.p;
-  double* partial = c.red.p + 64;
-  const int vb = vblocks(n);
+  double* nrm = c.red.p + 64 + GS_BLOCKS * MDOT_MAX;
+  const int vb = vblocks(n), gb = gs_blocks(n);
   HIPCHECK(hipMemsetAsync(x, 0, sizeof(double) * n, c.stream));
   std::vector<std::vector<double>> hh(m, std::vector<double>(m + 1, 0.0));
   std::vector<double> cs(m + 1), sn(m + 1), rs(m + 1);
@@ -410,11 +503,12 @@ static bool fgmres(Ctx& c, int prec, int pk, const double* b, double* x, int m, 
     }
     ro = std::sqrt(fetch(c, sc + S_B2));
     if (std::fabs(ro) <= EPSILON) { conv = true; break; }
-    k_scal_dev<<<vb, 256, 0, c.stream>>>(n, nullptr, 0, 1.0 / ro, Vb, V32);
+    k_scal<<<vb, 256, 0, c.stream>>>(n, 1.0 / ro, Vb, V32);
     if (iters == 0) { resid = ro; eps1 = eps * ro; }
     const double ro_cycle = ro;
     rs[0] = ro;
     int i = -1;
+    bool begun = false;
     while (true) {
       i++;
       iters++;
@@ -422,32 +516,25 @@ static bool fgmres(Ctx& c, int prec, int pk, const double* b, double* x, int m, 
       double* vi = Vb + (size_t)i * n;
       double* vi1 = Vb + (size_t)i1 * n;
       double* zi = Zb + (size_t)i * n;
-      precond(c, prec, pk, vi, zi);
+      if (begun) coarse_finish(c, prec, zi);
+      else precond(c, prec, pk, vi, zi);
       dev_spmv(c, prec, zi, vi1);
       // classical Gram-Schmidt: all dots, then all updates
       const int kt = kt_begin(c, KT_GS, b32 ? 8.0 * i1 * ld32 + 24.0 * n : 16.0 * i1 * n + 40.0 * n);
-      if (b32) {
-        k_mdot32<<<MDOT_BLOCKS, 256, 0, c.stream>>>(n, i1, V32, ld32, vi1, partial);
-        k_mfinish<<<i1, 256, 0, c.stream>>>(partial, sc + 16);
-        k_gs_update32<<<MDOT_BLOCKS, 256, 0, c.stream>>>(n, i1, sc + 16, V32, ld32, vi1, partial);
-        k_mfinish<<<1, 256, 0, c.stream>>>(partial, sc + S_B2);
-      } else {
-        k_mdot<<<MDOT_BLOCKS, 256, 0, c.stream>>>(n, i1, Vb, n, vi1, partial);
-        k_mfinish<<<i1, 256, 0, c.stream>>>(partial, sc + 16);
-        k_gs_update<<<vb, 256, 0, c.stream>>>(n, i1, sc + 16, Vb, n, vi1);
-        const double* xs[1] = { vi1 };
-        dev_dots(c, 1, xs, xs, sc + S_B2);
-      }
+      if (b32) gram_schmidt(c, i1, gb, V32, ld32, vi1);
+      else gram_schmidt(c, i1, gb, Vb, n, vi1);
       kt_end(c, kt);
-      HIPCHECK(hipMemcpyAsync(c.h_red, sc, sizeof(double) * (16 + i1), hipMemcpyDeviceToHost, c.stream));
-      HIPCHECK(hipStreamSynchronize(c.stream));
-      for (int j = 0; j <= i; j++) hh[i][j] = c.h_red[16 + j];
-      double tn = std::sqrt(c.h_red[S_B2]);
+      const unsigned long long tag = ++c.h_tag;
+      k_gs_scale<<<vb, GS_THREADS, 0, c.stream>>>(n, i1, gb, EPSILON, nrm, sc + 16, vi1,
+                                                  V32 ? V32 + i1 * ld32 : nullptr, c.h_red, tag);
+      HIPCHECK(hipGetLastError());
+      // the coarse part of the next preconditioning runs while the host reads the sums and
+      // decides (17 us an iteration otherwise); wasted once, where the solve ends here
+      begun = i1 < m && iters < maxIter && pk == RMX_PREC_SILU0C && coarse_begin(c, prec, vi1);
+      await_tag(c, tag);
+      for (int j = 0; j <= i; j++) hh[i][j] = c.h_red[1 + j];
+      double tn = std::sqrt(c.h_red[0]);
       hh[i][i1] = tn;
-      if (std::fabs(tn) > EPSILON)
-        k_scal_dev<<<vb, 256, 0, c.stream>>>(n, sc, S_B2, 1.0, vi1, V32 ? V32 + i1 * ld32 : nullptr);
-      else if (V32)      // no scaling (breakdown): the FP32 copy of the vector as it is
-        k_scal_dev<<<vb, 256, 0, c.stream>>>(n, nullptr, 0, 1.0, vi1, V32 + i1 * ld32);
       for (int k = 1; k <= i; k++) {
         const int k1 = k - 1;
         const double tt = hh[i][k1];

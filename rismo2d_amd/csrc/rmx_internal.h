@@ -391,6 +391,7 @@ struct Ctx {
   DBuf<double> w[10];
   DBuf<double> red;                           // reduction scratch
   double* h_red = nullptr;                    // pinned host mirror of red
+  unsigned long long h_tag = 0;               // last results handed over in it by a kernel
   // FGMRES basis
   DBuf<double> V_basis, Z_basis;
   DBuf<float> V32_basis;                      // FP32 copy for the Gram-Schmidt of FP32 solves
@@ -459,6 +460,8 @@ void coarse_setup(Ctx& c, const std::vector<int>& rp, const std::vector<int>& cl
                   const std::vector<int>& group, int nseg);
 int coarse_segments_of(const Ctx& c);          // coarse segments per strip in effect
 void coarse_factor(Ctx& c, int prec);
+bool coarse_begin(Ctx& c, int prec, const double* r);
+void coarse_finish(Ctx& c, int prec, double* z);
 void coarse_apply(Ctx& c, int prec, const double* r, double* z);   // device pointers
 void coarse_check(Ctx& c);                     // fails if a coarse solve gave up a wait
 void dev_precond(Ctx& c, int prec, int kind, const double* in, double* out);

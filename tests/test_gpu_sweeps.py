@@ -224,3 +224,37 @@ def test_factorisation_by_units(ctx, n, width, stride, run, zero):
     for _ in range(2):                       # the second pass meets flags of the first
         ctx.ilu0_factor(rmx.F32)
         np.testing.assert_array_equal(ctx.factors(rmx.F32), L32)
+
+
+# the Gram-Schmidt kernels: sizes around a quad of entries and a workgroup's 1,024, one and two
+# rounds of 512 workgroups, up to 8, 16 and 30 vectors.  A's diagonal exceeds its row's sum by 1,
+# so |A^-1| <= 1 and the error is at most the residual, eps |b|; twice that for rounding.
+@pytest.mark.parametrize("n,mkyrl", [(1, 3), (2, 5), (3, 7), (4, 7), (5, 15), (1023, 15), (1024, 30),
+                                     (1025, 30), (2050, 15), (4099, 30), (60001, 15), (524287, 15),
+                                     (524289, 30)])
+def test_fgmres_on_ragged_sizes(ctx, n, mkyrl):
+    import scipy.sparse as sp
+    from scipy.sparse.linalg import splu
+    print(f"[gpu] FGMRES({mkyrl}), {n} equations", flush=True)
+    rng = np.random.default_rng(41)
+    offs = [o for o in (1, 4, 9) if o < n]
+    diags = [rng.standard_normal(n - o) for o in offs] + [rng.standard_normal(n - o) for o in offs]
+    M = sp.diags(diags, offs + [-o for o in offs], shape=(n, n), format="csr") if offs else \
+        sp.csr_matrix((n, n))
+    d = np.asarray(abs(M).sum(axis=1)).ravel() + 1.0
+    rows, cols, vals = sp.find(M)
+    rows, cols = np.concatenate([np.arange(n), rows]), np.concatenate([np.arange(n), cols])
+    vals = np.concatenate([d, vals])
+    o = np.lexsort((cols, cols != rows, rows))           # the diagonal first in its row
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    cols, vals = cols[o].astype(np.int32), vals[o]
+    b = rng.standard_normal(n)
+    ctx.csr_upload(rp, cols, vals, b)
+    for prec, dt, eps in ((rmx.F64, np.float64, 1e-10), (rmx.F32, np.float32, 1e-5)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        out = ctx.solve(rmx.FGMRES, prec, rmx.PREC_NONE, max_iter=400, mkyrl=mkyrl, eps=eps)
+        assert out.converged
+        A = sp.csr_matrix((vals.astype(dt).astype(np.float64), cols, rp), shape=(n, n))
+        x = splu(A.tocsc()).solve(b)
+        assert np.abs(ctx.solution() - x).max() <= 2 * eps * np.linalg.norm(b), prec
