@@ -1686,6 +1686,293 @@ __global__ void __launch_bounds__(64 * NS_WAVES) k_node_sweep(const int4* __rest
 // ---------------------------------------------------------------------------------------
 // host set-up
 
+// ---------------------------------------------------------------------------------------
+// sweeps of blocks by chunks of 16 rows
+//
+// A block's triangular solve is a chain, of nodes if taken level by level (80 to 300 levels of
+// some 700 cycles in a block of 700 rows), and what bounds it is the latency of a link, not its
+// bytes.  A wave takes its block in the equations' own order, 16 rows at a time, with the
+// inverse of the 16 x 16 triangle (k_chunk_inv, FP64, once per factorisation): a link is then
+// the sparse sums over earlier chunks and one small product for 16 rows, 44 links a block.
+// Lane 4 c + q works a quarter of row c's sum (columns as LDS byte offsets, two a packet and
+// lane), then column c of the product for rows q, q + 4, q + 8, q + 12; the four are summed over
+// the columns by two half-wave exchanges that also part the rows and two rotations, without a
+// trip through LDS.  Packets and the inverse are loaded some chunks ahead, always the same number
+// of loads (past a chunk's packets the next one's), so that the compiler's waits name the right
+// ones.  Of the inverse the upper 4 x 4 blocks are not stored: plane j holds rows 4 j .. 4 j + 3,
+// columns up to 4 j + 3.
+// FP32, FP64 factors, both directions: 36 us at 5,600 rows (60 x 13 quads), 37 at 36,000, 42 at
+// 231,000, 72, 88 at 923,000, 142, 169 at 1.8 million (3 TB/s); node by node 63, 43, 209, 251,
+// 241 us (FP32).  A link takes 0.24 us: some 280 cycles of dependent FP64 operations, an LDS
+// write and read, the issue of the rest.  Matrix instructions for the row sums and the product
+// are not faster (0.27 us: a dependent 4x4x4 FP64 one takes 50 cycles, an addition 28); more
+// chunks ahead change nothing; chunks of 32 rows would take 1.6 times the bytes.
+
+constexpr int CH_ROWS = 16;       // rows of a chunk
+constexpr int CH_T = 160;         // stored entries of a chunk's inverse
+constexpr int CH_MAX = 128;       // chunks of a block
+constexpr int CH_DEEP2 = 4, CH_DEEP = 3;
+constexpr int CH_PK = 4;          // most packets of a chunk that are loaded ahead
+
+__device__ __forceinline__ double2 swap32(double a, double b)
+{
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a),
+                                                   (unsigned)__double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a),
+                                                   (unsigned)__double2hiint(b), false, false);
+  const unsigned l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+  return make_double2(__hiloint2double((int)h0, (int)l0), __hiloint2double((int)h1, (int)l1));
+}
+__device__ __forceinline__ double2 swap16(double a, double b)
+{
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a),
+                                                   (unsigned)__double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a),
+                                                   (unsigned)__double2hiint(b), false, false);
+  const unsigned l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+  return make_double2(__hiloint2double((int)h0, (int)l0), __hiloint2double((int)h1, (int)l1));
+}
+
+template <class VT, int PK> struct ChunkBuf {
+  VT v[PK][2];
+  unsigned id[PK];
+  double t[4], d;
+  int pk;
+};
+
+// One direction: chunks in processing order (UP: from the block's end, rows of a chunk from its
+// end).  cb: the block's first chunk, pb: its first packet; cnt: packets of every chunk.
+template <class VT, int PK, bool UP>
+__device__ __forceinline__ void chunk_sweep(int nch, int cb, int pb,
+                                            const unsigned char* __restrict__ cnt,
+                                            const unsigned* __restrict__ idx,
+                                            const VT* __restrict__ val,
+                                            const double* __restrict__ T,
+                                            const double* __restrict__ D, unsigned spare)
+{
+  using P = typename VQuad<VT>::P;
+  const int lane = threadIdx.x, c = lane >> 2, q = lane & 3;
+  const unsigned cd = (lane < nch ? (unsigned)cnt[cb + lane] : 0u) |
+                      (64 + lane < nch ? (unsigned)cnt[cb + 64 + lane] : 0u) << 16;
+  auto packets = [&](int t) {
+    const unsigned long long d = (unsigned)__builtin_amdgcn_readlane((int)cd, t & 63);
+    return (int)(d >> ((t >> 6) * 16) & 0xFFFF);
+  };
+  const int t0 = min(lane, 15), t1 = 16 + min(lane, 31), t2 = 48 + min(lane, 47), t3 = 96 + lane;
+  const unsigned* ip = idx + (size_t)pb * 64;
+  const P* vp = reinterpret_cast<const P*>(val) + (size_t)pb * 64;
+  const double* tp = T + (size_t)cb * CH_T;
+  const double* dp = UP ? D + (size_t)cb * CH_ROWS + c : nullptr;
+  int pk = 0;
+  auto load = [&](ChunkBuf<VT, PK>& b, int t) {
+#pragma unroll
+    for (int p = 0; p < PK; p++) {
+      b.id[p] = ip[64 * p + lane];
+      const P w = vp[64 * p + lane];
+      b.v[p][0] = w.x; b.v[p][1] = w.y;
+    }
+    b.t[0] = tp[t0]; b.t[1] = tp[t1]; b.t[2] = tp[t2]; b.t[3] = tp[t3];
+    if (UP) { b.d = *dp; dp += CH_ROWS; }
+    b.pk = pk;
+    const int np = packets(t);
+    ip += 64 * np;
+    vp += 64 * np;
+    tp += CH_T;
+    pk += np;
+  };
+  const bool keep = (c & 3) == q;                  // the lane's own row is its row of the product
+  const int r = 4 * (lane >> 4) + q;
+  unsigned own = 8u * (UP ? CH_ROWS * nch - 1 - c : c), to = 8u * (UP ? CH_ROWS * nch - 1 - r : r);
+  // a chunk's reads of LDS; its packets 2 and 3 (the last of 2 or 4 may be another chunk's) are
+  // read where it has more than 2
+  double x[2 * PK], s0;
+  int np;
+  auto fetch = [&](const ChunkBuf<VT, PK>& b, int t) {
+    np = packets(t);
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+      x[2 * p] = ld_lds(b.id[p] & 0xFFFFu);
+      x[2 * p + 1] = ld_lds(b.id[p] >> 16);
+    }
+    if (PK > 2 && np > 2) {
+#pragma unroll
+      for (int p = 2; p < PK; p++) {
+        x[2 * p] = ld_lds(b.id[p] & 0xFFFFu);
+        x[2 * p + 1] = ld_lds(b.id[p] >> 16);
+      }
+    }
+    s0 = ld_lds(own);
+    own += UP ? -8u * CH_ROWS : 8u * CH_ROWS;
+  };
+  auto step = [&](const ChunkBuf<VT, PK>& b) {
+    auto f = [](VT v) { return UP ? -(double)v : (double)v; };
+    double a0 = f(b.v[0][0]) * x[0], a1 = f(b.v[0][1]) * x[1];
+    a0 += f(np > 1 ? b.v[1][0] : (VT)0) * x[2];
+    a1 += f(np > 1 ? b.v[1][1] : (VT)0) * x[3];
+    if (np > 2) {
+      if (PK > 2) {
+#pragma unroll
+        for (int p = 2; p < PK; p++) {
+          a0 += f(p < PK - 1 || np > p ? b.v[p][0] : (VT)0) * x[2 * p];
+          a1 += f(p < PK - 1 || np > p ? b.v[p][1] : (VT)0) * x[2 * p + 1];
+        }
+      }
+      for (int p = PK; p < np; p++) {
+        const size_t at = (size_t)(pb + b.pk + p) * 64 + lane;
+        const unsigned id = idx[at];
+        const P w = reinterpret_cast<const P*>(val)[at];
+        a0 += f(w.x) * ld_lds(id & 0xFFFFu);
+        a1 += f(w.y) * ld_lds(id >> 16);
+      }
+    }
+    a0 += a1;
+    a0 += dpp_get<0xB1>(a0);                       // over the row's four lanes
+    a0 += dpp_get<0x4E>(a0);
+    const double s = s0 + a0;
+    const double p0 = (lane < 16 ? b.t[0] : 0.0) * s, p1 = (lane < 32 ? b.t[1] : 0.0) * s;
+    const double p2 = (lane < 48 ? b.t[2] : 0.0) * s, p3 = b.t[3] * s;
+    const double2 e = swap32(p0, p2), h = swap32(p1, p3);
+    const double2 g = swap16(e.x + e.y, h.x + h.y);
+    double y = g.x + g.y;
+    y += dpp_get<0x128>(y);                        // 8 lanes on
+    const double own_part = UP ? b.d * s + y : s + y;
+    st_lds(keep ? to : spare, own_part + dpp_get<0x124>(y));
+    to += UP ? -8u * CH_ROWS : 8u * CH_ROWS;
+  };
+  constexpr int R = PK == 2 ? CH_DEEP2 : CH_DEEP;
+  ChunkBuf<VT, PK> buf[R];
+#pragma unroll
+  for (int u = 0; u < R; u++) load(buf[u], u);
+  fetch(buf[0], 0);
+  for (int t = 0;; t += R) {
+#pragma unroll
+    for (int u = 0; u < R; u++) {
+      step(buf[u]);
+      if (t + u + 1 >= nch) return;
+      fetch(buf[(u + 1) % R], t + u + 1);
+      asm volatile("" ::: "memory");               // the loads ahead while LDS answers
+      load(buf[u], t + u + R);
+    }
+  }
+}
+
+template <class VT, int PK>
+__global__ void __launch_bounds__(64) k_chunk_sweep(const int4* __restrict__ info,
+                                                    const int* __restrict__ rows,
+                                                    const unsigned char* __restrict__ dlo,
+                                                    const unsigned* __restrict__ ilo,
+                                                    const VT* __restrict__ vlo,
+                                                    const double* __restrict__ tlo,
+                                                    const unsigned char* __restrict__ dup,
+                                                    const unsigned* __restrict__ iup,
+                                                    const VT* __restrict__ vup,
+                                                    const double* __restrict__ tup,
+                                                    const double* __restrict__ dgu,
+                                                    const double* __restrict__ b,
+                                                    double* __restrict__ x,
+                                                    const int* __restrict__ aidx,
+                                                    const double* __restrict__ aval)
+{
+  constexpr int U = 16;                            // rows a lane in flight
+  const int lane = threadIdx.x;
+  const int4 w0 = info[2 * blockIdx.x], w1 = info[2 * blockIdx.x + 1];
+  const int m = w0.y, nch = (m + CH_ROWS - 1) / CH_ROWS, all = nch * CH_ROWS;
+  const int* row = rows + w0.x;
+  for (int k0 = 0; k0 < all; k0 += 64 * U) {
+    int i[U];
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) i[u] = row[min(k0 + 64 * u + lane, m - 1)];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = b[i[u]];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = k0 + 64 * u + lane;
+      if (k < all) st_lds(8u * k, k < m ? v[u] : 0.0);
+    }
+  }
+  asm volatile("" ::: "memory");
+  const unsigned spare = 8u * (all + lane);
+  chunk_sweep<VT, PK, false>(nch, w0.z, w1.x, dlo, ilo, vlo, tlo, nullptr, spare);
+  asm volatile("" ::: "memory");
+  chunk_sweep<VT, PK, true>(nch, w0.z, w1.y, dup, iup, vup, tup, dgu, spare);
+  asm volatile("" ::: "memory");
+  for (int k0 = 0; k0 < m; k0 += 64 * U) {
+    int i[U];
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) i[u] = row[min(k0 + 64 * u + lane, m - 1)];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = aidx ? aval[aidx[i[u]]] : 0.0;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = k0 + 64 * u + lane;
+      if (k < m) x[i[u]] = ld_lds(8u * k) + v[u];
+    }
+  }
+}
+
+// Inverses of a chunk's triangles, one wave a chunk.  Both are taken as lower ones in processing
+// order: row r is (e_r + sum of g_rk times row k) / d_r, with g the stored (negated) multipliers
+// and d = 1 below, g = -u and d = u_rr above.  In twice FP64's digits (error-free sums and
+// products), so that the product with the inverse has only the rounding of its entries on top of
+// its own, and with the diagonals kept apart: a row's own term is added last.  The error of an
+// apply against extended precision is then that of a substitution (18 meshes: 1.0 times that of
+// the level sweeps where both are near rounding, 0.6 to 5 times, 1.3 in the mean, where the
+// factors amplify it; two orders of the same substitution differ as much).
+template <class VT>
+__global__ void __launch_bounds__(64) k_chunk_inv(const int4* __restrict__ chunks,
+                                                  const int* __restrict__ rows,
+                                                  const int* __restrict__ slot,
+                                                  const int* __restrict__ rp,
+                                                  const int* __restrict__ cols,
+                                                  const VT* __restrict__ LU,
+                                                  double* __restrict__ tlo, double* __restrict__ tup,
+                                                  double* __restrict__ dgu)
+{
+#pragma clang fp contract(off)
+  __shared__ double G[2][CH_ROWS][CH_ROWS + 1], D[2][CH_ROWS];
+  const int lane = threadIdx.x, h = blockIdx.x;
+  const int4 ch = chunks[h];                       // first row, rows, place in tlo, in tup
+  for (int k = lane; k < 2 * CH_ROWS * (CH_ROWS + 1); k += 64) (&G[0][0][0])[k] = 0.0;
+  if (lane < 2 * CH_ROWS) (&D[0][0])[lane] = 1.0;
+  __syncthreads();
+  const int r = lane >> 2, q = lane & 3;
+  if (r < ch.y) {
+    const int i = rows[ch.x + r], p0 = rp[i], p1 = rp[i + 1];
+    if (q == 0) D[1][CH_ROWS - 1 - r] = (double)LU[p0];
+    for (int e = p0 + 1 + q; e < p1; e += 4) {
+      const int j = cols[e], sl = slot[j];
+      if ((sl >> 4) != h) continue;
+      const int k = sl & (CH_ROWS - 1);
+      if (k < r) G[0][r][k] = (double)LU[e];
+      else G[1][CH_ROWS - 1 - r][CH_ROWS - 1 - k] = -(double)LU[e];
+    }
+  }
+  __syncthreads();
+  if (lane >= 2 * CH_ROWS) return;
+  const int dir = lane >> 4, c = lane & 15;
+  double* T = dir ? tup + (size_t)ch.w * CH_T : tlo + (size_t)ch.z * CH_T;
+  double z[CH_ROWS], zl[CH_ROWS];
+#pragma unroll
+  for (int k = 0; k < CH_ROWS; k++) {
+    double s = k == c ? 1.0 : 0.0, sl = 0.0;
+#pragma unroll
+    for (int l = 0; l < k; l++) {
+      const double g = G[dir][k][l], p = g * z[l], e = fma(g, z[l], -p);
+      const double t = s + p, v = t - s;
+      sl += fma(g, zl[l], e) + ((s - (t - v)) + (p - v));
+      s = t;
+    }
+    const double d = D[dir][k], q = s / d, r = (fma(-q, d, s) + sl) / d;
+    z[k] = q + r;
+    zl[k] = r - (z[k] - q);
+    const int j = k >> 2;
+    if (c < 4 * (j + 1)) T[8 * j * (j + 1) + 4 * c + (k & 3)] = k == c ? 0.0 : z[k];
+    if (dir && k == c) dgu[(size_t)ch.w * CH_ROWS + c] = z[k];
+  }
+}
+
 // RMX_SWEEP selects the sweep kernels (tuning and comparison), read when a system is set up
 // and at every application: 1 the staged level sweeps, 2 (default) the block sweeps where
 // every block has at most BS_ROWS rows, else the node sweeps where the rows alive at a time
@@ -2413,6 +2700,125 @@ std::vector<int> cut_segments(const std::vector<int>& bstart, const std::vector<
   return seg;
 }
 
+// Chunks of every block; off where a block has more than CH_MAX.
+static void build_chunks(Ilu& I, hipStream_t s)
+{
+  ChunkSweep& S = I.cs;
+  S.on = false;
+  const int n = I.n, nseg = std::max(1, I.nseg), nb = I.nblk * nseg;
+  const std::vector<int>& rp = I.h_rp;
+  auto segof = [&](int i) { return I.seg.empty() ? 0 : I.seg[i]; };
+  // rows of every block, ascending
+  std::vector<int> blk(n), start(nb + 1, 0), rows(n), at(n);
+  for (int b = 0; b < I.nblk; b++)
+    for (int i = I.bstart[b]; i < I.bstart[b + 1]; i++) start[(blk[i] = b * nseg + segof(i)) + 1]++;
+  int most = 0;
+  for (int b = 0; b < nb; b++) most = std::max(most, start[b + 1]);
+  if (most > BS_ROWS) return;
+  for (int b = 0; b < nb; b++) start[b + 1] += start[b];
+  {
+    std::vector<int> next(start.begin(), start.end() - 1);
+    for (int i = 0; i < n; i++) { at[i] = next[blk[i]] - start[blk[i]]; rows[next[blk[i]]++] = i; }
+  }
+  std::vector<int> cbase(nb + 1, 0);
+  for (int b = 0; b < nb; b++) cbase[b + 1] = cbase[b] + (start[b + 1] - start[b] + CH_ROWS - 1) / CH_ROWS;
+  const int nch = cbase[nb];
+  std::vector<int> slot(n);
+  std::vector<int4> chunks(nch);
+  std::vector<unsigned char> cdesc[2] = { std::vector<unsigned char>(nch), std::vector<unsigned char>(nch) };
+  std::vector<unsigned> idx[2];
+  std::vector<int> src[2], pbase[2] = { std::vector<int>(nb + 1, 0), std::vector<int>(nb + 1, 0) };
+  std::vector<long long> ne(nb, 0);
+  for (int pass = 0; pass < 2; pass++) {            // count packets, then fill
+    parallel_for(nb, [&](long long b0, long long b1) {
+      std::vector<std::pair<int, int>> e[CH_ROWS];  // column's place, CSR position
+      for (int b = (int)b0; b < (int)b1; b++) {
+        const int m = start[b + 1] - start[b], k1 = cbase[b + 1] - cbase[b];
+        for (int dir = 0; dir < 2; dir++) {
+          int pk = 0;
+          for (int t = 0; t < k1; t++) {
+            const int k = dir ? k1 - 1 - t : t;
+            size_t w = 0;
+            for (int c = 0; c < CH_ROWS; c++) {
+              const int pos = CH_ROWS * k + (dir ? CH_ROWS - 1 - c : c);
+              e[c].clear();
+              if (pos >= m) continue;
+              const int i = rows[start[b] + pos];
+              if (pass == 0 && dir == 0) slot[i] = (cbase[b] + k) * CH_ROWS + c;
+              for (int p = rp[i] + 1; p < rp[i + 1]; p++) {
+                const int j = I.h_cols[p];
+                if (blk[j] != b || (dir ? j < i : j > i) || at[j] / CH_ROWS == k) continue;
+                e[c].emplace_back(at[j], p);
+              }
+              w = std::max(w, (e[c].size() + 3) / 4);
+            }
+            const int np = std::max(1, (int)(w + 1) / 2);
+            if (pass == 1) {
+              const size_t p0 = (size_t)pbase[dir][b] + pk;
+              cdesc[dir][cbase[b] + t] = (unsigned char)np;
+              for (int c = 0; c < CH_ROWS; c++) {
+                std::sort(e[c].begin(), e[c].end());
+                ne[b] += (long long)e[c].size();
+                const unsigned own = 8u * (CH_ROWS * k + (dir ? CH_ROWS - 1 - c : c));
+                for (int p = 0; p < np; p++)
+                  for (int q = 0; q < 4; q++) {
+                    unsigned o[2] = { own, own };
+                    int from[2] = { -1, -1 };
+                    for (int h = 0; h < 2; h++) {
+                      const size_t l = 4 * (2 * p + h) + q;
+                      if (l < e[c].size()) { o[h] = 8u * e[c][l].first; from[h] = e[c][l].second; }
+                    }
+                    const size_t lane = (p0 + p) * 64 + 4 * c + q;
+                    idx[dir][lane] = o[0] | o[1] << 16;
+                    src[dir][2 * lane] = from[0];
+                    src[dir][2 * lane + 1] = from[1];
+                  }
+              }
+              if (dir == 0)
+                chunks[cbase[b] + k] = int4{ start[b] + CH_ROWS * k, std::min(CH_ROWS, m - CH_ROWS * k),
+                                             cbase[b] + k, cbase[b] + k1 - 1 - k };
+            }
+            pk += np;
+          }
+          if (pass == 0) pbase[dir][b + 1] = pk;
+        }
+      }
+    });
+    if (pass == 0)
+      for (int dir = 0; dir < 2; dir++) {
+        for (int b = 0; b < nb; b++) pbase[dir][b + 1] += pbase[dir][b];
+        // the last chunks' loads ahead end past the last packet
+        idx[dir].assign((size_t)(pbase[dir][nb] + CH_PK) * 64, 0);
+        src[dir].assign((size_t)(pbase[dir][nb] + CH_PK) * 128, -1);
+      }
+  }
+  std::vector<int4> info;
+  for (int b = 0; b < nb; b++)
+    if (start[b + 1] > start[b]) {
+      info.push_back(int4{ start[b], start[b + 1] - start[b], cbase[b], 0 });
+      info.push_back(int4{ pbase[0][b], pbase[1][b], 0, 0 });
+    }
+  S.nb = (int)info.size() / 2;
+  // loaded ahead: two packets where few chunks have more (their others are then loaded when
+  // they are due)
+  long long over = 0;
+  for (int dir = 0; dir < 2; dir++)
+    for (unsigned char np : cdesc[dir]) over += np > 2;
+  S.ahead = over * 20 > 2LL * nch ? CH_PK : 2;
+  S.nch = nch;
+  for (long long v : ne) S.ne += v;
+  S.lds = 8 * (size_t)(((most + CH_ROWS - 1) / CH_ROWS) * CH_ROWS + 64);
+  S.info.upload(info, s);
+  S.rows.upload(rows, s);
+  S.slot.upload(slot, s);
+  S.chunks.upload(chunks, s);
+  S.dlo.upload(cdesc[0], s); S.dup.upload(cdesc[1], s);
+  S.ilo.upload(idx[0], s); S.iup.upload(idx[1], s);
+  S.slo.upload(src[0], s); S.sup.upload(src[1], s);
+  HIPCHECK(hipStreamSynchronize(s));
+  S.on = true;
+}
+
 // Schedule of the row-by-row factorisation: rows by lower level of the whole pattern, per
 // level position {row, start, width, lower entries}, per sorted lower entry the start and
 // length (after the diagonal) of its pivot row, and the plan.
@@ -2592,14 +2998,17 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   // loaded inside the level instead of one level ahead
   int cap = level_cap;
   if (const char* e = getenv("RMX_LEVEL_CAP")) cap = std::max(0, atoi(e));
-  build_blocks(I, &unit, scol, spos, s);
-  I.nlo.on = I.nup.on = false;
-  if (!I.bs.on) {
+  // strip ILU: by chunks; the reference sweeps keep the order of the substitution
+  I.cs.on = false;
+  if (level_cap > 0) build_chunks(I, s);
+  I.bs.on = I.nlo.on = I.nup.on = false;
+  if (!I.cs.on) build_blocks(I, &unit, scol, spos, s);
+  if (!I.cs.on && !I.bs.on) {
     build_nodes(I.nlo, I, true, &unit, scol, spos, s);
     if (I.nlo.on) build_nodes(I.nup, I, false, &unit, scol, spos, s);
   }
   // the level sweeps where neither runs, or RMX_SWEEP asks for them
-  const bool full = !(I.bs.on || (I.nlo.on && I.nup.on)) || sweep_variant() < 2;
+  const bool full = !(I.cs.on || I.bs.on || (I.nlo.on && I.nup.on)) || sweep_variant() < 2;
   std::vector<int> olo, oup;
   build_sweep(I.lo, I, true, olo, s, cap, full);
   build_sweep(I.up, I, false, oup, s, cap, full);
@@ -2640,6 +3049,20 @@ template <> BSvals<double> bsvals<double>(BlockSweep& B)
 template <> BSvals<float> bsvals<float>(BlockSweep& B)
 {
   return { &B.vlo32, &B.vup32, &B.wlo32, &B.wup32, &B.rdg32 };
+}
+// chunk sweep values of one precision: entries, inverses (lower, upper)
+template <class VT> struct CSvals {
+  DBuf<VT> *vlo, *vup;
+  DBuf<double> *tlo, *tup, *dgu;
+};
+template <class VT> static CSvals<VT> csvals(ChunkSweep& S);
+template <> CSvals<double> csvals<double>(ChunkSweep& S)
+{
+  return { &S.vlo64, &S.vup64, &S.tlo64, &S.tup64, &S.dgu64 };
+}
+template <> CSvals<float> csvals<float>(ChunkSweep& S)
+{
+  return { &S.vlo32, &S.vup32, &S.tlo32, &S.tup32, &S.dgu32 };
 }
 // node sweep values of one precision: entries, couplings, reciprocal diagonals (upper)
 template <class VT> struct NSvals {
@@ -2801,6 +3224,19 @@ static void factor_t(Ctx& c, Ilu& I, const VT* A)
     rd.alloc(I.n);
     k_rcp_diag<VT><<<(I.n + 255) / 256, 256, 0, c.stream>>>(I.n, I.rp.p, LU.p, rd.p);
   }
+  if (I.cs.on) {                                // chunk sweeps: values, inverses
+    ChunkSweep& S = I.cs;
+    const CSvals<VT> V = csvals<VT>(S);
+    V.vlo->alloc(S.slo.n);
+    V.vup->alloc(S.sup.n);
+    V.tlo->alloc((size_t)(S.nch + CH_DEEP2) * CH_T);      // loads ahead end past the last chunk
+    V.tup->alloc((size_t)(S.nch + CH_DEEP2) * CH_T);
+    V.dgu->alloc((size_t)(S.nch + CH_DEEP2) * CH_ROWS);
+    k_pack<VT><<<4096, 256, 0, c.stream>>>((long long)S.slo.n, S.slo.p, LU.p, V.vlo->p);
+    k_pack<VT><<<4096, 256, 0, c.stream>>>((long long)S.sup.n, S.sup.p, LU.p, V.vup->p);
+    k_chunk_inv<VT><<<S.nch, 64, 0, c.stream>>>(S.chunks.p, S.rows.p, S.slot.p, I.rp.p, I.cols.p,
+                                                LU.p, V.tlo->p, V.tup->p, V.dgu->p);
+  }
   if (I.bs.on) {                                // block sweeps: values in their entry order
     BlockSweep& B = I.bs;
     const BSvals<VT> V = bsvals<VT>(B);
@@ -2888,6 +3324,32 @@ static void launch_blocks(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t
   HIPCHECK(hipGetLastError());
 }
 
+template <class VT>
+static void launch_chunks(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t* ev,
+                          const int* aidx, const double* aval)
+{
+  ChunkSweep& S = I.cs;
+  const CSvals<VT> V = csvals<VT>(S);
+  if (ev) HIPCHECK(hipEventRecord(ev[0], c.stream));
+  // algorithmic bytes: entry values and 2-byte columns, the inverses of the chunks, per row the
+  // gather index twice, right-hand side and result, the folded prolongation
+  const double bytes = (double)S.ne * (sizeof(VT) + 2.0) + 16.0 * CH_T * S.nch +
+                       32.0 * I.n + (aidx ? 12.0 * I.n : 0.0);
+  const int kt = kt_begin(c, KT_SWEEP_BLK, bytes);
+  auto run = [&](auto* kernel) {
+    kernel<<<S.nb, 64, S.lds, c.stream>>>(S.info.p, S.rows.p, S.dlo.p, S.ilo.p, V.vlo->p, V.tlo->p,
+                                          S.dup.p, S.iup.p, V.vup->p, V.tup->p, V.dgu->p, b, x, aidx, aval);
+  };
+  if (S.ahead == 2) run(k_chunk_sweep<VT, 2>);
+  else run(k_chunk_sweep<VT, CH_PK>);
+  kt_end(c, kt);
+  if (ev) {
+    HIPCHECK(hipEventRecord(ev[1], c.stream));
+    HIPCHECK(hipEventRecord(ev[2], c.stream));
+  }
+  HIPCHECK(hipGetLastError());
+}
+
 template <class VT, bool LOWER>
 static void launch_nodes(Ctx& c, Ilu& I, NodeSweep& S, const double* b, double* x)
 {
@@ -2913,6 +3375,7 @@ static bool apply_t(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t* ev, 
                     const double* aval)
 {
   const int v = sweep_variant();
+  if (I.cs.on && (v >= 2 || !I.lo.packed)) { launch_chunks<VT>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
   if (I.bs.on && (v >= 2 || !I.lo.packed)) { launch_blocks<VT>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
   if (I.nlo.on && I.nup.on && (v >= 2 || !I.lo.packed)) {
     if (ev) HIPCHECK(hipEventRecord(ev[0], c.stream));

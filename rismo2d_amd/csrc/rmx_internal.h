@@ -166,6 +166,27 @@ struct BlockSweep {
   DBuf<double> rdg32, rdg64;       // reciprocal diagonals of the FP32 / FP64 factors
 };
 
+// Sweeps of blocks by chunks of 16 rows (k_chunk_sweep); lower and upper layouts.
+struct ChunkSweep {
+  bool on = false;
+  int nb = 0, nch = 0;             // blocks, chunks
+  int ahead = 4;                   // packets of a chunk that are loaded ahead
+  size_t lds = 0;                  // dynamic LDS bytes of the largest block
+  long long ne = 0;                // entries outside the chunks' triangles
+  DBuf<int4> info;                 // [2 nb] {first place in rows, rows, first chunk, 0},
+                                   //        {first packet lower, upper, 0, 0}
+  DBuf<int> rows;                  // [n] equations block by block, ascending
+  DBuf<int> slot;                  // [n] chunk * 16 + place in it, of every equation
+  DBuf<int4> chunks;               // [nch] {first place in rows, rows, inverse lower, upper}
+  DBuf<unsigned char> dlo, dup;    // [nch] packets of a chunk, in processing order
+  DBuf<unsigned> ilo, iup;         // per packet and lane: two columns, LDS byte offsets
+  DBuf<int> slo, sup;              // CSR position of every value (-1: zero)
+  DBuf<float> vlo32, vup32;
+  DBuf<double> vlo64, vup64;
+  DBuf<double> tlo32, tup32, tlo64, tup64;      // inverses without their diagonals
+  DBuf<double> dgu32, dgu64;                    // diagonals of the upper ones
+};
+
 // Node sweep of one triangle (k_node_sweep): one workgroup per strip of any size, a pass per
 // level of nodes.
 struct NodeSweep {
@@ -207,6 +228,7 @@ struct Ilu {
   DBuf<long long> fpbase;       // per level position: offset of its plan entries
   DBuf<unsigned short> plan;    // per plan entry: pivot index | target position << 8
   SweepSet lo, up;
+  ChunkSweep cs;
   BlockSweep bs;
   NodeSweep nlo, nup;
   DBuf<double> LU64, plo64, pup64, pdg64;

@@ -258,3 +258,34 @@ def test_fgmres_on_ragged_sizes(ctx, n, mkyrl):
         A = sp.csr_matrix((vals.astype(dt).astype(np.float64), cols, rp), shape=(n, n))
         x = splu(A.tocsc()).solve(b)
         assert np.abs(ctx.solution() - x).max() <= 2 * eps * np.linalg.norm(b), prec
+
+
+# strip sweeps by chunks of 16 rows: blocks of one row, around one, three and four chunks (the
+# loads ahead) and of 2,047 rows; rows of no, few (two packets), many (up to eight rounds) and
+# more earlier entries than are loaded ahead (blocks of several strips: the two-level tests).  A sum of at most
+# 128 products of FP64 values and inverses of diagonally dominant triangles (entries at most 1):
+# 1e-12 as for the other sweeps.
+@pytest.mark.parametrize("n,width,stride,strips", [
+    (1, 0, 1, 1), (15, 3, 1, 1), (16, 3, 2, 1), (17, 3, 5, 1), (47, 2, 9, 1), (48, 5, 1, 1),
+    (49, 0, 1, 1), (64, 8, 7, 1), (65, 20, 3, 1), (700, 10, 20, 1), (1024, 30, 17, 1),
+    (1025, 50, 19, 1), (2047, 63, 17, 1), (2047, 4, 300, 1)])
+def test_strip_sweeps_by_chunks(ctx, n, width, stride, strips):
+    print(f"[gpu] {strips} strips, {n} rows, {width} entries a side", flush=True)
+    rp, cols, vals = _band_csr(n, [1 + stride * k for k in range(width)], 51)
+    b = np.random.default_rng(52).standard_normal(n)
+    ctx.set_strips(strips, 0)
+    ctx.csr_upload(rp, cols, vals, b)
+    block = ctx.blocks()
+    rows = np.repeat(np.arange(n), np.diff(rp))
+    keep = block[rows] == block[cols]
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=n))]).astype(np.int32)
+    for prec, dt in ((rmx.F64, np.float64), (rmx.F32, np.float32)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        ctx.silu0_factor(prec)
+        L, r = po.ilu0_factor(rp, cols, vals.astype(dt))
+        assert r == 0
+        ref = po.ilu0_solve(rp2, cols[keep], L[keep], b)
+        y = ctx.precond_apply(rmx.PREC_SILU0, b, prec)
+        assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
+    ctx.set_strips(0, 0)
