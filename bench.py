@@ -284,17 +284,16 @@ def comparison(R, a):
     return out
 
 
-KERNEL_NAMES = {"ilu_factor": "k_ilu_flow (dataflow ILU(0) factorisation, FP32)",
+KERNEL_NAMES = {"ilu_factor": "k_unit_flow (dataflow ILU(0) factorisation by nodes, FP32)",
                 "sweep_lower": "k_sweep_stage lower (strip ILU(0))",
                 "sweep_upper": "k_sweep_stage upper (strip ILU(0) + coarse prolongation)",
                 "spmv": "k_spmv_grp (FP32 row-group SpMV)",
                 "coarse": "coarse correction (restrict, block cyclic reduction, A P residual)",
                 "gram_schmidt": "k_gs_dots + k_gs_update (FP32 basis)",
                 "resid_fp64": "k_spmv<double> (FP64 refinement residual)",
-                "sweeps_block": "k_block_sweep (strip ILU(0), both triangles, one wave per block, "
+                "sweeps_block": "k_chunk_sweep (strip ILU(0), both triangles, one wave per block, "
                                 "+ coarse prolongation)"}
-TRAFFIC_KEYS = {"sweep_lower": "silu_sweep_fwd", "sweep_upper": "silu_sweep_bwd", "spmv": "spmv_f32",
-                "sweeps_block": "silu_block_sweep"}
+TRAFFIC_KEYS = {"sweep_lower": "silu_sweep_fwd", "sweep_upper": "silu_sweep_bwd", "spmv": "spmv_f32"}
 
 
 def main():
