@@ -2860,14 +2860,12 @@ static void build_rows(Ilu& I, const std::vector<int>& scol, hipStream_t s)
   HIPCHECK(hipStreamSynchronize(s));
 }
 
-// Schedule of the factorisation by units of up to `rows_max` rows.  False: a unit of more than
+// Schedule of the factorisation by units of up to `rows_max` rows.  None: a unit of more than
 // FP pivot units, or a pattern that couples a unit to some rows of another.
-static bool build_units(Ilu& I, const std::vector<int>& unit, int rows_max,
-                        const std::vector<int>& scol, hipStream_t s)
+static std::shared_ptr<FlowSchedule> build_units(const Ilu& I, const std::vector<int>& unit,
+                                                 int rows_max, const std::vector<int>& scol,
+                                                 hipStream_t s)
 {
-  FlowUnits& F = I.fu;
-  F.nu = 0;
-  F.desc.release(); F.list.release(); F.plan.release(); F.u32.release(); F.u64.release();
   const int n = I.n;
   const std::vector<int>& rp = I.h_rp;
   std::vector<int> start, of(n);
@@ -2893,17 +2891,17 @@ static bool build_units(Ilu& I, const std::vector<int>& unit, int rows_max,
     while (t < w && scol[p0 + t] < r0) {
       const int K = of[scol[p0 + t]], R = start[K + 1] - start[K];
       for (int q = 0; q < R; q++)
-        if (t + q >= w || scol[p0 + t + q] != start[K] + q) return false;
+        if (t + q >= w || scol[p0 + t + q] != start[K] + q) return nullptr;
       piv.push_back(int4{ (int)ub[K], t | R << 8, start[K + 1] - 1, K });
       lev[g] = std::max(lev[g], lev[K] + 1);
       t += R;
     }
     for (int q = 0; q < rows; q++)
-      if (t + q >= w || scol[p0 + t + q] != r0 + q) return false;
+      if (t + q >= w || scol[p0 + t + q] != r0 + q) return nullptr;
     sd[g] = t;
     top = std::max(top, lev[g]);
     lst[g + 1] = (int)piv.size();
-    if (lst[g + 1] - lst[g] > FP) return false;
+    if (lst[g + 1] - lst[g] > FP) return nullptr;
     ub[g + 1] = ub[g] + (w - t);
   }
   std::vector<int> ptr(top + 2, 0), at(nu);
@@ -2918,9 +2916,11 @@ static bool build_units(Ilu& I, const std::vector<int>& unit, int rows_max,
     desc[2 * (size_t)at[g] + 1] = int4{ lst[g], (int)lines, (int)ub[g], 0 };
     lines += (long long)np * (w > 64 ? 2 : 1);
   }
-  if (lines > INT_MAX || ub[nu] > INT_MAX) return false;
+  if (lines > INT_MAX || ub[nu] > INT_MAX) return nullptr;
   for (int4& e : piv) e.w = at[e.w];
   if (piv.empty()) piv.push_back(int4{ 0, 0, 0, 0 });
+  auto sch = std::make_shared<FlowSchedule>();
+  FlowSchedule& F = *sch;
   F.nu = nu;
   F.cols = ub[nu];
   F.desc.upload(desc, s);
@@ -2929,7 +2929,30 @@ static bool build_units(Ilu& I, const std::vector<int>& unit, int rows_max,
   k_unit_plan<<<nu, 64, 0, s>>>(F.desc.p, F.list.p, I.srt_cols.p, F.plan.p);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(s));
-  return true;
+  return sch;
+}
+
+// Every row's columns ascending, and their places in the row.
+static void sorted_columns(const std::vector<int>& rp, const std::vector<int>& cl,
+                           std::vector<int>& scol, std::vector<unsigned char>& spos)
+{
+  const int n = (int)rp.size() - 1;
+  scol.resize(rp[n]);
+  spos.resize(rp[n]);
+  for (int i = 0; i < n; i++)
+    if (rp[i + 1] - rp[i] > FW) fail(RMX_ERR_RANGE, "ILU(0): row wider than 128 columns");
+  parallel_for(n, [&](long long a, long long b) {
+    std::vector<std::pair<int, int>> tmp;
+    for (long long i = a; i < b; i++) {
+      tmp.clear();
+      for (int q = rp[i]; q < rp[i + 1]; q++) tmp.emplace_back(cl[q], q - rp[i]);
+      std::sort(tmp.begin(), tmp.end());
+      for (size_t t = 0; t < tmp.size(); t++) {
+        scol[rp[i] + t] = tmp[t].first;
+        spos[rp[i] + t] = (unsigned char)tmp[t].second;
+      }
+    }
+  });
 }
 
 // Strips: contiguous row ranges of about equal size.  With `group` (the node of every
@@ -2937,10 +2960,12 @@ static bool build_units(Ilu& I, const std::vector<int>& unit, int rows_max,
 // of one node stay in one strip.  level_cap > 0 splits the sweeps' levels into parts of at
 // most that many rows.
 // `unit`: rows of one unit of the block and node sweeps have one value (the node, or a run of
-// rows with one set of columns).
+// rows with one set of columns).  `twin`: an instance of the same pattern and units, whose
+// schedule of the factorisation serves this one too.
 void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>& cl, int nblk,
                const std::vector<int>* group, const std::vector<int>& unit, hipStream_t s,
-               const HostModel* hm, int nseg, int level_cap)
+               const HostModel* hm, int nseg, int level_cap, const std::vector<int>& scol,
+               const std::vector<unsigned char>& spos, const Ilu* twin)
 {
   I.ready = I.fac64 = I.fac32 = false;
   I.n = n;
@@ -2967,23 +2992,6 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   I.h_rp = rp;
   I.h_cols = cl;
   I.nnz = I.h_rp[n];
-  // per-row sorted columns for the factorisation lookups
-  std::vector<int> scol(I.nnz);
-  std::vector<unsigned char> spos(I.nnz);
-  for (int i = 0; i < n; i++)
-    if (I.h_rp[i + 1] - I.h_rp[i] > FW) fail(RMX_ERR_RANGE, "ILU(0): row wider than 128 columns");
-  parallel_for(n, [&](long long a, long long b) {
-    std::vector<std::pair<int, int>> tmp;
-    for (long long i = a; i < b; i++) {
-      tmp.clear();
-      for (int q = I.h_rp[i]; q < I.h_rp[i + 1]; q++) tmp.emplace_back(I.h_cols[q], q - I.h_rp[i]);
-      std::sort(tmp.begin(), tmp.end());
-      for (size_t t = 0; t < tmp.size(); t++) {
-        scol[I.h_rp[i] + t] = tmp[t].first;
-        spos[I.h_rp[i] + t] = (unsigned char)tmp[t].second;
-      }
-    }
-  });
   I.rp.upload(I.h_rp, s); I.cols.upload(I.h_cols, s);
   I.srt_cols.upload(scol, s); I.srt_pos.upload(spos, s);
   I.flev.clear();
@@ -2991,8 +2999,10 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   // units, of single rows where the pattern couples parts of runs, else row by row (single
   // rows, FP64, 36,000 in a band of 8 a side, 4,000 in one of 30: 54 and 6.2 ms, row by row 78
   // and 8.6)
-  if (!build_units(I, unit, FU, scol, s) && !build_units(I, unit, 1, scol, s))
-    build_rows(I, scol, s);
+  I.fu.u32.release(); I.fu.u64.release();
+  I.fu.sch = twin ? twin->fu.sch : build_units(I, unit, FU, scol, s);
+  if (!I.fu.sch && !twin) I.fu.sch = build_units(I, unit, 1, scol, s);
+  if (!I.fu.sch) build_rows(I, scol, s);
   // strip sweeps: a level of more rows than the staged sweep's row groups (512 threads, 4
   // lanes per row) is split, so that no level needs a second round, whose entries would be
   // loaded inside the level instead of one level ahead
@@ -3097,7 +3107,7 @@ static void factor_t(Ctx& c, Ilu& I, const VT* A)
   };
   const char* lv = getenv("RMX_ILU_LEVELS");
   if (!(lv && atoi(lv) == 1)) {
-    if (!I.fu.nu) need_rows();
+    if (!I.fu.sch) need_rows();
     // one persistent launch: rows in level order, pivot rows awaited by completion flags
     if (I.done.n != (size_t)I.n) {
       I.done.alloc(I.n);
@@ -3139,11 +3149,12 @@ static void factor_t(Ctx& c, Ilu& I, const VT* A)
       HIPCHECK(hipMemcpyAsync(I.flow_state.p, st, sizeof(int) * 4, hipMemcpyHostToDevice,
                               c.stream));
       const int kt = kt_begin(c, KT_FACTOR, 3.0 * (double)I.nnz * (sizeof(VT) + 4));
-      if (I.fu.nu && skip < 0) {
+      if (I.fu.sch && skip < 0) {
+        const FlowSchedule& F = *I.fu.sch;
         DBuf<VT>& U = FUbuf<VT>(I);
-        U.alloc(FU * (size_t)I.fu.cols);
-        k_unit_flow<VT><<<std::min(I.fu.nu, nwu), 64, 0, c.stream>>>(
-            I.fu.desc.p, I.fu.nu, I.fu.list.p, I.fu.plan.p, I.srt_pos.p, LU.p, U.p, I.done.p,
+        U.alloc(FU * (size_t)F.cols);
+        k_unit_flow<VT><<<std::min(F.nu, nwu), 64, 0, c.stream>>>(
+            F.desc.p, F.nu, F.list.p, F.plan.p, I.srt_pos.p, LU.p, U.p, I.done.p,
             I.epoch, I.flow_state.p, spin);
       } else {
         k_ilu_flow<VT><<<nwg, 64, 0, c.stream>>>(I.fdesc.p, I.n, I.cols.p, I.srt_cols.p,
@@ -3444,7 +3455,10 @@ void setup_ilu_schedule(Ctx& c)
       unit[i] = same ? unit[i - 1] : i;
     }
   }
-  ilu_setup(c.ilu, c.n, rp, cl, 1, nullptr, unit, c.stream, nullptr, 1, 0);
+  std::vector<int> scol;
+  std::vector<unsigned char> spos;
+  sorted_columns(rp, cl, scol, spos);
+  ilu_setup(c.ilu, c.n, rp, cl, 1, nullptr, unit, c.stream, nullptr, 1, 0, scol, spos, nullptr);
   // strip ILU: two strips per compute unit (two sweep workgroups fit one CU's LDS), at
   // least a few thousand rows each
   hipDeviceProp_t prop;
@@ -3452,7 +3466,7 @@ void setup_ilu_schedule(Ctx& c)
   int nblk = c.strips > 0 ? c.strips : 2 * prop.multiProcessorCount;
   nblk = std::max(1, std::min(nblk, c.n / 2048));
   ilu_setup(c.silu, c.n, rp, cl, nblk, c.csr_only ? nullptr : &group, unit, c.stream,
-            c.csr_only ? nullptr : &c.hm, strip_segments(c, nblk), STAGE_ROWS);
+            c.csr_only ? nullptr : &c.hm, strip_segments(c, nblk), STAGE_ROWS, scol, spos, &c.ilu);
   c.coarse.ready = c.coarse.fac = false;
   const int cseg = coarse_segments_of(c);
   if (!c.csr_only && cseg > 0) coarse_setup(c, rp, cl, group, cseg);

@@ -203,13 +203,16 @@ struct NodeSweep {
 };
 
 // One ILU(0) system: pattern, factorisation schedule, sweeps and factors.
-// Factorisation by units (the rows of a node): schedule, and the finished rows as its waves
-// hand them on.
-struct FlowUnits {
-  int nu = 0;                   // units (0: the pattern takes the row-by-row kernel)
+// Factorisation by units (the rows of a node): the schedule, shared by a context's two instances
+// of one pattern, and the finished rows as its waves hand them on.
+struct FlowSchedule {
+  int nu = 0;                   // units
   long long cols = 0;           // columns of the units from their first row on
   DBuf<int4> desc, list;        // two per unit in level order; one per pivot unit of a unit
   DBuf<unsigned char> plan;     // per pivot unit and column of a unit: the column's place there
+};
+struct FlowUnits {
+  std::shared_ptr<const FlowSchedule> sch;   // none: the pattern takes the row-by-row kernel
   DBuf<float> u32;              // [cols][3]
   DBuf<double> u64;
 };
