@@ -291,7 +291,7 @@ KERNEL_NAMES = {"ilu_factor": "k_unit_flow (dataflow ILU(0) factorisation by nod
                 "coarse": "coarse correction (restrict, block cyclic reduction, A P residual)",
                 "gram_schmidt": "k_gs_dots + k_gs_update (FP32 basis)",
                 "resid_fp64": "k_spmv<double> (FP64 refinement residual)",
-                "sweeps_block": "k_chunk_sweep (strip ILU(0), both triangles, one wave per block, "
+                "sweeps_block": "k_block_sweep, up to 3,584 blocks k_chunk_sweep (strip ILU(0), both triangles, "
                                 "+ coarse prolongation)"}
 TRAFFIC_KEYS = {"sweep_lower": "silu_sweep_fwd", "sweep_upper": "silu_sweep_bwd", "spmv": "spmv_f32"}
 

@@ -20,8 +20,9 @@
 // updates in the reference's order and, with FMA contraction off, the reference's
 // rounding.  Multipliers are stored negated as in the reference.
 //
-// Sweeps: blocks of at most BS_ROWS rows by a wave each with their values in LDS
-// (k_block_sweep); others by a workgroup per strip that walks the levels of nodes, LDS holding
+// Sweeps: blocks of at most BS_ROWS rows by a wave each with their values in LDS: of the strip
+// sweeps 16 rows at a time (k_chunk_sweep), of many blocks or in the reference order level by
+// level (k_block_sweep); others by a workgroup per strip that walks the levels of nodes, LDS holding
 // the rows that later levels still read (k_node_sweep); where those do not fit LDS, the staged
 // level sweep (k_sweep_stage), whose values go through an LDS ring of RING positions and a
 // global copy in processing order: a level reads a dependency from the ring while its slot has
@@ -1711,6 +1712,11 @@ __global__ void __launch_bounds__(64 * NS_WAVES) k_node_sweep(const int4* __rest
 constexpr int CH_ROWS = 16;       // rows of a chunk
 constexpr int CH_T = 160;         // stored entries of a chunk's inverse
 constexpr int CH_MAX = 128;       // chunks of a block
+// Up to this many blocks (3.5 waves a SIMD) the chain of a block is what counts; beyond, the
+// bytes, of which the level sweep of several blocks a wave (k_block_sweep) takes half: 142 us
+// against 219 at 3,072 blocks (1.8 million rows), 237 against 188 at 4,600, 607 against 353 at
+// 12,300.
+constexpr int CH_BLOCKS = 3584;
 constexpr int CH_DEEP2 = 4, CH_DEEP = 3;
 constexpr int CH_PK = 4;          // most packets of a chunk that are loaded ahead
 
@@ -2700,7 +2706,8 @@ std::vector<int> cut_segments(const std::vector<int>& bstart, const std::vector<
   return seg;
 }
 
-// Chunks of every block; off where a block has more than CH_MAX.
+// Chunks of every block; off where a block has more than BS_ROWS rows, or there are more than
+// CH_BLOCKS blocks.
 static void build_chunks(Ilu& I, hipStream_t s)
 {
   ChunkSweep& S = I.cs;
@@ -2714,7 +2721,7 @@ static void build_chunks(Ilu& I, hipStream_t s)
     for (int i = I.bstart[b]; i < I.bstart[b + 1]; i++) start[(blk[i] = b * nseg + segof(i)) + 1]++;
   int most = 0;
   for (int b = 0; b < nb; b++) most = std::max(most, start[b + 1]);
-  if (most > BS_ROWS) return;
+  if (most > BS_ROWS || nb > CH_BLOCKS) return;
   for (int b = 0; b < nb; b++) start[b + 1] += start[b];
   {
     std::vector<int> next(start.begin(), start.end() - 1);
@@ -3008,7 +3015,7 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   // loaded inside the level instead of one level ahead
   int cap = level_cap;
   if (const char* e = getenv("RMX_LEVEL_CAP")) cap = std::max(0, atoi(e));
-  // strip ILU: by chunks; the reference sweeps keep the order of the substitution
+  // strip ILU of few blocks: by chunks; the reference sweeps keep the order of the substitution
   I.cs.on = false;
   if (level_cap > 0) build_chunks(I, s);
   I.bs.on = I.nlo.on = I.nup.on = false;

@@ -289,3 +289,34 @@ def test_strip_sweeps_by_chunks(ctx, n, width, stride, strips):
         y = ctx.precond_apply(rmx.PREC_SILU0, b, prec)
         assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
     ctx.set_strips(0, 0)
+
+
+# the same strips cut into blocks of some ten rows: 3,400 (by chunks) and 3,740 (level by level);
+# 1e-12 as for the other sweeps
+@pytest.mark.parametrize("segments", [200, 220])
+def test_strip_sweeps_of_many_blocks(ctx, segments):
+    from rismo2d_amd import deck as dk
+    d = dk.meander(30, 130, reach=93.75)
+    ctx.set_strips(17, segments)
+    ctx.upload_mesh(d)
+    ctx.time_step(30.0, 0.7, first=True)
+    n = ctx.prepare()
+    block = ctx.blocks()
+    print(f"[gpu] strip sweeps, {n} equations in {len(np.unique(block))} blocks", flush=True)
+    ctx.assemble(rmx.F64)
+    ctx.scale_l2()
+    rp, cols = ctx.pattern()
+    A, _ = ctx.matrix(rmx.F64)
+    b = np.random.default_rng(61).standard_normal(n)
+    rows = np.repeat(np.arange(n), np.diff(rp))
+    keep = block[rows] == block[cols]
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=n))]).astype(np.int32)
+    for prec, dt in ((rmx.F64, np.float64), (rmx.F32, np.float32)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        ctx.silu0_factor(prec)
+        L, _ = po.ilu0_factor(rp, cols, A.astype(dt))
+        ref = po.ilu0_solve(rp2, cols[keep], L[keep], b)
+        y = ctx.precond_apply(rmx.PREC_SILU0, b, prec)
+        assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
+    ctx.set_strips(0, 0)
