@@ -416,11 +416,12 @@ rmx_status rmx_profile_kernels(rmx_ctx* ctx, int prec, int reps, rmx_kernel_time
  * sweep, 3 Krylov SpMV (the storage precision of the solve, product or residual form),
  * 4 coarse correction (restriction, coarse solve, A P residual), 5 Gram-Schmidt (dots and
  * update), 6 FP64 residual of the refinement, 7 both triangular sweeps of the strip ILU(0)
- * in one launch (block sweeps: one wave per block).  bytes: the algorithmic bytes of each
+ * in one launch (block or chunk sweeps: one wave per block).  bytes: the algorithmic bytes of each
  * launch summed (factorisation 3 nnz (v + 4); sweep: kept entries (v + 4) + 20 or 24 bytes
  * per row; block sweeps: kept entries of both triangles v bytes, 2 bytes per column of a
  * node and triangle, 32 + 16 v per node, 8 per slot descriptor, 4 per pass, 20 per row, + 12
- * per row with the folded prolongation; SpMV: the bytes of the layout it ran on;
+ * per row with the folded prolongation; chunk sweeps: v + 2 bytes per entry outside the 16-row
+ * triangles, 2560 per chunk, 32 per row, + 12 with the prolongation; SpMV: the bytes of the layout it ran on;
  * Gram-Schmidt: the basis vectors read, FP32 or FP64, and the vector read and written;
  * coarse: the vectors, maps and A P entries it reads). */
 typedef struct {
