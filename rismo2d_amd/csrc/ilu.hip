@@ -1711,7 +1711,6 @@ __global__ void __launch_bounds__(64 * NS_WAVES) k_node_sweep(const int4* __rest
 
 constexpr int CH_ROWS = 16;       // rows of a chunk
 constexpr int CH_T = 160;         // stored entries of a chunk's inverse
-constexpr int CH_MAX = 128;       // chunks of a block
 // Up to this many blocks (3.5 waves a SIMD) the chain of a block is what counts; beyond, the
 // bytes, of which the level sweep of several blocks a wave (k_block_sweep) takes half: 142 us
 // against 219 at 3,072 blocks (1.8 million rows), 237 against 188 at 4,600, 607 against 353 at
