@@ -309,6 +309,13 @@ typedef struct {
 } rmx_sweep_info;
 rmx_status rmx_get_sweep_info(rmx_ctx* ctx, int kind, rmx_sweep_info* out);
 
+/* Layout of the strip sweeps by chunks for a pattern cut into blocks (block of every row, 0 ..
+ * nblocks - 1; blocks of at most 2,047 rows), on the host alone: the rows of every block, and one
+ * more than the last place among them that its loads can name, those ahead of a chunk included.
+ * Empty blocks are left out; count: the blocks there are. */
+rmx_status rmx_chunk_reach(int n, const int* rowptr, const int* cols, const int* block, int nblocks,
+                           int* rows, int* reach, int* count);
+
 /* r = A x: replaces CRSMAT::MulVec (CRSMat.cpp:466).  Host pointers. */
 rmx_status rmx_spmv(rmx_ctx* ctx, int prec, const double* x, double* r);
 

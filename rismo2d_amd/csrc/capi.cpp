@@ -796,6 +796,35 @@ rmx_status rmx_get_sweep_info(rmx_ctx* p, int kind, rmx_sweep_info* out)
   API_END
 }
 
+rmx_status rmx_chunk_reach(int n, const int* rowptr, const int* cols, const int* block, int nblocks,
+                           int* rows, int* reach, int* count)
+{
+  API_BEGIN
+  if (n <= 0 || nblocks <= 0 || !rowptr || !cols || !block || !rows || !reach || !count)
+    fail(RMX_ERR_ARG, "chunk layout: missing arrays");
+  for (int i = 0; i < n; i++) {
+    if (block[i] < 0 || block[i] >= nblocks) fail(RMX_ERR_ARG, "chunk layout: block out of range");
+    if (rowptr[i] < 0 || rowptr[i + 1] <= rowptr[i]) fail(RMX_ERR_ARG, "chunk layout: empty row");
+    for (int q = rowptr[i]; q < rowptr[i + 1]; q++)
+      if (cols[q] < 0 || cols[q] >= n) fail(RMX_ERR_ARG, "chunk layout: column out of range");
+  }
+  Ilu I;
+  I.n = n;
+  I.nseg = nblocks;
+  I.bstart = { 0, n };
+  I.seg.assign(block, block + n);
+  I.h_rp.assign(rowptr, rowptr + n + 1);
+  I.h_cols.assign(cols, cols + rowptr[n]);
+  ChunkLayout L;
+  if (!chunk_layout(I, L)) fail(RMX_ERR_RANGE, "chunk layout: a block too large, or too many blocks");
+  std::vector<int> m, top;
+  chunk_reach(L, m, top);
+  std::copy(m.begin(), m.end(), rows);
+  std::copy(top.begin(), top.end(), reach);
+  *count = (int)m.size();
+  API_END
+}
+
 rmx_status rmx_get_blocks(rmx_ctx* p, int* block)
 {
   API_BEGIN

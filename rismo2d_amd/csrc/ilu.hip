@@ -2705,12 +2705,10 @@ std::vector<int> cut_segments(const std::vector<int>& bstart, const std::vector<
   return seg;
 }
 
-// Chunks of every block; off where a block has more than BS_ROWS rows, or there are more than
-// CH_BLOCKS blocks.
-static void build_chunks(Ilu& I, hipStream_t s)
+// Chunk layout of every block (host); false where a block has more than BS_ROWS rows, or there
+// are more than CH_BLOCKS blocks.
+bool chunk_layout(const Ilu& I, ChunkLayout& L)
 {
-  ChunkSweep& S = I.cs;
-  S.on = false;
   const int n = I.n, nseg = std::max(1, I.nseg), nb = I.nblk * nseg;
   const std::vector<int>& rp = I.h_rp;
   auto segof = [&](int i) { return I.seg.empty() ? 0 : I.seg[i]; };
@@ -2720,7 +2718,7 @@ static void build_chunks(Ilu& I, hipStream_t s)
     for (int i = I.bstart[b]; i < I.bstart[b + 1]; i++) start[(blk[i] = b * nseg + segof(i)) + 1]++;
   int most = 0;
   for (int b = 0; b < nb; b++) most = std::max(most, start[b + 1]);
-  if (most > BS_ROWS || nb > CH_BLOCKS) return;
+  if (most > BS_ROWS || nb > CH_BLOCKS) return false;
   for (int b = 0; b < nb; b++) start[b + 1] += start[b];
   {
     std::vector<int> next(start.begin(), start.end() - 1);
@@ -2786,41 +2784,84 @@ static void build_chunks(Ilu& I, hipStream_t s)
             }
             pk += np;
           }
-          if (pass == 0) pbase[dir][b + 1] = pk;
+          // the loads ahead of the last chunks end in packets of zeros times the block's first row,
+          // not in the next block's, whose columns may lie past this block's rows
+          if (pass == 0) pbase[dir][b + 1] = pk + CH_PK;
         }
       }
     });
     if (pass == 0)
       for (int dir = 0; dir < 2; dir++) {
         for (int b = 0; b < nb; b++) pbase[dir][b + 1] += pbase[dir][b];
-        // the last chunks' loads ahead end past the last packet
-        idx[dir].assign((size_t)(pbase[dir][nb] + CH_PK) * 64, 0);
-        src[dir].assign((size_t)(pbase[dir][nb] + CH_PK) * 128, -1);
+        idx[dir].assign((size_t)pbase[dir][nb] * 64, 0);
+        src[dir].assign((size_t)pbase[dir][nb] * 128, -1);
       }
   }
-  std::vector<int4> info;
   for (int b = 0; b < nb; b++)
     if (start[b + 1] > start[b]) {
-      info.push_back(int4{ start[b], start[b + 1] - start[b], cbase[b], 0 });
-      info.push_back(int4{ pbase[0][b], pbase[1][b], 0, 0 });
+      L.info.push_back(int4{ start[b], start[b + 1] - start[b], cbase[b], 0 });
+      L.info.push_back(int4{ pbase[0][b], pbase[1][b], 0, 0 });
     }
-  S.nb = (int)info.size() / 2;
   // loaded ahead: two packets where few chunks have more (their others are then loaded when
   // they are due)
   long long over = 0;
   for (int dir = 0; dir < 2; dir++)
     for (unsigned char np : cdesc[dir]) over += np > 2;
-  S.ahead = over * 20 > 2LL * nch ? CH_PK : 2;
-  S.nch = nch;
-  for (long long v : ne) S.ne += v;
-  S.lds = 8 * (size_t)(((most + CH_ROWS - 1) / CH_ROWS) * CH_ROWS + 64);
-  S.info.upload(info, s);
-  S.rows.upload(rows, s);
-  S.slot.upload(slot, s);
-  S.chunks.upload(chunks, s);
-  S.dlo.upload(cdesc[0], s); S.dup.upload(cdesc[1], s);
-  S.ilo.upload(idx[0], s); S.iup.upload(idx[1], s);
-  S.slo.upload(src[0], s); S.sup.upload(src[1], s);
+  L.ahead = over * 20 > 2LL * nch ? CH_PK : 2;
+  L.nch = nch;
+  L.most = most;
+  for (long long v : ne) L.ne += v;
+  L.rows.swap(rows);
+  L.slot.swap(slot);
+  L.chunks.swap(chunks);
+  for (int dir = 0; dir < 2; dir++) {
+    L.cnt[dir].swap(cdesc[dir]);
+    L.idx[dir].swap(idx[dir]);
+    L.src[dir].swap(src[dir]);
+  }
+  return true;
+}
+
+// Rows of every block of a layout, and of the places that its sweeps read in LDS, the packets
+// loaded past a chunk's own included (as chunk_sweep takes them), one more than the highest.
+void chunk_reach(const ChunkLayout& L, std::vector<int>& rows, std::vector<int>& reach)
+{
+  rows.clear(); reach.clear();
+  for (size_t b = 0; 2 * b < L.info.size(); b++) {
+    const int m = L.info[2 * b].y, cb = L.info[2 * b].z, nch = (m + CH_ROWS - 1) / CH_ROWS;
+    unsigned top = 0;
+    for (int dir = 0; dir < 2; dir++) {
+      size_t p = dir ? L.info[2 * b + 1].y : L.info[2 * b + 1].x;
+      for (int t = 0; t < nch; t++) {
+        const int np = L.cnt[dir][cb + t], read = np <= 2 ? 2 : std::max(np, L.ahead);
+        for (size_t k = p * 64; k < (p + read) * 64; k++)
+          top = std::max({ top, L.idx[dir][k] & 0xFFFFu, L.idx[dir][k] >> 16 });
+        p += np;
+      }
+    }
+    rows.push_back(m);
+    reach.push_back((int)(top / 8) + 1);
+  }
+}
+
+static void build_chunks(Ilu& I, hipStream_t s)
+{
+  ChunkSweep& S = I.cs;
+  ChunkLayout L;
+  S.on = false;
+  if (!chunk_layout(I, L)) return;
+  S.nb = (int)L.info.size() / 2;
+  S.ahead = L.ahead;
+  S.nch = L.nch;
+  S.ne += L.ne;
+  S.lds = 8 * (size_t)(((L.most + CH_ROWS - 1) / CH_ROWS) * CH_ROWS + 64);
+  S.info.upload(L.info, s);
+  S.rows.upload(L.rows, s);
+  S.slot.upload(L.slot, s);
+  S.chunks.upload(L.chunks, s);
+  S.dlo.upload(L.cnt[0], s); S.dup.upload(L.cnt[1], s);
+  S.ilo.upload(L.idx[0], s); S.iup.upload(L.idx[1], s);
+  S.slo.upload(L.src[0], s); S.sup.upload(L.src[1], s);
   HIPCHECK(hipStreamSynchronize(s));
   S.on = true;
 }

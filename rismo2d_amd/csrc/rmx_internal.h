@@ -187,6 +187,18 @@ struct ChunkSweep {
   DBuf<double> dgu32, dgu64;                    // diagonals of the upper ones
 };
 
+// The host side of it: packets of a direction (0 lower, 1 upper) block by block in processing
+// order, a block's stream closed by as many packets of zeros as are loaded ahead.
+struct ChunkLayout {
+  int nch = 0, ahead = 2, most = 0;             // most: rows of the largest block
+  long long ne = 0;
+  std::vector<int4> info, chunks;
+  std::vector<int> rows, slot;
+  std::vector<unsigned char> cnt[2];
+  std::vector<unsigned> idx[2];
+  std::vector<int> src[2];
+};
+
 // Node sweep of one triangle (k_node_sweep): one workgroup per strip of any size, a pass per
 // level of nodes.
 struct NodeSweep {
@@ -483,6 +495,8 @@ std::vector<int> cut_segments(const std::vector<int>& bstart, const std::vector<
                               const HostModel& hm, int nseg);
 void coarse_setup(Ctx& c, const std::vector<int>& rp, const std::vector<int>& cl,
                   const std::vector<int>& group, int nseg);
+bool chunk_layout(const Ilu& I, ChunkLayout& L);
+void chunk_reach(const ChunkLayout& L, std::vector<int>& rows, std::vector<int>& reach);
 int coarse_segments_of(const Ctx& c);          // coarse segments per strip in effect
 void coarse_factor(Ctx& c, int prec);
 bool coarse_begin(Ctx& c, int prec, const double* r);

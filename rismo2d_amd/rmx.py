@@ -152,6 +152,7 @@ def lib():
             "rmx_set_coarse": [_v, C.c_int], "rmx_coarse_factor": [_v, C.c_int],
             "rmx_get_aggregates": [_v, _i, _i], "rmx_precond_apply": [_v, C.c_int, C.c_int, _d, _d],
             "rmx_get_sweep_info": [_v, C.c_int, C.POINTER(SweepInfo)],
+            "rmx_chunk_reach": [C.c_int, _i, _i, _i, C.c_int, _i, _i, _i],
             "rmx_solve": [_v, C.POINTER(KrylovOpts), C.POINTER(KrylovOut)],
             "rmx_get_matrix": [_v, C.c_int, _v, _d], "rmx_get_factors": [_v, C.c_int, _v],
             "rmx_get_solution": [_v, _d], "rmx_set_rhs": [_v, _d], "rmx_set_solution": [_v, _d],
@@ -552,6 +553,18 @@ class Context:
         kt = KernelTimes()
         _check(lib().rmx_profile_kernels(self.h, prec, reps, C.byref(kt)))
         return kt
+
+
+def chunk_reach(rowptr, cols, block):
+    """Rows of every block of a pattern in the strip sweeps by chunks, and one more than the last
+    place among them that its loads can name (host code)."""
+    rp, cl, blk = _c(rowptr, np.int32), _c(cols, np.int32), _c(block, np.int32)
+    nb = int(blk.max()) + 1
+    rows, reach = np.zeros(nb, np.int32), np.zeros(nb, np.int32)
+    count = C.c_int()
+    _check(lib().rmx_chunk_reach(len(blk), _p(rp, _i), _p(cl, _i), _p(blk, _i), nb, _p(rows, _i),
+                                 _p(reach, _i), C.byref(count)))
+    return rows[:count.value], reach[:count.value]
 
 
 def hydrograph(tQS, time):

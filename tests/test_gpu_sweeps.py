@@ -320,3 +320,40 @@ def test_strip_sweeps_of_many_blocks(ctx, segments):
         y = ctx.precond_apply(rmx.PREC_SILU0, b, prec)
         assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
     ctx.set_strips(0, 0)
+
+
+# blocks whose neighbours have more chunks (the automatic cut of this mesh: 33 blocks, some of
+# 703 rows before one of 705), after an apply of a vector of NaN to some 700 blocks that leaves
+# them in the LDS of every compute unit; 1e-12 as for the other sweeps
+def test_chunk_sweeps_after_nan_in_lds(ctx):
+    from rismo2d_amd import deck as dk
+    other = rmx.Context(0)
+    systems = []
+    for c, d in ((other, dk.meander(160, 320, reach=500.0)), (ctx, dk.meander(40, 64, reach=125.0))):
+        c.upload_mesh(d)
+        c.time_step(30.0, 0.7, first=True)
+        n = c.prepare()
+        c.assemble(rmx.F64)
+        c.scale_l2()
+        c.convert(rmx.F32)
+        c.silu0_factor(rmx.F32)
+        systems.append(n)
+    rp, cols = ctx.pattern()
+    A, _ = ctx.matrix(rmx.F64)
+    block = ctx.blocks()
+    rows, reach = rmx.chunk_reach(rp, cols, block)
+    chunks = (rows + 15) // 16
+    assert (reach <= 16 * chunks).all() and (chunks[1:] > chunks[:-1]).any()
+    print(f"[gpu] strip sweeps, {systems[1]} equations in {len(rows)} blocks, after NaN in LDS", flush=True)
+    L, _ = po.ilu0_factor(rp, cols, A.astype(np.float32))
+    of = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+    keep = block[of] == block[cols]
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(of[keep], minlength=len(rp) - 1))]).astype(np.int32)
+    b = np.random.default_rng(71).standard_normal(systems[1])
+    ref = po.ilu0_solve(rp2, cols[keep], L[keep], b)
+    for _ in range(3):
+        y = other.precond_apply(rmx.PREC_SILU0, np.full(systems[0], np.nan), rmx.F32)
+        assert np.isnan(y).all()
+        y = ctx.precond_apply(rmx.PREC_SILU0, b, rmx.F32)
+        assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
+    other.close()
