@@ -309,6 +309,11 @@ typedef struct {
 } rmx_sweep_info;
 rmx_status rmx_get_sweep_info(rmx_ctx* ctx, int kind, rmx_sweep_info* out);
 
+/* The sweeps that an application of an ILU(0) instance runs: by levels in stages, by levels of
+ * nodes, the blocks' levels of nodes, or chunks of 16 rows. */
+enum { RMX_SWEEPS_LEVELS = 1, RMX_SWEEPS_NODES = 2, RMX_SWEEPS_BLOCKS = 3, RMX_SWEEPS_CHUNKS = 4 };
+rmx_status rmx_get_sweeps(rmx_ctx* ctx, int kind, int* sweeps);
+
 /* Layout of the strip sweeps by chunks for a pattern cut into blocks (block of every row, 0 ..
  * nblocks - 1; blocks of at most 2,047 rows), on the host alone: the rows of every block, and one
  * more than the last place among them that its loads can name, those ahead of a chunk included.

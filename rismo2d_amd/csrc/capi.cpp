@@ -796,6 +796,18 @@ rmx_status rmx_get_sweep_info(rmx_ctx* p, int kind, rmx_sweep_info* out)
   API_END
 }
 
+rmx_status rmx_get_sweeps(rmx_ctx* p, int kind, int* sweeps)
+{
+  API_BEGIN
+  Ctx& c = *need(p);
+  if (!sweeps) fail(RMX_ERR_ARG, "null output");
+  if (kind != RMX_PREC_ILU0 && kind != RMX_PREC_SILU0) fail(RMX_ERR_ARG, "kind must be an ILU(0)");
+  const Ilu& I = ilu_of(c, kind);
+  if (!c.prepared || !I.ready) fail(RMX_ERR_ARG, "no system");
+  *sweeps = ilu_sweeps(I);
+  API_END
+}
+
 rmx_status rmx_chunk_reach(int n, const int* rowptr, const int* cols, const int* block, int nblocks,
                            int* rows, int* reach, int* count)
 {

@@ -1979,13 +1979,13 @@ __global__ void __launch_bounds__(64) k_chunk_inv(const int4* __restrict__ chunk
 }
 
 // RMX_SWEEP selects the sweep kernels (tuning and comparison), read when a system is set up
-// and at every application: 1 the staged level sweeps, 2 (default) the block sweeps where
-// every block has at most BS_ROWS rows, else the node sweeps where the rows alive at a time
-// fit LDS, else 1.
+// and at every application: 1 the staged level sweeps; 2 the block sweeps where every block has
+// at most BS_ROWS rows, else the node sweeps where the rows alive at a time fit LDS, else 1;
+// 3 (default) the chunk sweeps of the strip ILU(0) where its blocks fit them, else 2.
 static int sweep_variant()
 {
   const char* e = getenv("RMX_SWEEP");
-  return e ? atoi(e) : 2;
+  return e ? atoi(e) : 3;
 }
 
 // Level sets of the lower or upper dependency graph of rows [a, e), entries with a column
@@ -3056,8 +3056,10 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   int cap = level_cap;
   if (const char* e = getenv("RMX_LEVEL_CAP")) cap = std::max(0, atoi(e));
   // strip ILU of few blocks: by chunks; the reference sweeps keep the order of the substitution
+  // (and the block sweeps where RMX_SWEEP or their pass caps ask for them)
   I.cs.on = false;
-  if (level_cap > 0) build_chunks(I, s);
+  if (level_cap > 0 && sweep_variant() != 2 && !getenv("RMX_BLOCK_LEVEL_ROWS") &&
+      !getenv("RMX_BLOCK_LEVEL_PAIRS")) build_chunks(I, s);
   I.bs.on = I.nlo.on = I.nup.on = false;
   if (!I.cs.on) build_blocks(I, &unit, scol, spos, s);
   if (!I.cs.on && !I.bs.on) {
@@ -3428,14 +3430,23 @@ static void launch_nodes(Ctx& c, Ilu& I, NodeSweep& S, const double* b, double* 
   kt_end(c, kt);
 }
 
+// The sweeps that an application runs (RMX_SWEEPS_*).
+int ilu_sweeps(const Ilu& I)
+{
+  if (sweep_variant() < 2 && I.lo.packed) return RMX_SWEEPS_LEVELS;
+  if (I.cs.on) return RMX_SWEEPS_CHUNKS;
+  if (I.bs.on) return RMX_SWEEPS_BLOCKS;
+  return I.nlo.on && I.nup.on ? RMX_SWEEPS_NODES : RMX_SWEEPS_LEVELS;
+}
+
 template <class VT>
 static bool apply_t(Ctx& c, Ilu& I, const double* b, double* x, hipEvent_t* ev, const int* aidx,
                     const double* aval)
 {
-  const int v = sweep_variant();
-  if (I.cs.on && (v >= 2 || !I.lo.packed)) { launch_chunks<VT>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
-  if (I.bs.on && (v >= 2 || !I.lo.packed)) { launch_blocks<VT>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
-  if (I.nlo.on && I.nup.on && (v >= 2 || !I.lo.packed)) {
+  const int sw = ilu_sweeps(I);
+  if (sw == RMX_SWEEPS_CHUNKS) { launch_chunks<VT>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
+  if (sw == RMX_SWEEPS_BLOCKS) { launch_blocks<VT>(c, I, b, x, ev, aidx, aval); return aidx != nullptr; }
+  if (sw == RMX_SWEEPS_NODES) {
     if (ev) HIPCHECK(hipEventRecord(ev[0], c.stream));
     launch_nodes<VT, true>(c, I, I.nlo, b, I.lo.xp.p);
     if (ev) HIPCHECK(hipEventRecord(ev[1], c.stream));

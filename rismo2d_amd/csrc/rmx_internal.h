@@ -495,6 +495,7 @@ std::vector<int> cut_segments(const std::vector<int>& bstart, const std::vector<
                               const HostModel& hm, int nseg);
 void coarse_setup(Ctx& c, const std::vector<int>& rp, const std::vector<int>& cl,
                   const std::vector<int>& group, int nseg);
+int ilu_sweeps(const Ilu& I);                  // RMX_SWEEPS_* of an application
 bool chunk_layout(const Ilu& I, ChunkLayout& L);
 void chunk_reach(const ChunkLayout& L, std::vector<int>& rows, std::vector<int>& reach);
 int coarse_segments_of(const Ctx& c);          // coarse segments per strip in effect

@@ -152,6 +152,7 @@ def lib():
             "rmx_set_coarse": [_v, C.c_int], "rmx_coarse_factor": [_v, C.c_int],
             "rmx_get_aggregates": [_v, _i, _i], "rmx_precond_apply": [_v, C.c_int, C.c_int, _d, _d],
             "rmx_get_sweep_info": [_v, C.c_int, C.POINTER(SweepInfo)],
+            "rmx_get_sweeps": [_v, C.c_int, _i],
             "rmx_chunk_reach": [C.c_int, _i, _i, _i, C.c_int, _i, _i, _i],
             "rmx_solve": [_v, C.POINTER(KrylovOpts), C.POINTER(KrylovOut)],
             "rmx_get_matrix": [_v, C.c_int, _v, _d], "rmx_get_factors": [_v, C.c_int, _v],
@@ -419,6 +420,12 @@ class Context:
     def sweep_entries(self, kind=PREC_SILU0):
         si = self.sweep_info(kind)
         return si.lower_entries, si.upper_entries
+
+    def sweeps(self, kind=PREC_SILU0):
+        """The sweeps that an application runs: "levels", "nodes", "blocks" or "chunks"."""
+        k = C.c_int()
+        _check(lib().rmx_get_sweeps(self.h, kind, C.byref(k)))
+        return ("levels", "nodes", "blocks", "chunks")[k.value - 1]
 
     def set_coarse(self, segments):
         _check(lib().rmx_set_coarse(self.h, int(segments)))

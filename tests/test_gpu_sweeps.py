@@ -357,3 +357,57 @@ def test_chunk_sweeps_after_nan_in_lds(ctx):
         y = ctx.precond_apply(rmx.PREC_SILU0, b, rmx.F32)
         assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
     other.close()
+
+
+# the sweeps that run where several could: blocks of the strip ILU(0) by chunks, by levels of
+# nodes (RMX_SWEEP=2, or caps of their passes) or in stages (1); more rows a block than 2,047
+@pytest.mark.parametrize("strips,segments,env,kind", [
+    (17, 4, {}, "chunks"), (17, 4, {"RMX_SWEEP": "2"}, "blocks"), (17, 4, {"RMX_SWEEP": "1"}, "levels"),
+    (17, 4, {"RMX_BLOCK_LEVEL_ROWS": "3"}, "blocks"), (17, 4, {"RMX_BLOCK_LEVEL_PAIRS": "5"}, "blocks"),
+    (17, 220, {}, "blocks"), (1, 1, {}, "nodes"), (1, 1, {"RMX_SWEEP": "2"}, "nodes")])
+def test_sweeps_that_run(ctx, strips, segments, env, kind, monkeypatch):
+    for k in ("RMX_SWEEP", "RMX_BLOCK_LEVEL_ROWS", "RMX_BLOCK_LEVEL_PAIRS"):
+        monkeypatch.delenv(k, raising=False)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    ctx.upload_mesh(golden_deck(load_golden("channel200x20")))
+    ctx.prepare()
+    ctx.set_strips(strips, segments)
+    assert ctx.sweeps() == kind
+    ctx.set_strips(0, 0)
+
+
+def _check_block_sweeps(ctx, strips, segments):
+    """FP64 and FP32 applies of a channel's strip ILU(0) by block sweeps against the oracle's
+    triangular solves of the block-restricted factors, 1e-12 as for the other sweeps."""
+    ctx.upload_mesh(golden_deck(load_golden("channel200x20")))
+    ctx.prepare()
+    ctx.set_strips(strips, segments)
+    assert ctx.sweeps() == "blocks"
+    ctx.assemble(rmx.F64)
+    ctx.scale_l2()
+    rp, cols = ctx.pattern()
+    A, B = ctx.matrix(rmx.F64)
+    block = ctx.blocks()
+    rows = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+    keep = block[rows] == block[cols]
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=len(rp) - 1))])
+    for prec, dt in ((rmx.F64, np.float64), (rmx.F32, np.float32)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        ctx.silu0_factor(prec)
+        L, _ = po.ilu0_factor(rp, cols, A.astype(dt))
+        ref = po.ilu0_solve(rp2.astype(np.int32), cols[keep], L[keep], B)
+        y = ctx.silu0_apply(B, prec)
+        assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), prec
+    ctx.set_strips(0, 0)
+    return block
+
+
+# block sweeps of strips that the chunk sweeps take by default: a block a wave, and 61 and 256
+# waves for 128 and 300 segments, two or more blocks of a strip sharing a wave
+@pytest.mark.parametrize("strips,segments", [(17, 2), (17, 4), (4, 8), (4, 32), (17, 128), (4, 300)])
+def test_block_sweeps_on_strips(ctx, strips, segments, monkeypatch):
+    print(f"[gpu] block sweeps, {strips} strips x {segments} segments", flush=True)
+    monkeypatch.setenv("RMX_SWEEP", "2")
+    _check_block_sweeps(ctx, strips, segments)
