@@ -2159,11 +2159,14 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
   // Blocks per wave: neighbouring segments of a strip share a wave, level by level, where a
   // wave per block would leave each SIMD more than one (their levels hold a few nodes each,
   // so a wave alone uses a few of its 16 slots and the chip issues mostly empty lanes): about
-  // BS_WAVES groups in all, of at most BS_GROUP_ROWS rows.
+  // BS_WAVES groups in all (RMX_BLOCK_WAVES: fewer or more, for tests of their size), of at most
+  // BS_GROUP_ROWS rows.
+  int waves = BS_WAVES;
+  if (const char* e = getenv("RMX_BLOCK_WAVES")) waves = std::max(1, atoi(e));
   std::vector<int> gps(nstrip, nseg);          // groups of every strip
   for (int b = 0; b < nstrip; b++) {
     const int rows = I.bstart[b + 1] - I.bstart[b];
-    int k = std::max(1, std::min(nseg, (BS_WAVES + nstrip - 1) / nstrip));
+    int k = std::max(1, std::min(nseg, (waves + nstrip - 1) / nstrip));
     while (k < nseg && (long long)rows * ((nseg + k - 1) / k) > (long long)BS_GROUP_ROWS * nseg * 9 / 10) k++;
     gps[b] = k;
   }

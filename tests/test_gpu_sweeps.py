@@ -411,3 +411,17 @@ def test_block_sweeps_on_strips(ctx, strips, segments, monkeypatch):
     print(f"[gpu] block sweeps, {strips} strips x {segments} segments", flush=True)
     monkeypatch.setenv("RMX_SWEEP", "2")
     _check_block_sweeps(ctx, strips, segments)
+
+
+# blocks that share waves of more than 2,047 rows, up to the most that the rule gives a wave (9/10
+# of 4,093 rows on average): a strip's `segments` blocks cut into `groups` waves of neighbouring ones
+@pytest.mark.parametrize("strips,segments,groups", [(2, 64, 5), (5, 4, 2), (5, 32, 2), (10, 16, 1),
+                                                    (16, 128, 1)])
+def test_block_sweeps_of_long_waves(ctx, strips, segments, groups, monkeypatch):
+    print(f"[gpu] block sweeps, {strips} strips x {segments} segments in {groups} waves", flush=True)
+    monkeypatch.setenv("RMX_SWEEP", "2")
+    monkeypatch.setenv("RMX_BLOCK_WAVES", "1")
+    block = _check_block_sweeps(ctx, strips, segments)
+    rows = np.bincount(block // segments * groups + block % segments * groups // segments)
+    assert len(rows) == strips * groups and 2047 < rows.max() <= 4093
+    assert rows.mean() <= 0.9 * 4093
