@@ -2856,7 +2856,7 @@ static void build_chunks(Ilu& I, hipStream_t s)
   S.nb = (int)L.info.size() / 2;
   S.ahead = L.ahead;
   S.nch = L.nch;
-  S.ne += L.ne;
+  S.ne = L.ne;
   S.lds = 8 * (size_t)(((L.most + CH_ROWS - 1) / CH_ROWS) * CH_ROWS + 64);
   S.info.upload(L.info, s);
   S.rows.upload(L.rows, s);

@@ -425,3 +425,25 @@ def test_block_sweeps_of_long_waves(ctx, strips, segments, groups, monkeypatch):
     rows = np.bincount(block // segments * groups + block % segments * groups // segments)
     assert len(rows) == strips * groups and 2047 < rows.max() <= 4093
     assert rows.mean() <= 0.9 * 4093
+
+
+# the bytes reported for a launch are those of its system, however many were set up before
+def test_reported_bytes_of_a_sweep(ctx, monkeypatch):
+    monkeypatch.delenv("RMX_SWEEP", raising=False)
+    ctx.upload_mesh(golden_deck(load_golden("channel200x20")))
+    ctx.prepare()
+    seen = []
+    for strips, segments, kind in ((17, 4, "chunks"), (17, 220, "blocks"), (17, 4, "chunks"), (17, 4, "chunks"),
+                                   (17, 220, "blocks"), (1, 1, "nodes")):
+        ctx.set_strips(strips, segments)
+        assert ctx.sweeps() == kind
+        ctx.assemble(rmx.F64)
+        ctx.scale_l2()
+        _, B = ctx.matrix(rmx.F64)
+        ctx.silu0_factor(rmx.F64)
+        ctx.kernel_stats(True)
+        ctx.silu0_apply(B, rmx.F64)
+        seen.append(ctx.kernel_stats(False)["sweeps_block"][1])
+    assert seen[0] > 0 and seen[1] > 0
+    assert seen[2] == seen[3] == seen[0] and seen[4] == seen[1] and seen[5] == 0
+    ctx.set_strips(0, 0)
