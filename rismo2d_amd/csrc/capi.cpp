@@ -705,6 +705,7 @@ rmx_status rmx_precond_apply(rmx_ctx* p, int kind, int prec, const double* b, do
   if (!b || !x) fail(RMX_ERR_ARG, "null vector");
   const int pr = prec == RMX_F32 ? RMX_F32 : RMX_F64;
   c.w[0].upload(b, c.n, c.stream);
+  coarse_start(c);
   dev_precond(c, pr, kind, c.w[0].p, c.w[1].p);
   c.w[1].download(x, c.n, c.stream);
   HIPCHECK(hipStreamSynchronize(c.stream));

@@ -889,6 +889,16 @@ static void cr_apply(Ctx& c, Coarse& C)
   HIPCHECK(hipGetLastError());
 }
 
+// A solve or an application starts: no wait of it has been given up yet.  What an earlier one left
+// of the flag, if it ended with another error before coarse_check, is not its own.
+void coarse_start(Ctx& c)
+{
+  Coarse& C = c.coarse;
+  if (C.applied && C.d_state.p)
+    HIPCHECK(hipMemsetAsync(C.d_state.p + 1, 0, sizeof(unsigned long long), c.stream));
+  C.applied = false;
+}
+
 // Whether a coarse solve gave up a wait (the stream must have synchronised).
 void coarse_check(Ctx& c)
 {
@@ -1066,6 +1076,7 @@ void coarse_factor(Ctx& c, int prec)
   HIPCHECK(hipGetLastError());
   C.fac = false;
   C.cr_fac = false;
+  coarse_start(c);
   if (C.cr_ok && !C.d_state.p) {                 // task counter, abort flag, exchanged words
     C.d_state.alloc(2 + 4 * (size_t)C.nb * C.bs);
     HIPCHECK(hipMemsetAsync(C.d_state.p, 0, sizeof(unsigned long long) * C.d_state.n, c.stream));

@@ -737,6 +737,7 @@ void dev_solve(Ctx& c, const rmx_krylov_opts& o0, rmx_krylov_out& out)
 {
   check_opts(c, o0);
   ensure_work(c);
+  coarse_start(c);
   c.X.alloc(c.n);
   const auto t0 = std::chrono::steady_clock::now();
   const rmx_krylov_opts* o = &o0;

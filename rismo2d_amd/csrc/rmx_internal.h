@@ -503,6 +503,7 @@ void coarse_factor(Ctx& c, int prec);
 bool coarse_begin(Ctx& c, int prec, const double* r);
 void coarse_finish(Ctx& c, int prec, double* z);
 void coarse_apply(Ctx& c, int prec, const double* r, double* z);   // device pointers
+void coarse_start(Ctx& c);                     // before the coarse solves that coarse_check sees
 void coarse_check(Ctx& c);                     // fails if a coarse solve gave up a wait
 void dev_precond(Ctx& c, int prec, int kind, const double* in, double* out);
 void spmv_setup(Ctx& c, const int* rowptr, const int* cols);   // host pattern

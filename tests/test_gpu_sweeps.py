@@ -447,3 +447,40 @@ def test_reported_bytes_of_a_sweep(ctx, monkeypatch):
     assert seen[0] > 0 and seen[1] > 0
     assert seen[2] == seen[3] == seen[0] and seen[4] == seen[1] and seen[5] == 0
     ctx.set_strips(0, 0)
+
+
+# A coarse solve's bounded wait (one poll): every workgroup gives up and ends, the call reports
+# it, and factored anew the apply is right again.  `caught`: the wait is given up inside a solve
+# that ends with another error before it is reported; the factors still serve the next apply.
+# 1e-9 as for the other two-level tests.
+@pytest.mark.parametrize("caught", [False, True])
+def test_coarse_wait_given_up(ctx, caught, monkeypatch):
+    from rismo2d_amd import deck as dk
+    ctx.set_coarse(16)
+    ctx.set_strips(0, 0)
+    ctx.upload_mesh(dk.meander(60, 260, reach=187.5))
+    ctx.time_step(30.0, 0.7, first=True)
+    n = ctx.prepare()
+    print(f"[gpu] coarse solve with a wait of one poll, {n} equations, caught {caught}", flush=True)
+    ctx.assemble(rmx.F64)
+    ctx.scale_l2()
+    r = np.random.default_rng(3).standard_normal(n)
+    ctx.silu0_factor(rmx.F64)
+    ctx.coarse_factor(rmx.F64)
+    ref = ctx.precond_apply(rmx.PREC_SILU0C, r, rmx.F64)
+    two = _two_level_reference(ctx, rmx.F64, np.float64, r)
+    assert np.abs(ref - two).max() <= 1e-9 * np.abs(two).max()
+    monkeypatch.setenv("RMX_COARSE_SPIN", "1")
+    if caught:
+        with pytest.raises(rmx.RmxError, match="proceed > 0 without a next solver"):
+            ctx.solve(rmx.FGMRES, rmx.F64, rmx.PREC_SILU0C, max_iter=2, mkyrl=2, eps=1e-30, proceed=1)
+    else:
+        with pytest.raises(rmx.RmxError, match="wait for its neighbours"):
+            ctx.precond_apply(rmx.PREC_SILU0C, r, rmx.F64)
+        with pytest.raises(rmx.RmxError, match="not factored"):
+            ctx.precond_apply(rmx.PREC_SILU0C, r, rmx.F64)
+        ctx.coarse_factor(rmx.F64)
+    monkeypatch.delenv("RMX_COARSE_SPIN")
+    for _ in range(3):
+        np.testing.assert_array_equal(ctx.precond_apply(rmx.PREC_SILU0C, r, rmx.F64), ref)
+    ctx.set_coarse(-1)
