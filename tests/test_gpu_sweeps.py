@@ -484,3 +484,39 @@ def test_coarse_wait_given_up(ctx, caught, monkeypatch):
     for _ in range(3):
         np.testing.assert_array_equal(ctx.precond_apply(rmx.PREC_SILU0C, r, rmx.F64), ref)
     ctx.set_coarse(-1)
+
+
+# the factorisation's bounded wait (64 polls, with far more rows taken than can be ready): every
+# wave gives up and ends, the call reports it, and the next factorisation has the oracle's bits;
+# by units of three rows, and row by row (128 rows that are all coupled but for pairs, so that each
+# is a unit, of more pivots than a unit takes)
+@pytest.mark.parametrize("kind", ["units", "rows"])
+def test_factorisation_wait_given_up(ctx, kind, monkeypatch):
+    rng = np.random.default_rng(81)
+    rp, cols, vals = [0], [], []
+    n = 9000 if kind == "units" else 128
+    for i in range(n):
+        if kind == "units":
+            js = np.arange(max(0, i // 3 - 4) * 3, min(n, (i // 3 + 5) * 3))
+            js = js[js != i]
+        else:
+            js = np.arange(n)
+            js = js[js % 64 != i % 64]
+        v = rng.standard_normal(len(js))
+        cols += [i] + js.tolist()
+        vals += [np.abs(v).sum() + 1.0] + v.tolist()
+        rp.append(len(cols))
+    rp, cols, vals = np.asarray(rp, np.int32), np.asarray(cols, np.int32), np.asarray(vals)
+    print(f"[gpu] factorisation by {kind} with a wait of 64 polls, {n} rows", flush=True)
+    ctx.csr_upload(rp, cols, vals, np.ones(n))
+    ctx.convert(rmx.F32)
+    monkeypatch.setenv("RMX_ILU_SPIN", "32")
+    monkeypatch.setenv("RMX_ILU_WAVES", "4096")
+    with pytest.raises(rmx.RmxError, match="wait for its pivot rows"):
+        ctx.ilu0_factor(rmx.F32)
+    monkeypatch.delenv("RMX_ILU_SPIN")
+    monkeypatch.delenv("RMX_ILU_WAVES")
+    L, _ = po.ilu0_factor(rp, cols, vals.astype(np.float32))
+    for _ in range(2):
+        ctx.ilu0_factor(rmx.F32)
+        np.testing.assert_array_equal(ctx.factors(rmx.F32), L)
