@@ -1321,8 +1321,9 @@ __device__ __forceinline__ T ld_off(const void* base, unsigned off)
 {
   return *reinterpret_cast<const T*>(static_cast<const char*>(base) + off);
 }
-// doubles at a byte offset of the dynamic LDS (kernels without static LDS: it starts at 0, so
-// the offset is the address)
+// doubles at a byte offset of the dynamic LDS (kernels without static LDS, as the set-up makes sure
+// by lds_from_zero: it starts at 0, so the offset is the address; an address from the array's
+// base takes one more instruction an access)
 typedef __attribute__((address_space(3))) double lds_double;
 __device__ __forceinline__ double ld_lds(unsigned off) { return *(const lds_double*)off; }
 __device__ __forceinline__ void st_lds(unsigned off, double v) { *(lds_double*)off = v; }
@@ -1988,6 +1989,17 @@ static int sweep_variant()
   return e ? atoi(e) : 3;
 }
 
+// Fails where one of the kernels that take LDS offsets for addresses has LDS of its own.
+template <class... K>
+static void lds_from_zero(K*... kernels)
+{
+  for (const void* k : { (const void*)kernels... }) {
+    hipFuncAttributes a;
+    HIPCHECK(hipFuncGetAttributes(&a, k));
+    if (a.sharedSizeBytes != 0) fail(RMX_ERR_HIP, "sweeps: dynamic LDS does not start at address 0");
+  }
+}
+
 // Level sets of the lower or upper dependency graph of rows [a, e), entries with a column
 // outside [a, e) or (with `seg`) in another segment ignored.
 static void levels(int a, int e, const std::vector<int>& rp, const std::vector<int>& cl, bool lower,
@@ -2405,6 +2417,7 @@ static void build_blocks(Ilu& I, const std::vector<int>* group, const std::vecto
     std::copy(P.dsrc.begin(), P.dsrc.end(), dsrc.begin() + 4 * ub);
     k++; rb += m; ub += P.usrc[0].size() / 8;
   }
+  lds_from_zero(k_block_sweep<float>, k_block_sweep<double>);
   B.nb = (int)nb; B.lds = (lds + 15) & ~(size_t)15;
   B.ne_lo = std::count_if(src[0].begin(), src[0].end(), [](int q) { return q >= 0; });
   B.ne_up = std::count_if(src[1].begin(), src[1].end(), [](int q) { return q >= 0; });
@@ -2655,6 +2668,11 @@ static void build_nodes(NodeSweep& S, const Ilu& I, bool lower, const std::vecto
         }
     }
   });
+  lds_from_zero(k_node_sweep<float, true, 0>, k_node_sweep<float, true, 1>, k_node_sweep<float, true, 2>,
+                k_node_sweep<float, false, 0>, k_node_sweep<float, false, 1>, k_node_sweep<float, false, 2>,
+                k_node_sweep<double, true, 0>, k_node_sweep<double, true, 1>, k_node_sweep<double, true, 2>,
+                k_node_sweep<double, false, 0>, k_node_sweep<double, false, 1>,
+                k_node_sweep<double, false, 2>);
   S.lgmax = std::min(2, lgmax);
   S.info.upload(info, s); S.tab.upload(tab, s); S.desc.upload(desc, s);
   S.cols.upload(col, s); S.src.upload(src, s); S.wsrc.upload(wsrc, s);
@@ -2853,6 +2871,8 @@ static void build_chunks(Ilu& I, hipStream_t s)
   ChunkLayout L;
   S.on = false;
   if (!chunk_layout(I, L)) return;
+  lds_from_zero(k_chunk_sweep<float, 2>, k_chunk_sweep<float, CH_PK>, k_chunk_sweep<double, 2>,
+                k_chunk_sweep<double, CH_PK>);
   S.nb = (int)L.info.size() / 2;
   S.ahead = L.ahead;
   S.nch = L.nch;
