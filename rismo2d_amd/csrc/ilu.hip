@@ -32,6 +32,7 @@
 // is older than the last such barrier (nr <= RING/4).  Wider levels read everything from the
 // global copy between full barriers.
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -3002,8 +3003,8 @@ static std::shared_ptr<FlowSchedule> build_units(const Ilu& I, const std::vector
   return sch;
 }
 
-// Every row's columns ascending, and their places in the row.
-static void sorted_columns(const std::vector<int>& rp, const std::vector<int>& cl,
+// Every row's columns ascending, and their places in the row; whether a row has a column twice.
+static bool sorted_columns(const std::vector<int>& rp, const std::vector<int>& cl,
                            std::vector<int>& scol, std::vector<unsigned char>& spos)
 {
   const int n = (int)rp.size() - 1;
@@ -3011,6 +3012,7 @@ static void sorted_columns(const std::vector<int>& rp, const std::vector<int>& c
   spos.resize(rp[n]);
   for (int i = 0; i < n; i++)
     if (rp[i + 1] - rp[i] > FW) fail(RMX_ERR_RANGE, "ILU(0): row wider than 128 columns");
+  std::atomic<bool> twice{false};
   parallel_for(n, [&](long long a, long long b) {
     std::vector<std::pair<int, int>> tmp;
     for (long long i = a; i < b; i++) {
@@ -3020,9 +3022,11 @@ static void sorted_columns(const std::vector<int>& rp, const std::vector<int>& c
       for (size_t t = 0; t < tmp.size(); t++) {
         scol[rp[i] + t] = tmp[t].first;
         spos[rp[i] + t] = (unsigned char)tmp[t].second;
+        if (t > 0 && tmp[t].first == tmp[t - 1].first) twice = true;
       }
     }
   });
+  return twice;
 }
 
 // Strips: contiguous row ranges of about equal size.  With `group` (the node of every
@@ -3031,11 +3035,13 @@ static void sorted_columns(const std::vector<int>& rp, const std::vector<int>& c
 // most that many rows.
 // `unit`: rows of one unit of the block and node sweeps have one value (the node, or a run of
 // rows with one set of columns).  `twin`: an instance of the same pattern and units, whose
-// schedule of the factorisation serves this one too.
+// schedule of the factorisation serves this one too.  `twice`: a row has a column more than once,
+// whose values add up: only the row-by-row factorisation and the level sweeps take every entry
+// of a row by itself.
 void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>& cl, int nblk,
                const std::vector<int>* group, const std::vector<int>& unit, hipStream_t s,
                const HostModel* hm, int nseg, int level_cap, const std::vector<int>& scol,
-               const std::vector<unsigned char>& spos, const Ilu* twin)
+               const std::vector<unsigned char>& spos, const Ilu* twin, bool twice)
 {
   I.ready = I.fac64 = I.fac32 = false;
   I.n = n;
@@ -3070,8 +3076,8 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   // rows, FP64, 36,000 in a band of 8 a side, 4,000 in one of 30: 54 and 6.2 ms, row by row 78
   // and 8.6)
   I.fu.u32.release(); I.fu.u64.release();
-  I.fu.sch = twin ? twin->fu.sch : build_units(I, unit, FU, scol, s);
-  if (!I.fu.sch && !twin) I.fu.sch = build_units(I, unit, 1, scol, s);
+  I.fu.sch = twin ? twin->fu.sch : twice ? nullptr : build_units(I, unit, FU, scol, s);
+  if (!I.fu.sch && !twin && !twice) I.fu.sch = build_units(I, unit, 1, scol, s);
   if (!I.fu.sch) build_rows(I, scol, s);
   // strip sweeps: a level of more rows than the staged sweep's row groups (512 threads, 4
   // lanes per row) is split, so that no level needs a second round, whose entries would be
@@ -3081,11 +3087,11 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   // strip ILU of few blocks: by chunks; the reference sweeps keep the order of the substitution
   // (and the block sweeps where RMX_SWEEP or their pass caps ask for them)
   I.cs.on = false;
-  if (level_cap > 0 && sweep_variant() != 2 && !getenv("RMX_BLOCK_LEVEL_ROWS") &&
+  if (level_cap > 0 && !twice && sweep_variant() != 2 && !getenv("RMX_BLOCK_LEVEL_ROWS") &&
       !getenv("RMX_BLOCK_LEVEL_PAIRS")) build_chunks(I, s);
   I.bs.on = I.nlo.on = I.nup.on = false;
-  if (!I.cs.on) build_blocks(I, &unit, scol, spos, s);
-  if (!I.cs.on && !I.bs.on) {
+  if (!I.cs.on && !twice) build_blocks(I, &unit, scol, spos, s);
+  if (!I.cs.on && !I.bs.on && !twice) {
     build_nodes(I.nlo, I, true, &unit, scol, spos, s);
     if (I.nlo.on) build_nodes(I.nup, I, false, &unit, scol, spos, s);
   }
@@ -3538,8 +3544,8 @@ void setup_ilu_schedule(Ctx& c)
   }
   std::vector<int> scol;
   std::vector<unsigned char> spos;
-  sorted_columns(rp, cl, scol, spos);
-  ilu_setup(c.ilu, c.n, rp, cl, 1, nullptr, unit, c.stream, nullptr, 1, 0, scol, spos, nullptr);
+  const bool twice = sorted_columns(rp, cl, scol, spos);
+  ilu_setup(c.ilu, c.n, rp, cl, 1, nullptr, unit, c.stream, nullptr, 1, 0, scol, spos, nullptr, twice);
   // strip ILU: two strips per compute unit (two sweep workgroups fit one CU's LDS), at
   // least a few thousand rows each
   hipDeviceProp_t prop;
@@ -3547,7 +3553,7 @@ void setup_ilu_schedule(Ctx& c)
   int nblk = c.strips > 0 ? c.strips : 2 * prop.multiProcessorCount;
   nblk = std::max(1, std::min(nblk, c.n / 2048));
   ilu_setup(c.silu, c.n, rp, cl, nblk, c.csr_only ? nullptr : &group, unit, c.stream,
-            c.csr_only ? nullptr : &c.hm, strip_segments(c, nblk), STAGE_ROWS, scol, spos, &c.ilu);
+            c.csr_only ? nullptr : &c.hm, strip_segments(c, nblk), STAGE_ROWS, scol, spos, &c.ilu, twice);
   c.coarse.ready = c.coarse.fac = false;
   const int cseg = coarse_segments_of(c);
   if (!c.csr_only && cseg > 0) coarse_setup(c, rp, cl, group, cseg);

@@ -520,3 +520,69 @@ def test_factorisation_wait_given_up(ctx, kind, monkeypatch):
     for _ in range(2):
         ctx.ilu0_factor(rmx.F32)
         np.testing.assert_array_equal(ctx.factors(rmx.F32), L)
+
+
+def _ilu0(n, rows):
+    """ILU(0) of rows {column: value}, row by row; (lower multipliers, upper rows)."""
+    low, up = [], []
+    for i in range(n):
+        a = dict(rows[i])
+        for k in sorted(c for c in a if c < i):
+            a[k] /= up[k][k]
+            for c, u in up[k].items():
+                if c > k and c in a:
+                    a[c] -= a[k] * u
+        low.append({c: v for c, v in a.items() if c < i})
+        up.append({c: v for c, v in a.items() if c >= i})
+    return low, up
+
+
+def _ilu0_solve(low, up, b):
+    x = np.array(b, float)
+    for i in range(len(x)):
+        x[i] -= sum(v * x[c] for c, v in low[i].items())
+    for i in range(len(x) - 1, -1, -1):
+        x[i] = (x[i] - sum(v * x[c] for c, v in up[i].items() if c > i)) / up[i][i]
+    return x
+
+
+# a caller's CSR rows as they may come: columns in any order, a pattern that is not symmetric,
+# entries of value zero, a lower column twice in a row (its values add up, as in a product);
+# one block (block and chunk sweeps) and more rows than a block takes (node sweeps).  Diagonally
+# dominant; sums of some ten products and quotients in FP64: 1e-12 as for the other sweeps.
+@pytest.mark.parametrize("form", ["asymmetric", "zeros", "repeated", "repeated runs"])
+@pytest.mark.parametrize("n", [12, 300, 3000])
+def test_csr_row_forms(ctx, n, form):
+    print(f"[gpu] {n} CSR rows, {form}", flush=True)
+    rng = np.random.default_rng(91)
+    run = 3 if form == "repeated runs" else 1
+    near = [np.unique(np.clip(i // run + rng.integers(-9, 10, 5), 0, n // run - 1)) for i in range(0, n, run)]
+    if form != "asymmetric":
+        near = [np.unique(np.concatenate([near[i], [j for j in range(len(near)) if abs(i - j) < 10 and i in near[j]],
+                                          [i]])).astype(int) for i in range(len(near))]
+    rows, rp, cols, vals = [], [0], [], []
+    for i in range(n):
+        js = [run * int(j) + q for j in near[i // run] for q in range(run) if run * j + q != i]
+        v = rng.standard_normal(len(js))
+        if form == "zeros":
+            v *= rng.random(len(js)) < 0.6
+        rows.append({i: float(np.abs(v).sum() + 1.0), **{j: float(x) for j, x in zip(js, v)}})
+        ent = list(zip(js, v))
+        if form.startswith("repeated"):
+            part = rng.random(len(js))
+            ent = [(j, x * p if j < i else x) for (j, x), p in zip(ent, part)] + \
+                [(j, x - x * p) for (j, x), p in zip(ent, part) if j < i]
+        o = rng.permutation(len(ent))
+        cols += [i] + [ent[k][0] for k in o]
+        vals += [rows[i][i]] + [ent[k][1] for k in o]
+        rp.append(len(cols))
+    rp, cols, vals = np.asarray(rp, np.int32), np.asarray(cols, np.int32), np.asarray(vals, float)
+    b = rng.standard_normal(n)
+    ref = _ilu0_solve(*_ilu0(n, rows), b)
+    ctx.set_strips(1, 0)
+    ctx.csr_upload(rp, cols, vals, b)
+    ctx.ilu0_factor(rmx.F64)
+    ctx.silu0_factor(rmx.F64)
+    for y in (ctx.ilu0_apply(b, rmx.F64), ctx.precond_apply(rmx.PREC_SILU0, b, rmx.F64)):
+        assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
+    ctx.set_strips(0, 0)
