@@ -380,8 +380,10 @@ rmx_status rmx_set_rhs(rmx_ctx* ctx, const double* B);
 /* The Newton correction rmx_newton_update applies: a caller that solved the system itself
  * (as EQS_UVS2D::Execute gets X from EQS::Solve, EqsUVS2D.cpp:365) hands it over. */
 rmx_status rmx_set_solution(rmx_ctx* ctx, const double* X /* neq */);
-/* Load an arbitrary CSR system (diagonal first in every row): lets a caller that keeps
- * the reference's own EQS/CRSMAT host code hand its pattern and values over. */
+/* Load an arbitrary CSR system (diagonal first in every row, the other columns in any order): lets
+ * a caller that keeps the reference's own EQS/CRSMAT host code hand its pattern and values over.
+ * A column is to be given once; a lower column given more than once counts with the sum of its
+ * values (with the slower general kernels of the ILU(0)). */
 rmx_status rmx_csr_upload(rmx_ctx* ctx, int n, const int* rowptr, const int* cols,
                           const double* vals, const double* B);
 

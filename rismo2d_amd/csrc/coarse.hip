@@ -355,6 +355,11 @@ __global__ void __launch_bounds__(CR_THREADS) k_cr_solve(int nb, int bs, int lev
 // read of 8 nc^2 bytes spread over the chip, in place of the chain of exchanges: the unit
 // vectors are taken through the reduction's steps together, W row-major (row i * bs + r: block
 // i's row r; column J: the unit vector of aggregate J), and W is the inverse.
+// Product and chain, us an application, and the inverse, ms a factorisation (meanders 320 cells
+// wide): 432 rows 4.4 and 28, 0.6; 1,344 rows 6.3 and 35, 0.8; 2,712 rows 12 and 41, 1.0; 3,384 rows
+// 17 and 47, 1.3; 4,056 rows 24 and 47, 1.5; 4,728 rows 38 and 47, 1.8; 5,736 rows 56 and 48, 2.3;
+// 10,800 rows 189 and 56, 6.4.  They cross at some 5,200 rows for the application alone; the line
+// lies below, where some 40 applications pay the inverse back (65 at 4,056 rows, 200 at 4,728).
 
 constexpr int CR_DENSE = 3072;
 constexpr int CR_TILE = 64;       // columns of W per workgroup

@@ -15,7 +15,8 @@
 //    not the preconditioner, decides the answer.
 //
 // Factorisation: one persistent launch, one wave per unit of up to three rows (k_unit_flow), or
-// per row where the pattern does not allow that and after a pivot repair (k_ilu_flow); row i
+// per row where the pattern does not allow that (a row with a column twice among them) and after a
+// pivot repair (k_ilu_flow); row i
 // eliminates its lower entries in increasing column order, so every factor entry gets its
 // updates in the reference's order and, with FMA contraction off, the reference's
 // rounding.  Multipliers are stored negated as in the reference.
@@ -23,8 +24,8 @@
 // Sweeps: blocks of at most BS_ROWS rows by a wave each with their values in LDS: of the strip
 // sweeps 16 rows at a time (k_chunk_sweep), of many blocks or in the reference order level by
 // level (k_block_sweep); others by a workgroup per strip that walks the levels of nodes, LDS holding
-// the rows that later levels still read (k_node_sweep); where those do not fit LDS, the staged
-// level sweep (k_sweep_stage), whose values go through an LDS ring of RING positions and a
+// the rows that later levels still read (k_node_sweep); where those do not fit LDS, or a row has a
+// column twice, the staged level sweep (k_sweep_stage), whose values go through an LDS ring of RING positions and a
 // global copy in processing order: a level reads a dependency from the ring while its slot has
 // not been reused (position >= P + nr - RING for a level of nr rows starting at P) and from the
 // global copy otherwise, which is safe because a full barrier (global release / acquire) is
@@ -1377,11 +1378,12 @@ __device__ __forceinline__ double node_solve(double x, double s, const W2& w, do
 // The passes of one triangle of one block.  A pass holds up to 16 slots of 4 lanes; a slot
 // holds up to 16 columns of one node, a node takes 1, 2, 4 or 8 neighbouring slots, and the
 // nodes of a pass do not depend on each other.  Lane q of a slot multiplies column group q
-// into the node's row sums; every lane of the node gets them and solves the node's rows in
-// registers; lane r of its first slot writes row r.  Column groups that a slot does not have read the block's zero group and the zero slot
-// before x; rows that a node does not have read what follows and are not used.
-// The chain from one pass to the next is one LDS read, four products, two exchanges, the
-// node's solve and one LDS write, and a wave working alone is bound by its instructions
+// into the node's row sums; they end in the node's first slot, row r's in lane r (node_sum), the
+// rows are solved across those lanes (node_solve) and lane r writes row r.  Column groups that a
+// slot does not have read the block's zero group and the zero slot before x; rows that a node does
+// not have read what follows and are not used.
+// The chain from one pass to the next is one LDS read, four products, two exchanges (more for
+// nodes of several slots), the node's solve and one LDS write, and a wave working alone is bound by its instructions
 // (about 105 a pass, 4 cycles each; a branch costs about 70): nothing waits for memory, since
 // values, columns, couplings and reciprocal diagonals are loaded D passes ahead into a
 // register ring, the descriptors that name them 2 D, and the pass table's entries 3 D ahead.
@@ -1687,9 +1689,6 @@ __global__ void __launch_bounds__(64 * NS_WAVES) k_node_sweep(const int4* __rest
 }
 
 // ---------------------------------------------------------------------------------------
-// host set-up
-
-// ---------------------------------------------------------------------------------------
 // sweeps of blocks by chunks of 16 rows
 //
 // A block's triangular solve is a chain, of nodes if taken level by level (80 to 300 levels of
@@ -1704,12 +1703,15 @@ __global__ void __launch_bounds__(64 * NS_WAVES) k_node_sweep(const int4* __rest
 // of loads (past a chunk's packets the next one's), so that the compiler's waits name the right
 // ones.  Of the inverse the upper 4 x 4 blocks are not stored: plane j holds rows 4 j .. 4 j + 3,
 // columns up to 4 j + 3.
-// FP32, FP64 factors, both directions: 36 us at 5,600 rows (60 x 13 quads), 37 at 36,000, 42 at
-// 231,000, 72, 88 at 923,000, 142, 169 at 1.8 million (3 TB/s); node by node 63, 43, 209, 251,
+// FP32, FP64 factors, both directions: 35, 33 us at 5,600 rows (60 x 13 quads), 35, 36 at 36,000,
+// 39 at 231,000, 70, 84 at 923,000, 140, 164 at 1.8 million (3 TB/s); node by node 63, 43, 209, 251,
 // 241 us (FP32).  A link takes 0.24 us: some 280 cycles of dependent FP64 operations, an LDS
 // write and read, the issue of the rest.  Matrix instructions for the row sums and the product
-// are not faster (0.27 us: a dependent 4x4x4 FP64 one takes 50 cycles, an addition 28); more
-// chunks ahead change nothing; chunks of 32 rows would take 1.6 times the bytes.
+// are not faster (0.27 us: a dependent 4x4x4 FP64 one takes 50 cycles, an addition 28); chunks of
+// 32 rows would take 1.6 times the bytes.
+// A packet loaded past a chunk's own is the next chunk's; past a block's last chunk the stream
+// holds packets of zeros that name the block's first row, so that LDS is read at the block's rows
+// alone (what lies behind them is not written, and zero times a NaN is a NaN).
 
 constexpr int CH_ROWS = 16;       // rows of a chunk
 constexpr int CH_T = 160;         // stored entries of a chunk's inverse
@@ -1718,6 +1720,9 @@ constexpr int CH_T = 160;         // stored entries of a chunk's inverse
 // against 219 at 3,072 blocks (1.8 million rows), 237 against 188 at 4,600, 607 against 353 at
 // 12,300.
 constexpr int CH_BLOCKS = 3584;
+// Chunks in flight with two packets ahead each and with four (FP32, one less, this, and 6 and 4: 40,
+// 39, 39 us at 231,000 rows with two packets; 37, 35, 34 at 36,000 and 43, 39, 37 at 145,000, cells
+// of a channel, 139, 140, 139 at 1.8 million with four).
 constexpr int CH_DEEP2 = 4, CH_DEEP = 3;
 constexpr int CH_PK = 4;          // most packets of a chunk that are loaded ahead
 
@@ -1980,6 +1985,9 @@ __global__ void __launch_bounds__(64) k_chunk_inv(const int4* __restrict__ chunk
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// host set-up
+
 // RMX_SWEEP selects the sweep kernels (tuning and comparison), read when a system is set up
 // and at every application: 1 the staged level sweeps; 2 the block sweeps where every block has
 // at most BS_ROWS rows, else the node sweeps where the rows alive at a time fit LDS, else 1;
@@ -2131,7 +2139,7 @@ static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>&
 // passes of at most 16 slots.  Local positions list the units in lower order, a unit's rows
 // together.  The first column group and the first 3 row groups of a block's streams are zero.
 // Entries keep the strip sweeps' rule (the strict triangle inside the row's
-// block), minus the couplings inside a unit, which go to the unit's record.  Off (the strip
+// block), minus the couplings inside a unit, which go to the unit's record.  Off (the node
 // sweeps run) when a block has more than BS_ROWS rows or a group does not fit the
 // descriptors.
 // scol, spos: every row's columns ascending and their places in the row.
@@ -2824,8 +2832,11 @@ bool chunk_layout(const Ilu& I, ChunkLayout& L)
       L.info.push_back(int4{ start[b], start[b + 1] - start[b], cbase[b], 0 });
       L.info.push_back(int4{ pbase[0][b], pbase[1][b], 0, 0 });
     }
-  // loaded ahead: two packets where few chunks have more (their others are then loaded when
-  // they are due)
+  // loaded ahead: two packets where at most a tenth of the chunks has more (their others are then
+  // loaded when they are due), else four.  FP32, us with two and with four: rows of up to 16 entries
+  // a side, 2,047 of them, 68 and 80, 700 of them 26 and 30; meanders of 231,000 and 923,000 rows
+  // (below the tenth) 39 and 39, 70 and 70; channels of 36,000 and 145,000 rows (above it) 36 and 34,
+  // 46 and 39, quadrilaterals of 5,600 rows 39 and 35, 1.8 million rows 143 and 140.
   long long over = 0;
   for (int dir = 0; dir < 2; dir++)
     for (unsigned char np : cdesc[dir]) over += np > 2;

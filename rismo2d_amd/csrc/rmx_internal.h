@@ -170,7 +170,7 @@ struct BlockSweep {
 struct ChunkSweep {
   bool on = false;
   int nb = 0, nch = 0;             // blocks, chunks
-  int ahead = 4;                   // packets of a chunk that are loaded ahead
+  int ahead = 2;                   // packets of a chunk that are loaded ahead (2 or CH_PK)
   size_t lds = 0;                  // dynamic LDS bytes of the largest block
   long long ne = 0;                // entries outside the chunks' triangles
   DBuf<int4> info;                 // [2 nb] {first place in rows, rows, first chunk, 0},
@@ -214,7 +214,6 @@ struct NodeSweep {
   DBuf<double> v64, w64, rdg32, rdg64;
 };
 
-// One ILU(0) system: pattern, factorisation schedule, sweeps and factors.
 // Factorisation by units (the rows of a node): the schedule, shared by a context's two instances
 // of one pattern, and the finished rows as its waves hand them on.
 struct FlowSchedule {
@@ -229,6 +228,7 @@ struct FlowUnits {
   DBuf<double> u64;
 };
 
+// One ILU(0) system: pattern, factorisation schedule, sweeps and factors.
 struct Ilu {
   bool ready = false;
   int n = 0, nblk = 1, nseg = 1;
