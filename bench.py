@@ -293,7 +293,8 @@ KERNEL_NAMES = {"ilu_factor": "k_unit_flow (dataflow ILU(0) factorisation by nod
                 "resid_fp64": "k_spmv<double> (FP64 refinement residual)",
                 "sweeps_block": "k_block_sweep, up to 3,584 blocks k_chunk_sweep (strip ILU(0), both triangles, "
                                 "+ coarse prolongation)"}
-TRAFFIC_KEYS = {"sweep_lower": "silu_sweep_fwd", "sweep_upper": "silu_sweep_bwd", "spmv": "spmv_f32"}
+TRAFFIC_KEYS = {"sweep_lower": "silu_sweep_fwd", "sweep_upper": "silu_sweep_bwd", "spmv": "spmv_f32",
+                "sweeps_block": "silu_block_sweep"}
 
 
 def main():
