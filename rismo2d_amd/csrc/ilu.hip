@@ -1705,10 +1705,10 @@ __global__ void __launch_bounds__(64 * NS_WAVES) k_node_sweep(const int4* __rest
 // columns up to 4 j + 3.
 // FP32, FP64 factors, both directions: 35, 33 us at 5,600 rows (60 x 13 quads), 35, 36 at 36,000,
 // 39 at 231,000, 70, 84 at 923,000, 140, 164 at 1.8 million (3 TB/s); node by node 63, 43, 209, 251,
-// 241 us (FP32).  A link takes 0.24 us: some 280 cycles of dependent FP64 operations, an LDS
-// write and read, the issue of the rest.  Matrix instructions for the row sums and the product
-// are not faster (0.27 us: a dependent 4x4x4 FP64 one takes 50 cycles, an addition 28); chunks of
-// 32 rows would take 1.6 times the bytes.
+// 241 us (FP32).  A link takes 0.25 us (two packets a chunk) to 0.3 (four): some 280 cycles of
+// dependent FP64 operations, an LDS write and read, the issue of the rest.  Matrix instructions for
+// the row sums and the product are slower by a tenth (a dependent 4x4x4 FP64 one takes 50 cycles, an
+// addition 28); chunks of 32 rows would take 1.6 times the bytes.
 // A packet loaded past a chunk's own is the next chunk's; past a block's last chunk the stream
 // holds packets of zeros that name the block's first row, so that LDS is read at the block's rows
 // alone (what lies behind them is not written, and zero times a NaN is a NaN).
