@@ -20,6 +20,13 @@ constexpr int HOST_TAG = 63;      // word of the pinned mirror that a kernel's r
 
 enum { S_RHO = 0, S_RV = 2, S_TS = 3, S_TT = 4, S_RR = 5, S_B2 = 6 };
 
+// BiCGStab's omega = (t, s) / (t, t).  t is zero where s is: the preconditioner solved the system
+// exactly (a diagonal, a dense block), the step along p ends it, and 0 / 0 would lose it.
+__device__ __forceinline__ double bicg_omega(const double* __restrict__ sc)
+{
+  return sc[S_TT] != 0.0 ? sc[S_TS] / sc[S_TT] : 0.0;
+}
+
 __global__ void k_copy3(long long n, const double* __restrict__ b, double* __restrict__ r,
                         double* __restrict__ r0, double* __restrict__ p, double* __restrict__ x)
 {
@@ -45,7 +52,7 @@ __global__ void k_bicg_xr(long long n, const double* __restrict__ sc, int rho,
                           double* __restrict__ r)
 {
   const double alpha = sc[rho] / sc[S_RV];
-  const double omega = sc[S_TS] / sc[S_TT];
+  const double omega = bicg_omega(sc);
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {
     double xi = x[i] + alpha * p[i];
@@ -60,8 +67,8 @@ __global__ void k_bicg_p(long long n, const double* __restrict__ sc, int rho_old
                          double* __restrict__ p)
 {
   const double alpha = sc[rho_old] / sc[S_RV];
-  const double omega = sc[S_TS] / sc[S_TT];
-  const double beta = sc[rho_new] * alpha / (sc[rho_old] * omega);
+  const double omega = bicg_omega(sc);
+  const double beta = omega != 0.0 ? sc[rho_new] * alpha / (sc[rho_old] * omega) : 0.0;
   const double bo = -beta * omega;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (long long)gridDim.x * blockDim.x) {

@@ -586,3 +586,34 @@ def test_csr_row_forms(ctx, n, form):
     for y in (ctx.ilu0_apply(b, rmx.F64), ctx.precond_apply(rmx.PREC_SILU0, b, rmx.F64)):
         assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
     ctx.set_strips(0, 0)
+
+
+# BiCGStab where the preconditioner solves the system exactly: a diagonal and small dense systems
+# whose factors' solve leaves s = 0 to the last bit.  Diagonally dominant: |A^-1| <= 1, and x is off
+# by at most some ten roundings of its terms.
+@pytest.mark.parametrize("n,dense", [(1, False), (2, True), (3, True), (5, False), (12, True), (300, False),
+                                     (5000, False)])
+@pytest.mark.parametrize("seed", [0, 1, 2, 3])
+def test_bicgstab_with_an_exact_preconditioner(ctx, n, dense, seed):
+    print(f"[gpu] BiCGStab, {n} rows, exact preconditioner", flush=True)
+    rng = np.random.default_rng(seed)
+    A = np.zeros((n, n)) if dense else None
+    rp, cols, vals = [0], [], []
+    for i in range(n):
+        js = rng.permutation([j for j in range(n) if j != i]) if dense else np.zeros(0, int)
+        v = rng.standard_normal(len(js))
+        cols += [i] + [int(j) for j in js]
+        vals += [float(np.abs(v).sum() + 1.0 + rng.random())] + v.tolist()
+        rp.append(len(cols))
+    rp, cols, vals = np.asarray(rp, np.int32), np.asarray(cols, np.int32), np.asarray(vals, float)
+    b = rng.standard_normal(n)
+    ctx.csr_upload(rp, cols, vals, b)
+    ctx.ilu0_factor(rmx.F64)
+    out = ctx.solve(rmx.BICGSTAB, rmx.F64, rmx.PREC_ILU0, max_iter=20, eps=1e-12)
+    if dense:
+        A[np.repeat(np.arange(n), np.diff(rp)), cols] = vals
+        x = np.linalg.solve(A, b)
+    else:
+        x = b / vals
+    assert out.converged
+    assert np.abs(ctx.solution() - x).max() <= 1e-12 * np.abs(b).max()
