@@ -789,8 +789,9 @@ rmx_status rmx_get_sweep_info(rmx_ctx* p, int kind, rmx_sweep_info* out)
   Ctx& c = *need(p);
   if (!out) fail(RMX_ERR_ARG, "null output");
   if (kind != RMX_PREC_ILU0 && kind != RMX_PREC_SILU0) fail(RMX_ERR_ARG, "kind must be an ILU(0)");
-  const Ilu& I = ilu_of(c, kind);
+  Ilu& I = ilu_of(c, kind);
   if (!c.prepared || !I.ready) fail(RMX_ERR_ARG, "no system");
+  sweep_levels(I);
   out->lower_entries = I.lo.ne; out->upper_entries = I.up.ne;
   out->lower_levels = I.lo.nlev_max; out->upper_levels = I.up.nlev_max;
   out->strips = I.nblk; out->segments = I.nseg;

@@ -2043,16 +2043,16 @@ static void levels(int a, int e, const std::vector<int>& rp, const std::vector<i
   else { for (int i = e - 1; i >= a; i--) rows[fill[lev[i]]++] = i; }
 }
 
-// Packed layout of one sweep over all blocks; without `full` only its counts (the block or
-// node sweeps run).
-static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>& order,
-                        hipStream_t s, int cap, bool full)
+// Rows of the levels of every strip, levels of more than cap rows split: per strip its first
+// level and position, per level its first position (and one more, a sentinel).
+static void strip_levels(SweepSet& S, const Ilu& I, bool lower, int cap, std::vector<int>& blev,
+                         std::vector<int>& bpos, std::vector<int>& levp, std::vector<int>& prow)
 {
   const int n = I.n, nb = I.nblk;
   const std::vector<int>& rp = I.h_rp;
   const std::vector<int>& cl = I.h_cols;
   std::vector<int> lev(n, 0);
-  std::vector<int> blev(nb + 1, 0), bpos(nb + 1, 0), levp, prow;
+  blev.assign(nb + 1, 0); bpos.assign(nb + 1, 0); levp.clear(); prow.clear();
   levp.reserve(n / 8);
   prow.reserve(n);
   int maxnr = 0, nlev_tot = 0;
@@ -2075,6 +2075,51 @@ static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>&
     prow.insert(prow.end(), rows.begin(), rows.end());
     nlev_tot = std::max(nlev_tot, nl);
   }
+  S.nlev_max = nlev_tot;
+  S.max_nr = maxnr;
+  S.nlev_sum = blev[nb];
+}
+
+// Entries that the sweeps of I keep: the strict lower / upper part inside a row's strip and segment.
+static void count_entries(Ilu& I)
+{
+  std::atomic<long long> lo{0}, up{0};
+  const bool sg = !I.seg.empty();
+  std::vector<int> blk(I.nblk > 1 ? I.n : 0);
+  if (I.nblk > 1)
+    for (int b = 0; b < I.nblk; b++) std::fill(blk.begin() + I.bstart[b], blk.begin() + I.bstart[b + 1], b);
+  parallel_for(I.n, [&](long long a, long long e) {
+    long long l = 0, u = 0;
+    for (long long i = a; i < e; i++)
+      for (int q = I.h_rp[i] + 1; q < I.h_rp[i + 1]; q++) {
+        const int c = I.h_cols[q];
+        if ((I.nblk > 1 && blk[c] != blk[i]) || (sg && I.seg[c] != I.seg[i])) continue;
+        l += c < i;
+        u += c > i;
+      }
+    lo += l;
+    up += u;
+  });
+  I.lo.ne = lo;
+  I.up.ne = up;
+}
+
+// Levels of a system whose sweeps do not walk them, worked out where they are asked for.
+void sweep_levels(Ilu& I)
+{
+  std::vector<int> blev, bpos, levp, prow;
+  if (I.lo.nlev_max < 0) strip_levels(I.lo, I, true, I.level_cap, blev, bpos, levp, prow);
+  if (I.up.nlev_max < 0) strip_levels(I.up, I, false, I.level_cap, blev, bpos, levp, prow);
+}
+
+// Packed layout of one sweep over all blocks.
+static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>& order, hipStream_t s)
+{
+  const int n = I.n, nb = I.nblk;
+  const std::vector<int>& rp = I.h_rp;
+  const std::vector<int>& cl = I.h_cols;
+  std::vector<int> blev, bpos, levp, prow;
+  strip_levels(S, I, lower, I.level_cap, blev, bpos, levp, prow);
   // positions: local to each block
   std::vector<int> pos(n);
   for (int b = 0; b < nb; b++)
@@ -2099,8 +2144,8 @@ static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>&
   });
   for (int r = 0; r < n; r++) prs[r + 1] += prs[r];
   const long long ne = prs[n];
-  std::vector<int> pcol(full ? ne : 0), psrc(full ? ne : 0);
-  if (full) parallel_for(n, [&](long long a, long long b) {
+  std::vector<int> pcol(ne), psrc(ne);
+  parallel_for(n, [&](long long a, long long b) {
     for (long long r = a; r < b; r++) {
       const int i = prow[r];
       int j = prs[r];
@@ -2109,21 +2154,15 @@ static void build_sweep(SweepSet& S, const Ilu& I, bool lower, std::vector<int>&
     }
   });
   S.nblk = nb;
-  S.nlev_max = nlev_tot;
-  S.max_nr = maxnr;
   S.ne = ne;
-  S.nlev_sum = blev[nb];
   if (getenv("RMX_DEBUG"))
     fprintf(stderr, "[rmx] %s sweep, %d strip(s) x %d segment(s): %d levels (longest strip), "
             "%.1f rows/level, max %d, %lld entries\n", lower ? "lower" : "upper", nb, I.nseg,
-            nlev_tot, (double)n / std::max(1, blev[nb]), maxnr, ne);
-  S.xp.alloc(n);
-  S.packed = full;
-  if (full) {
-    S.blev.upload(blev, s); S.bpos.upload(bpos, s); S.lev_ptr.upload(levp, s);
-    S.prs.upload(prs, s); S.prow.upload(prow, s); S.pcol.upload(pcol, s); S.psrc.upload(psrc, s);
-    HIPCHECK(hipStreamSynchronize(s));
-  }
+            S.nlev_max, (double)n / std::max(1, S.nlev_sum), S.max_nr, ne);
+  S.packed = true;
+  S.blev.upload(blev, s); S.bpos.upload(bpos, s); S.lev_ptr.upload(levp, s);
+  S.prs.upload(prs, s); S.prow.upload(prow, s); S.pcol.upload(pcol, s); S.psrc.upload(psrc, s);
+  HIPCHECK(hipStreamSynchronize(s));
   order = prow;
 }
 
@@ -3093,8 +3132,8 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   // strip sweeps: a level of more rows than the staged sweep's row groups (512 threads, 4
   // lanes per row) is split, so that no level needs a second round, whose entries would be
   // loaded inside the level instead of one level ahead
-  int cap = level_cap;
-  if (const char* e = getenv("RMX_LEVEL_CAP")) cap = std::max(0, atoi(e));
+  I.level_cap = level_cap;
+  if (const char* e = getenv("RMX_LEVEL_CAP")) I.level_cap = std::max(0, atoi(e));
   // strip ILU of few blocks: by chunks; the reference sweeps keep the order of the substitution
   // (and the block sweeps where RMX_SWEEP or their pass caps ask for them)
   I.cs.on = false;
@@ -3108,11 +3147,16 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   }
   // the level sweeps where neither runs, or RMX_SWEEP asks for them
   const bool full = !(I.cs.on || I.bs.on || (I.nlo.on && I.nup.on)) || sweep_variant() < 2;
-  std::vector<int> olo, oup;
-  build_sweep(I.lo, I, true, olo, s, cap, full);
-  build_sweep(I.up, I, false, oup, s, cap, full);
+  I.lo.packed = I.up.packed = false;
+  I.lo.nlev_max = I.up.nlev_max = -1;
+  if (full || I.nlo.on) I.lo.xp.alloc(n);
+  if (full) I.up.xp.alloc(n);
+  else count_entries(I);
   // forward position (global, concatenated) of the row at each backward position
   if (full) {
+    std::vector<int> olo, oup;
+    build_sweep(I.lo, I, true, olo, s);
+    build_sweep(I.up, I, false, oup, s);
     std::vector<int> fpos(n), f2b(n);
     for (int r = 0; r < n; r++) fpos[olo[r]] = r;
     for (int r = 0; r < n; r++) f2b[r] = fpos[oup[r]];

@@ -126,11 +126,11 @@ struct Params {
 
 constexpr int RING = 8192;     // LDS ring of solved x values in the packed sweeps
 
-// Packed layout of one triangular sweep by levels over all strips of an ILU system (its
-// counts alone unless `packed`).
+// Packed layout of one triangular sweep by levels over all strips of an ILU system (the count of
+// its entries alone unless `packed`; levels -1 until sweep_levels).
 struct SweepSet {
   bool packed = false;
-  int nblk = 0, nlev_max = 0, nlev_sum = 0, max_nr = 0;
+  int nblk = 0, nlev_max = -1, nlev_sum = 0, max_nr = 0;
   long long ne = 0;
   DBuf<int> blev, bpos;         // per strip: first level, first position
   DBuf<int> lev_ptr;            // per strip: local level offsets + sentinel
@@ -232,6 +232,7 @@ struct FlowUnits {
 struct Ilu {
   bool ready = false;
   int n = 0, nblk = 1, nseg = 1;
+  int level_cap = 0;            // most rows of a level (0: any)
   std::vector<int> seg;         // segment of every row (empty: one segment per strip)
   long long nnz = 0;
   std::vector<int> bstart, h_rp, h_cols, flev;
@@ -495,6 +496,7 @@ std::vector<int> cut_segments(const std::vector<int>& bstart, const std::vector<
                               const HostModel& hm, int nseg);
 void coarse_setup(Ctx& c, const std::vector<int>& rp, const std::vector<int>& cl,
                   const std::vector<int>& group, int nseg);
+void sweep_levels(Ilu& I);
 int ilu_sweeps(const Ilu& I);                  // RMX_SWEEPS_* of an application
 bool chunk_layout(const Ilu& I, ChunkLayout& L);
 void chunk_reach(const ChunkLayout& L, std::vector<int>& rows, std::vector<int>& reach);

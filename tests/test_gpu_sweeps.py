@@ -617,3 +617,25 @@ def test_bicgstab_with_an_exact_preconditioner(ctx, n, dense, seed):
         x = b / vals
     assert out.converged
     assert np.abs(ctx.solution() - x).max() <= 1e-12 * np.abs(b).max()
+
+
+# what is told of a system's sweeps is the same whichever run: entries and levels of the packed level
+# sweeps (RMX_SWEEP=1) and of the others, whose set-up has no use for levels
+@pytest.mark.parametrize("strips,segments", [(0, 0), (1, 1), (5, 3), (17, 220)])
+def test_sweep_info_of_every_kind(ctx, strips, segments, monkeypatch):
+    ctx.upload_mesh(golden_deck(load_golden("channel200x20")))
+    ctx.prepare()
+    seen = {}
+    for sweep in ("1", None):
+        monkeypatch.setenv("RMX_SWEEP", sweep) if sweep else monkeypatch.delenv("RMX_SWEEP", raising=False)
+        ctx.set_strips(strips, segments)
+        assert (ctx.sweeps() == "levels") == (sweep == "1")
+        for kind in (rmx.PREC_ILU0, rmx.PREC_SILU0):
+            i = ctx.sweep_info(kind)
+            seen[sweep, kind] = (i.lower_entries, i.upper_entries, i.lower_levels, i.upper_levels, i.strips,
+                                 i.segments)
+            assert min(seen[sweep, kind]) > 0
+            assert ctx.sweep_info(kind).upper_levels == i.upper_levels
+    for kind in (rmx.PREC_ILU0, rmx.PREC_SILU0):
+        assert seen["1", kind] == seen[None, kind]
+    ctx.set_strips(0, 0)
