@@ -38,6 +38,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <future>
 #include <type_traits>
 
 #include "rmx_internal.h"
@@ -2518,6 +2519,7 @@ static void build_nodes(NodeSweep& S, const Ilu& I, bool lower, const std::vecto
         for (int k = i; k < j; k++) w += rp[k + 1] - rp[k];
         if (w > BS_MAXW) j = i + 1;
       }
+      for (int k = i; k < j; k++) uof[k] = (int)ustart.size();
       ustart.push_back(i);
       ustrip.push_back(b);
       i = j;
@@ -2545,39 +2547,30 @@ static void build_nodes(NodeSweep& S, const Ilu& I, bool lower, const std::vecto
       uc.erase(std::unique(uc.begin(), uc.end()), uc.end());
     }
   };
+  // the units that a unit reads, their number if `out` is null
+  auto units = [&](const std::vector<int>& uc, int* out) {
+    int last = -1, k = 0;
+    for (int c : uc)
+      if (uof[c] != last) { last = uof[c]; if (out) out[k] = last; k++; }
+    return k;
+  };
+  std::vector<long long> dp(nu + 1, 0);
   parallel_for(nu, [&](long long u0, long long u1) {
     std::vector<int> uc;
     for (long long U = u0; U < u1; U++) {
       uone[U] = one_set(ustart[U], ustart[U + 1]);
-      for (int i = ustart[U]; i < ustart[U + 1]; i++) uof[i] = (int)U;
       cols_of((int)U, uc);
       uw[U] = (int)uc.size();
       while ((16 << ulg[U]) < uw[U]) ulg[U]++;
+      dp[U + 1] = units(uc, nullptr);
     }
   });
-  // units that every unit reads
-  std::vector<long long> dp(nu + 1, 0);
-  std::vector<int> dep;
-  {
-    std::vector<int> cnt(nu, 0);
-    auto units = [&](int U, std::vector<int>& uc, int* out) {
-      cols_of(U, uc);
-      int last = -1, k = 0;
-      for (int c : uc)
-        if (uof[c] != last) { last = uof[c]; if (out) out[k] = last; k++; }
-      return k;
-    };
-    parallel_for(nu, [&](long long u0, long long u1) {
-      std::vector<int> uc;
-      for (long long U = u0; U < u1; U++) cnt[U] = units((int)U, uc, nullptr);
-    });
-    for (int U = 0; U < nu; U++) dp[U + 1] = dp[U] + cnt[U];
-    dep.resize(dp[nu]);
-    parallel_for(nu, [&](long long u0, long long u1) {
-      std::vector<int> uc;
-      for (long long U = u0; U < u1; U++) units((int)U, uc, dep.data() + dp[U]);
-    });
-  }
+  for (int U = 0; U < nu; U++) dp[U + 1] += dp[U];
+  std::vector<int> dep(dp[nu]);
+  if (dp[nu] > 0) parallel_for(nu, [&](long long u0, long long u1) {
+    std::vector<int> uc;
+    for (long long U = u0; U < u1; U++) { cols_of((int)U, uc); units(uc, dep.data() + dp[U]); }
+  });
   std::vector<int> place(nu, 0), order(nu), nlev(nstrip, 0), live(nstrip, 1), lbeg;
   std::vector<std::vector<int>> lptr(nstrip);    // level offsets of a strip into its order
   parallel_for(nstrip, [&](long long b0, long long b1) {
@@ -3142,8 +3135,15 @@ void ilu_setup(Ilu& I, int n, const std::vector<int>& rp, const std::vector<int>
   I.bs.on = I.nlo.on = I.nup.on = false;
   if (!I.cs.on && !twice) build_blocks(I, &unit, scol, spos, s);
   if (!I.cs.on && !I.bs.on && !twice) {
+    // both triangles side by side (their schedules are serial in a strip)
+    int dev = 0;
+    HIPCHECK(hipGetDevice(&dev));
+    auto up = std::async(std::launch::async, [&] {
+      HIPCHECK(hipSetDevice(dev));
+      build_nodes(I.nup, I, false, &unit, scol, spos, s);
+    });
     build_nodes(I.nlo, I, true, &unit, scol, spos, s);
-    if (I.nlo.on) build_nodes(I.nup, I, false, &unit, scol, spos, s);
+    up.get();
   }
   // the level sweeps where neither runs, or RMX_SWEEP asks for them
   const bool full = !(I.cs.on || I.bs.on || (I.nlo.on && I.nup.on)) || sweep_variant() < 2;
