@@ -1754,8 +1754,11 @@ template <class VT, int PK> struct ChunkBuf {
 };
 
 // One direction: chunks in processing order (UP: from the block's end, rows of a chunk from its
-// end).  cb: the block's first chunk, pb: its first packet; cnt: packets of every chunk.
-template <class VT, int PK, bool UP>
+// end).  cb: the block's first chunk, pb: its first packet; cnt: packets of every chunk.  A zero
+// stands for what a row does not have (another chunk's packets, entries of the inverse), and zero
+// times an infinity is a NaN: with ANY, the right-hand side may hold either, and such products are
+// left out, so that they reach the rows that depend on them and no others.
+template <class VT, int PK, bool UP, bool ANY>
 __device__ __forceinline__ void chunk_sweep(int nch, int cb, int pb,
                                             const unsigned char* __restrict__ cnt,
                                             const unsigned* __restrict__ idx,
@@ -1819,6 +1822,11 @@ __device__ __forceinline__ void chunk_sweep(int nch, int cb, int pb,
   };
   auto step = [&](const ChunkBuf<VT, PK>& b) {
     auto f = [](VT v) { return UP ? -(double)v : (double)v; };
+    if (ANY) {
+#pragma unroll
+      for (int p = 1; p < PK; p++)
+        if (p >= np) x[2 * p] = x[2 * p + 1] = 0.0;
+    }
     double a0 = f(b.v[0][0]) * x[0], a1 = f(b.v[0][1]) * x[1];
     a0 += f(np > 1 ? b.v[1][0] : (VT)0) * x[2];
     a1 += f(np > 1 ? b.v[1][1] : (VT)0) * x[3];
@@ -1842,8 +1850,9 @@ __device__ __forceinline__ void chunk_sweep(int nch, int cb, int pb,
     a0 += dpp_get<0xB1>(a0);                       // over the row's four lanes
     a0 += dpp_get<0x4E>(a0);
     const double s = s0 + a0;
-    const double p0 = (lane < 16 ? b.t[0] : 0.0) * s, p1 = (lane < 32 ? b.t[1] : 0.0) * s;
-    const double p2 = (lane < 48 ? b.t[2] : 0.0) * s, p3 = b.t[3] * s;
+    auto times = [&](double t) { return ANY && t == 0.0 ? 0.0 : t * s; };
+    const double p0 = times(lane < 16 ? b.t[0] : 0.0), p1 = times(lane < 32 ? b.t[1] : 0.0);
+    const double p2 = times(lane < 48 ? b.t[2] : 0.0), p3 = times(b.t[3]);
     const double2 e = swap32(p0, p2), h = swap32(p1, p3);
     const double2 g = swap16(e.x + e.y, h.x + h.y);
     double y = g.x + g.y;
@@ -1891,6 +1900,7 @@ __global__ void __launch_bounds__(64) k_chunk_sweep(const int4* __restrict__ inf
   const int4 w0 = info[2 * blockIdx.x], w1 = info[2 * blockIdx.x + 1];
   const int m = w0.y, nch = (m + CH_ROWS - 1) / CH_ROWS, all = nch * CH_ROWS;
   const int* row = rows + w0.x;
+  bool finite = true;
   for (int k0 = 0; k0 < all; k0 += 64 * U) {
     int i[U];
     double v[U];
@@ -1901,14 +1911,21 @@ __global__ void __launch_bounds__(64) k_chunk_sweep(const int4* __restrict__ inf
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int k = k0 + 64 * u + lane;
+      finite = finite && __builtin_isfinite(v[u]);
       if (k < all) st_lds(8u * k, k < m ? v[u] : 0.0);
     }
   }
   asm volatile("" ::: "memory");
   const unsigned spare = 8u * (all + lane);
-  chunk_sweep<VT, PK, false>(nch, w0.z, w1.x, dlo, ilo, vlo, tlo, nullptr, spare);
-  asm volatile("" ::: "memory");
-  chunk_sweep<VT, PK, true>(nch, w0.z, w1.y, dup, iup, vup, tup, dgu, spare);
+  if (__all(finite)) {
+    chunk_sweep<VT, PK, false, false>(nch, w0.z, w1.x, dlo, ilo, vlo, tlo, nullptr, spare);
+    asm volatile("" ::: "memory");
+    chunk_sweep<VT, PK, true, false>(nch, w0.z, w1.y, dup, iup, vup, tup, dgu, spare);
+  } else {
+    chunk_sweep<VT, PK, false, true>(nch, w0.z, w1.x, dlo, ilo, vlo, tlo, nullptr, spare);
+    asm volatile("" ::: "memory");
+    chunk_sweep<VT, PK, true, true>(nch, w0.z, w1.y, dup, iup, vup, tup, dgu, spare);
+  }
   asm volatile("" ::: "memory");
   for (int k0 = 0; k0 < m; k0 += 64 * U) {
     int i[U];

@@ -639,3 +639,61 @@ def test_sweep_info_of_every_kind(ctx, strips, segments, monkeypatch):
     for kind in (rmx.PREC_ILU0, rmx.PREC_SILU0):
         assert seen["1", kind] == seen[None, kind]
     ctx.set_strips(0, 0)
+
+
+# a right-hand side with an infinity or a NaN: it reaches the rows that depend on it, as in the
+# oracle's triangular solves, and the others keep their values (1e-12 as for the other sweeps):
+# groups of rows coupled among themselves (5 within a chunk, 40 over several), and a channel
+@pytest.mark.parametrize("group,width", [(1, 0), (5, 2), (40, 6), (23, 9)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_chunk_sweeps_of_non_finite_vectors(ctx, group, width, bad):
+    print(f"[gpu] strip sweeps, groups of {group} rows, {bad} in the right-hand side", flush=True)
+    n = 700
+    rp0, c0, v0 = _band_csr(n, [1 + k for k in range(width)], 95)
+    rows = np.repeat(np.arange(n), np.diff(rp0))
+    keep = rows // group == c0 // group
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=n))]).astype(np.int32)
+    cols, vals = c0[keep], v0[keep]
+    b = np.random.default_rng(96).standard_normal(n)
+    b[[0, 17, 350, 359, 698]] = bad
+    ctx.set_strips(1, 0)
+    ctx.csr_upload(rp, cols, vals, np.ones(n))
+    assert ctx.sweeps() == "chunks"
+    for prec, dt in ((rmx.F64, np.float64), (rmx.F32, np.float32)):
+        if prec == rmx.F32:
+            ctx.convert(rmx.F32)
+        ctx.silu0_factor(prec)
+        L, _ = po.ilu0_factor(rp, cols, vals.astype(dt))
+        ref = po.ilu0_solve(rp, cols, L, b)
+        y = ctx.precond_apply(rmx.PREC_SILU0, b, prec)
+        ok = np.isfinite(ref)
+        assert ok.any() and not ok.all()
+        np.testing.assert_array_equal(np.isfinite(y), ok)
+        assert np.abs(y[ok] - ref[ok]).max() <= 1e-12 * np.abs(ref[ok]).max(), prec
+    ctx.set_strips(0, 0)
+
+
+def test_chunk_sweeps_of_non_finite_vectors_on_a_mesh(ctx):
+    from rismo2d_amd import deck as dk
+    ctx.upload_mesh(dk.channel(60, 13, length=300.0, width=65.0))
+    ctx.time_step(30.0, 0.7, first=True)
+    n = ctx.prepare()
+    ctx.assemble(rmx.F64)
+    ctx.scale_l2()
+    ctx.silu0_factor(rmx.F64)
+    assert ctx.sweeps() == "chunks"
+    rp, cols = ctx.pattern()
+    A, _ = ctx.matrix(rmx.F64)
+    block = ctx.blocks()
+    of = np.repeat(np.arange(n), np.diff(rp))
+    keep = block[of] == block[cols]
+    rp2 = np.concatenate([[0], np.cumsum(np.bincount(of[keep], minlength=n))]).astype(np.int32)
+    L, _ = po.ilu0_factor(rp, cols, A)
+    for row in (0, n // 3, n // 2 + 5, n - 1):
+        b = np.random.default_rng(97).standard_normal(n)
+        b[row] = np.nan
+        ref = po.ilu0_solve(rp2, cols[keep], L[keep], b)
+        y = ctx.precond_apply(rmx.PREC_SILU0, b, rmx.F64)
+        ok = np.isfinite(ref)
+        assert np.isfinite(y[ok]).all()
+        assert np.abs(y[ok] - ref[ok]).max() <= 1e-12 * np.abs(ref[ok]).max()
